@@ -1,0 +1,381 @@
+// Advection steps fused in LDS with the coefficients in registers (the
+// register form of strategy LINE_LDS, see bkma_tuned.hip).
+//
+// A work-group owns a tile: kTileRows consecutive rows per thread of one
+// column of one slab, RT threads along the rows, CT threads times V columns
+// across, SB slabs.  The tile's values live in LDS as FP64, one plane of
+// rows per (slab, column); a thread computes the foot and the six
+// coefficients of its rows once per pass and keeps them in registers for all
+// the steps of the pass, since they depend on (i0, i1) only.  A step reads the
+// kTileRows + 5 rows around a thread's shifted position (consecutive LDS
+// addresses, immediate offsets) and writes its kTileRows results back, so a
+// cell costs 3 LDS accesses and 6 multiply-adds per step; the foot arithmetic
+// (about 55 FP64 instructions per row) and HBM are paid once per pass.
+//  - WRAP tiles hold whole lines.  The first rows are repeated after the last
+//    one, so a window never wraps inside.  A pass may fuse any number of
+//    steps.
+//  - SEG tiles hold a segment of a longer line and the halo rows that the
+//    pass's steps reach (per slab: |s| + 6 rows per step), every row of the
+//    buffer is computed at every step and the rows next to the ends, which
+//    read outside the buffer, are discarded as the halo shrinks.  Rows that
+//    other work-groups overwrite in the same pass come from a snapshot.
+// Five rows per thread: the LDS row stride of neighbouring threads is then 5
+// doubles, which spreads 32 lanes over all 64 banks, and the coefficients take
+// 60 VGPRs, which leaves 4 wavefronts per SIMD.
+//
+// What bounds it: at 20 steps on [512][1024][512] the VALU is 58% and the LDS
+// 55% busy (FP32 storage 45% and 64%), with two work-groups per CU whose
+// barriers alternate the two.  Measured (steps kernel before -> this one):
+//   [300][1000][100]    FP64, 20 steps   2.93 -> 0.57 ms (column pair before)
+//   [4096][10000][1]    FP64, 20 steps  11.68 -> 0.70 ms
+//   [256][262144][4]    FP32, 20 steps  12.93 -> 7.4 ms (halo rows are 28% of
+//                       a tile there, the shifts reach 262 cells)
+//   [512][1024][512]    20 steps        1240 Gcell/s FP64, 1480 FP32
+// Rows of one thread that round to different shifts (a slab whose shift is an
+// integer up to rounding) take a form that reads every row's own six taps.
+//
+// Arithmetic: FP64 with the reference's separately rounded products and sums
+// (FUSED = false), or fused (FP32 storage in the plans).  RND rounds the
+// values to FP32 after every step: a pass then equals as many passes of one
+// step each.
+#pragma once
+
+#include "common.hpp"
+
+namespace bkma {
+
+constexpr int kTileRows = 5;               // rows per thread
+constexpr int kTileWin = kTileRows + 5;    // rows a thread's step reads
+constexpr int kTileGhost = 2 * kTileRows;  // rows repeated after a whole line
+constexpr int kTileLow = kTileRows;        // SEG: rows a thread's window may start before the buffer
+constexpr int kTileThreads = 1024;         // largest work-group
+constexpr int kTileMaxSteps = 256;         // steps per pass
+
+struct TileArgs {
+    AdvDev p;
+    int rt, ct, cb, sb;  // row threads per plane, column threads, columns and slabs per tile
+    int nct;             // column tiles per slab
+    int rows;            // SEG: rows of the buffer (rt * kTileRows)
+    int pl;              // plane pitch in doubles
+    int ns;              // steps in this pass
+    int nseg;            // SEG: work-groups per (slab, column tile); a slab uses as many as its halos need
+    int hb_max, ha_max;  // SEG: largest halo rows per step before and after a segment
+    int hrows;           // SEG: snapshot rows per (slab, segment)
+    unsigned mcb, mn1;   // ceil(2^32 / cb) (cb > 1), ceil(2^32 / n1): quotients of tile indexes (below 2^16)
+    i64 units;
+};
+
+// Halo rows per step of slab i0 before and after a segment (the stencil of
+// row i1 reads rows i1-d-2 .. i1-d+3, d in [floor(s), floor(s)+1]).
+__host__ __device__ __forceinline__ void tile_halo(const AdvDev &p, i64 i0, int hb_max, int ha_max, int &hb, int &ha) {
+    const double v = p.minRealVx + (double)(int)i0 * p.dvx;
+    const double s = v * p.dt * p.inv_dx;
+    const double dlo = floor(s - 1e-6), dhi = floor(s + 1e-6) + 1.0;
+    const double b = dhi + 2.0 > 0.0 ? dhi + 2.0 : 0.0, a = 3.0 - dlo > 0.0 ? 3.0 - dlo : 0.0;
+    hb = b < (double)hb_max ? (int)b : hb_max;
+    ha = a < (double)ha_max ? (int)a : ha_max;
+}
+
+// Segment `seg` of slab i0: rows [r0, r0 + nr) with ns*hb and ns*ha halo rows.
+struct TileSeg {
+    int hb, ha, r0, nr;
+};
+__device__ __forceinline__ TileSeg tile_segment(const TileArgs &a, i64 i0, int seg) {
+    TileSeg s;
+    tile_halo(a.p, i0, a.hb_max, a.ha_max, s.hb, s.ha);
+    const int n1 = (int)a.p.n1;
+    const int cap = a.rows - a.ns * (s.hb + s.ha);
+    const int cnt = (n1 + cap - 1) / cap;
+    const int len = (n1 + cnt - 1) / cnt;
+    s.r0 = seg * len;
+    s.nr = min(len, n1 - s.r0);  // <= 0: the slab needs fewer segments
+    return s;
+}
+
+// Old rows around every segment: ns*hb rows before it, then ns*ha after it
+// (periodic), hrows rows of n2 columns per (slab, segment).
+template <class T>
+__device__ __forceinline__ void tile_snapshot_unit(const T *__restrict__ data, T *__restrict__ halo, const TileArgs &a,
+                                                   i64 unit) {
+    const i64 i0 = unit / a.nseg;
+    const TileSeg s = tile_segment(a, i0, (int)(unit - i0 * a.nseg));
+    if (s.nr <= 0) return;
+    const i64 n2 = a.p.n2, line = a.p.n1 * n2;
+    const T *slab = data + i0 * line;
+    T *dst = halo + unit * a.hrows * n2;
+    const i64 before = (i64)a.ns * s.hb * n2, total = before + (i64)a.ns * s.ha * n2;
+    const i64 b0 = (i64)s.r0 * n2 - before, a0 = (i64)(s.r0 + s.nr) * n2 - before;
+    for (i64 e = threadIdx.x; e < total; e += blockDim.x) {
+        i64 src = e + (e < before ? b0 : a0);
+        if (src < 0) src += line;
+        if (src >= line) src -= line;
+        dst[e] = slab[src];
+    }
+}
+
+// adv_foot for |v*dt| below half the width (every tile's caller checks it):
+// the argument of the periodic remainder lies in [0, 3W), where a - W and
+// a - 2W are exact, so no library fmod is needed.
+__device__ __forceinline__ int tile_foot(const AdvDev &p, int i0, int i1, double &d_prev1) {
+    const double x = adv_coord(i1, p.minRealX, p.dx);
+    const double vx = adv_coord(i0, p.minRealVx, p.dvx);
+    const double displx = p.dt * vx;
+    const double a = p.realWidthX + x - displx - p.minRealX, w2 = 2.0 * p.realWidthX;
+    const double xFoot = p.minRealX + (a - (a >= w2 ? w2 : a >= p.realWidthX ? p.realWidthX : 0.0));
+    const int leftNode = (int)floor((xFoot - p.minRealX) * p.inv_dx);
+    d_prev1 = 2 + p.inv_dx * (xFoot - adv_coord(leftNode, p.minRealX, p.dx));
+    return leftNode;
+}
+
+// Six-tap sum over w[0..5].
+template <bool FUSED> __device__ __forceinline__ double tile_taps(const double (&c)[6], const double *w) {
+    double acc = c[0] * w[0];
+#pragma unroll
+    for (int k = 1; k < 6; ++k) {
+        if constexpr (FUSED)
+            acc = fma(c[k], w[k], acc);
+        else
+            acc = acc + c[k] * w[k];
+    }
+    return acc;
+}
+
+template <class T, bool FUSED, bool RND, int V, bool WRAP>
+__device__ __forceinline__ void tile_unit(T *__restrict__ data, const T *__restrict__ halo, const TileArgs &a, i64 unit,
+                                          double *__restrict__ lds) {
+    constexpr int E = kTileRows;
+    if constexpr (!WRAP) lds += kTileLow;
+    const int n1 = (int)a.p.n1;
+    const i64 n2 = a.p.n2;
+    const int tid = (int)threadIdx.x, nthr = (int)blockDim.x;
+    const int cb = a.cb, pl = a.pl, ns = a.ns;
+
+    // ---- the tile ----
+    const i64 grp = unit / a.nct;
+    const i64 col0 = (unit - grp * a.nct) * cb;
+    const int cbw = (int)min((i64)cb, n2 - col0);
+    i64 i0b;       // first slab
+    int nsl = 1;   // slabs
+    int nrow;      // rows staged (all slabs)
+    int hbn = 0, r0 = 0, nr = 0;
+    const T *hsrc = nullptr;
+    if constexpr (WRAP) {
+        i0b = grp * a.sb;
+        nsl = (int)min((i64)a.sb, a.p.n0 - i0b);
+        nrow = nsl * n1;
+    } else {
+        i0b = grp / a.nseg;
+        const TileSeg s = tile_segment(a, i0b, (int)(grp - i0b * a.nseg));
+        if (s.nr <= 0) return;  // uniform over the work-group
+        hbn = ns * s.hb;
+        r0 = s.r0;
+        nr = s.nr;
+        nrow = hbn + nr + ns * s.ha;
+        hsrc = halo + grp * a.hrows * n2 + col0;
+    }
+    T *base = data + i0b * n1 * n2 + col0;
+
+    // ---- stage, kTileRows loads in flight per thread ----
+#pragma unroll 1
+    for (int u = 0; u < V; ++u) {
+        const int q0 = tid + u * E * nthr;
+        T ld[E];
+#pragma unroll
+        for (int i = 0; i < E; ++i) {
+            const unsigned q = (unsigned)(q0 + i * nthr);
+            const unsigned row = cb == 1 ? q : __umulhi(q, a.mcb);
+            const unsigned col = q - row * (unsigned)cb;
+            ld[i] = (T)0;
+            if ((int)row < nrow && (int)col < cbw) {
+                if constexpr (WRAP) {
+                    ld[i] = base[(i64)row * n2 + col];
+                } else {
+                    const int b = (int)row - hbn;
+                    const T *src = b >= 0 && b < nr ? base + (i64)(r0 + b) * n2 : hsrc + (i64)(b < 0 ? (int)row : (int)row - nr) * n2;
+                    ld[i] = src[col];
+                }
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < E; ++i) {
+            const unsigned q = (unsigned)(q0 + i * nthr);
+            unsigned row = cb == 1 ? q : __umulhi(q, a.mcb);
+            const unsigned col = q - row * (unsigned)cb;
+            if ((int)row < nrow && (int)col < cbw) {
+                unsigned s = 0;
+                if constexpr (WRAP) {
+                    s = __umulhi(row, a.mn1);
+                    row -= s * (unsigned)n1;
+                }
+                double *dst = lds + (int)(s * (unsigned)cb + col) * pl + (int)row;
+                dst[0] = (double)ld[i];
+                if constexpr (WRAP) {
+                    if ((int)row < kTileGhost) dst[n1] = (double)ld[i];
+                }
+            }
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+
+    // ---- this thread's rows: feet, coefficients, window position ----
+    const int c = tid / a.rt, g = tid - c * a.rt;
+    const int sl = c / a.ct, cc = c - sl * a.ct;
+    const bool act = sl < nsl && cc < cbw;
+    const int half = n1 / 2;
+    double coef[E][6];
+    int d0 = 0;
+    int turn = 0;  // rows whose shift differs from the first row's: two bits per row, 1 + shift - d0 (0: the same)
+#pragma unroll
+    for (int j = 0; j < E; ++j) {
+        int lr = g * E + j;
+        bool in = act;
+        if constexpr (WRAP) {
+            in = act && lr < n1;
+        } else {
+            lr += r0 - hbn;
+            if (lr < 0) lr += n1;
+            if (lr >= n1) lr -= n1;
+        }
+        double d_prev1 = 2.0;
+        int d = in ? lr - tile_foot(a.p, (int)(i0b + sl), lr, d_prev1) : d0;
+        adv_lag_basis(d_prev1, coef[j]);
+        if (in && d > half) d -= n1;
+        if (in && d < -half) d += n1;
+        if (j == 0) d0 = d;
+        if (d != d0) turn |= (d > d0 ? 2 : 3) << (2 * j);  // two adjacent shifts at most
+        __builtin_amdgcn_sched_barrier(0);  // one row's temporaries at a time
+    }
+    int rb = g * E - d0 - 2;
+    if constexpr (WRAP) {
+        if (rb < 0) rb += n1;
+        if (rb >= n1) rb -= n1;
+    } else {
+        rb = min(max(rb, 1 - kTileLow), a.rows - 1);  // beyond: every row of the thread is discarded
+    }
+    __syncthreads();
+
+    // ---- steps ----
+    const int plane = (sl * cb + cc) * pl;
+    const int vstep = a.ct * pl;
+    const int nv = (cbw + a.ct - 1) / a.ct;  // columns per thread in this tile (uniform)
+    double *src = lds;                       // V = 1: two buffers in turn, one barrier per step
+    double *alt = lds + a.sb * cb * pl;
+    // o = the step's results of this thread's rows of the column whose window
+    // starts at w0 (row rb)
+    auto column = [&](const double *w0, double (&o)[E]) __attribute__((always_inline)) {
+        if (turn == 0) {
+            double w[kTileWin];
+#pragma unroll
+            for (int t = 0; t < kTileWin; ++t) w[t] = w0[t];
+#pragma unroll
+            for (int j = 0; j < E; ++j) o[j] = tile_taps<FUSED>(coef[j], w + j);
+        } else {
+            int tb = turn, r = rb;
+            asm volatile("" : "+v"(tb), "+v"(r));  // nothing of this rare form is kept across the steps
+#pragma unroll
+            for (int j = 0; j < E; ++j) {
+                const int t = (tb >> (2 * j)) & 3;
+                int b = j - (t == 2 ? 1 : t == 3 ? -1 : 0);
+                if (WRAP && r + b < 0) b += n1;
+                double w[6];
+#pragma unroll
+                for (int k = 0; k < 6; ++k) w[k] = w0[b + k];
+                o[j] = tile_taps<FUSED>(coef[j], w);
+            }
+        }
+        if constexpr (RND) {
+#pragma unroll
+            for (int j = 0; j < E; ++j) o[j] = (double)(float)o[j];
+        }
+    };
+    // Results to the thread's rows at dst, the first rows also after the last.
+    const int left = WRAP ? n1 - g * E : E;  // rows of the line from this thread's first on
+    auto put = [&](double *dst, const double (&o)[E]) __attribute__((always_inline)) {
+        if (left >= E) {
+#pragma unroll
+            for (int j = 0; j < E; ++j) dst[j] = o[j];
+        } else {
+#pragma unroll
+            for (int j = 0; j < E - 1; ++j)
+                if (j < left) dst[j] = o[j];
+        }
+        if constexpr (WRAP) {
+            if (g * E < kTileGhost) {
+#pragma unroll
+                for (int j = 0; j < E; ++j) dst[n1 + j] = o[j];
+            }
+        }
+    };
+    for (int s = 0; s < ns; ++s) {
+        double o[E];
+        if constexpr (V == 1) {
+            if (act) {
+                column(src + plane + rb, o);
+                put(alt + plane + g * E, o);
+            }
+            __syncthreads();
+            double *t = src;
+            src = alt;
+            alt = t;
+        } else {
+            // a column is written while the next one is read: one barrier
+            // per column separates its reads from its writes
+            double *w = lds + plane + g * E;
+            const int shift = rb - g * E;
+            int col = act ? cc : cbw;
+#pragma unroll 1
+            for (int v = 0; v < nv; ++v) {
+                const bool on = col < cbw;
+                if (on) column(w + shift, o);
+                __syncthreads();
+                if (on) put(w, o);
+                w += vstep;
+                col += a.ct;
+            }
+            if (nv == 1) __syncthreads();
+        }
+    }
+    if constexpr (V > 1) __syncthreads();
+
+    // ---- store ----
+    const int nout = WRAP ? nrow : nr;
+#pragma unroll 1
+    for (int u = 0; u < V; ++u) {
+#pragma unroll
+        for (int i = 0; i < E; ++i) {
+            const unsigned q = (unsigned)(tid + (u * E + i) * nthr);
+            const unsigned row = cb == 1 ? q : __umulhi(q, a.mcb);
+            const unsigned col = q - row * (unsigned)cb;
+            if ((int)row < nout && (int)col < cbw) {
+                if constexpr (WRAP) {
+                    const unsigned s = __umulhi(row, a.mn1);
+                    base[(i64)row * n2 + col] = (T)src[(int)(s * (unsigned)cb + col) * pl + (int)(row - s * (unsigned)n1)];
+                } else {
+                    base[(i64)(r0 + (int)row) * n2 + col] = (T)src[(int)col * pl + hbn + (int)row];
+                }
+            }
+        }
+    }
+}
+
+// Launch shape of one problem (host side).
+struct TileShape {
+    TileArgs a{};
+    int v = 1;
+    bool wrap = true;
+    int threads = 0;
+    u64 lds_bytes = 0;
+    u64 halo_bytes = 0;  // SEG: snapshot buffer
+};
+
+// The tile of a problem for passes of at most ns steps (ns = 0: chosen here,
+// and returned in a.ns).  False where the tile form does not fit: lines
+// shorter than 16 rows, or whose halos leave too few rows of a segment.
+bool tile_shape(const bkma_adv_params &p, u64 elem_size, int ns, u64 lds_max, TileShape *out);
+
+// One pass of ns steps (at most the shape's).  `fused`: fused sums (FP32
+// storage), `rnd`: rounded to FP32 after every step.
+bkma_status launch_tile(const TileShape &sh, bkma_dtype dt, bool fused, bool rnd, void *data, void *halo, int ns,
+                        hipStream_t s);
+
+}  // namespace bkma

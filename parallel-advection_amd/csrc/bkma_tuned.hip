@@ -7,7 +7,8 @@
 // Strategy COLUMN_PAIR: the column stream for slabs whose rows take at most
 // two adjacent shifts (adv_pair.hpp): seven-tap windows, no shift branches.
 // Strategy LINE_LDS (any n2, any shift): slabs or segments of them staged in
-// LDS (adv_lds.hpp), up to 4 steps per pass.
+// LDS: with the coefficients in registers (adv_tile.hpp, lines from 16 rows
+// on), or computed at every step (adv_lds.hpp, up to 4 steps per pass).
 // Strategy LINE_SHFL (contiguous lines, n2 = 1, of 256 k <= 4096 cells, or
 // of 16): each line held in registers by one work-group (or one 16-lane row)
 // for a pass of up to 256 steps, stencil neighbours through DPP wavefront
@@ -30,6 +31,7 @@
 #include "adv_pair.hpp"
 #include "adv_shfl.hpp"
 #include "adv_stream.hpp"
+#include "adv_tile.hpp"
 #include "common.hpp"
 
 namespace bkma {
@@ -137,6 +139,8 @@ struct TunedPlan {
     LdsArgs lds{};
     u64 lds_bytes = 0;
     int lds_threads = 256;  // threads per work-group: 256, 512 or 1024
+    bool tiled = false;     // LINE_LDS with the coefficients in registers (adv_tile.hpp)
+    TileShape tile{};
     void *halo = nullptr;  // segmented mode: halo snapshot buffer (owned)
     ~TunedPlan() {
         if (halo) (void)hipFree(halo);
@@ -441,6 +445,7 @@ bkma_status plan_launch(const TunedPlan &pl, void *data, hipStream_t s, int ns) 
         BKMA_HIP_TRY(hipStreamWaitEvent(s, pl.join, 0));
         return st;
     }
+    if (pl.tiled) return launch_tile(pl.tile, pl.dtype, true, false, data, pl.halo, ns, s);
     if (pl.cfg.strategy == BKMA_STRATEGY_LINE_LDS)
         return pl.dtype == BKMA_F64 ? launch_lds<double>(pl, data, s, ns) : launch_lds<float>(pl, data, s, ns);
     if (pl.cfg.strategy == BKMA_STRATEGY_LINE_SHFL) {
@@ -470,7 +475,10 @@ bkma_status plan_launch(const TunedPlan &pl, void *data, hipStream_t s, int ns) 
 
 // nsteps steps: full passes of the plan's steps per pass, then the rest.
 bkma_status plan_steps(const TunedPlan &pl, void *data, u64 nsteps, hipStream_t s) {
-    const u64 ns = (u64)pl.ns;
+    u64 ns = (u64)pl.ns;
+    // FP64 storage of the register tiles: equal passes (the split does not
+    // change the results, and a short last pass pays a whole staging)
+    if (pl.tiled && pl.dtype == BKMA_F64 && nsteps > ns) ns = ceil_div(nsteps, ceil_div(nsteps, ns));
     for (u64 t = 0; t + ns <= nsteps; t += ns) BKMA_TRY(plan_launch(pl, data, s, (int)ns));
     if (nsteps % ns) BKMA_TRY(plan_launch(pl, data, s, (int)(nsteps % ns)));
     return BKMA_OK;
@@ -490,6 +498,13 @@ std::string lds_name(bkma_dtype dt, const LdsArgs &a, int threads) {
                        : ",whole_line") +
            (a.slabs > 1 ? ",slabs" + std::to_string(a.slabs) : "") + (a.ns > 1 ? ",steps" + std::to_string(a.ns) : "") +
            (threads != 256 ? ",wg" + std::to_string(threads) : "") + ">";
+}
+
+std::string tile_name(bkma_dtype dt, const TileShape &t) {
+    return std::string("line_lds<") + (dt == BKMA_F64 ? "f64" : "f32") + ",regs" + std::to_string(kTileRows) +
+           (t.wrap ? std::string(",whole_line") + (t.a.sb > 1 ? ",slabs" + std::to_string(t.a.sb) : "")
+                   : ",seg" + std::to_string(t.a.rows - t.a.hrows)) +
+           ",cols" + std::to_string(t.a.cb) + ",steps" + std::to_string(t.a.ns) + ",wg" + std::to_string(t.threads) + ">";
 }
 
 // Resident work-groups on the whole device for a variant (persistent grid).
@@ -594,6 +609,26 @@ bkma_status build_plan(const bkma_adv_params &p, bkma_dtype dt, const bkma_tuned
         pl->name = "hybrid_adaptivewg<pref" + std::to_string(cfg.seg_rows) + ",local" +
                    std::to_string(cfg.chunk_segs) + "%>";
         return BKMA_OK;
+    }
+    if (cfg.strategy == BKMA_STRATEGY_LINE_LDS && cfg.prefetch == kTileRows) {
+        // coefficients in registers, where that form fits (else below)
+        u64 lds_max = 0;
+        BKMA_TRY(lds_limit_bytes(&lds_max));
+        const int ns = steps_per_pass(cfg);
+        if (ns <= kTileMaxSteps && shift_supported(p, &why) && tile_shape(p, dt == BKMA_F64 ? 8 : 4, ns, lds_max, &pl->tile)) {
+            if (pl->tile.halo_bytes && hipMalloc(&pl->halo, pl->tile.halo_bytes) != hipSuccess) {
+                pl->halo = nullptr;
+                return fail(BKMA_ERR_OUT_OF_MEMORY, "tuned advection: halo buffer allocation failed");
+            }
+            pl->tiled = true;
+            pl->ns = ns;
+            pl->cfg.steps_per_pass = ns;
+            pl->cfg.seg_rows = pl->tile.wrap ? 0 : pl->tile.a.rows - pl->tile.a.hrows;
+            pl->cfg.chunk_segs = pl->tile.a.sb;
+            pl->cfg.waves_per_wg = pl->tile.threads / 64;
+            pl->name = tile_name(dt, pl->tile);
+            return BKMA_OK;
+        }
     }
     if (cfg.strategy == BKMA_STRATEGY_LINE_LDS) {
         const int ns = steps_per_pass(cfg);
@@ -702,6 +737,16 @@ std::vector<bkma_tuned_config> candidates(const bkma_adv_params &p, bkma_dtype d
     LdsArgs a;
     u64 bytes, lds_max = 0;
     if (lds_limit_bytes(&lds_max) != BKMA_OK) lds_max = 0;
+    // the LDS tile with register coefficients, at its own steps per pass
+    TileShape ts;
+    if (shift_supported(p, nullptr) && tile_shape(p, esz, 0, lds_max, &ts)) {
+        bkma_tuned_config c;
+        std::memset(&c, 0, sizeof(c));
+        c.strategy = BKMA_STRATEGY_LINE_LDS;
+        c.prefetch = kTileRows;
+        c.steps_per_pass = ts.a.ns;
+        out.push_back(c);
+    }
     int dlo = 0, dhi = 0;
     if (params_finite(p)) shift_range(p, &dlo, &dhi);
     const i64 halo_rows = std::max(0, dhi + 2) + std::max(0, 3 - dlo);
@@ -774,14 +819,35 @@ std::vector<bkma_tuned_config> candidates(const bkma_adv_params &p, bkma_dtype d
     return out;
 }
 
-// Heuristic (measured on the strided 2048x1024x512 workload): column pair
-// when every slab has at most two shifts (FP32 with the DPP broadcast at 5,
-// FP64 at 4 steps per pass), else the column stream with the smallest window (FP32 at 2, FP64 at
-// 3 steps per pass; more steps push the register window past the occupancy
-// that hides HBM latency), widest vector, deepest prefetch; contiguous
-// lines that fit LINE_SHFL with 256 steps per pass, 8 cells per lane from
-// 4096 lines on (measured on [2^21][1024][1]), else 4 (on [256][1024][1]);
-// else LINE_LDS whole line, else the longest segment.
+// Whether the column kernels keep the GPU busy on a shape: they run one
+// wavefront per 64*VEC columns of a slab (VEC = 2 from 128 columns on), a
+// serial walk along the line, and a tile that the columns do not fill runs
+// their slow body with range checks.  Both sides measured at 1, 5 and 20
+// steps (time of the column pair over that of the LINE_LDS register tiles):
+//   FP64 [n0][1000][128]: 512 wavefronts 0.8 / 1.5 / 1.9, 1024 0.8 / 1.2 / 1.2;
+//   FP64 [n0][1000][300] (a tile in three not full): 1023 wavefronts
+//     1.7 / 2.3 / 2.2, 2046 1.2 / 1.8 / 1.8;
+//   FP32 [n0][1000][128]: 256 wavefronts 0.9 / 1.4 / 2.2, 512 0.6 / 0.8 / 1.3;
+//   FP32 [n0][1000][300]: 510 wavefronts 3.2 / 1.5 / 2.3, 1023 1.7 / 0.9 / 1.4;
+// lines of 3000 rows, with narrower register tiles, move the lines down by
+// about a factor of two.
+bool columns_fill(const bkma_adv_params &p, bkma_dtype dt) {
+    if (p.n2 < (dt == BKMA_F64 ? 64 : 128)) return false;
+    const u64 width = p.n2 >= 128 ? 128 : 64;
+    const bool even = p.n2 % width == 0;
+    u64 enough = dt == BKMA_F64 ? (even ? 1024 : 4096) : (even ? 384 : 768);
+    if (p.n1 > 2500) enough /= 2;
+    return p.n0 * ceil_div(p.n2, width) >= enough;
+}
+
+// Heuristic: contiguous lines that fit LINE_SHFL, with 256 steps per pass, 8
+// cells per lane from 4096 lines on (measured on [2^21][1024][1]), else 4 (on
+// [256][1024][1]); where the column kernels fill the GPU, column pair when
+// every slab has at most two shifts (FP32 with the DPP broadcast at 5, FP64
+// at 4 steps per pass), else LINE_LDS register tiles, which take every other
+// shape of lines from 16 rows on; then the column stream with the smallest
+// window, the reference's executor for short lines, and LINE_LDS whole lines
+// or the longest segment.
 int heuristic_score(const bkma_tuned_config &c, bkma_dtype dt, const bkma_adv_params &p) {
     if (c.strategy == BKMA_STRATEGY_PLAIN)  // short lines: one work-group per slab would idle
         return (p.n1 < 64 ? 900000000 : 10000000) - std::abs(c.seg_rows - 256);
@@ -790,7 +856,7 @@ int heuristic_score(const bkma_tuned_config &c, bkma_dtype dt, const bkma_adv_pa
         // 256 steps per pass; 8 cells per lane when the lines fill the GPU
         // several times over, else 4 (twice the wavefronts)
         const bool many = p.n0 >= 4096;
-        return 600000000 + ((c.vec == 8) == many ? 1000 : 0) - std::abs(steps_per_pass(c) - 256);
+        return 1300000000 + ((c.vec == 8) == many ? 1000 : 0) - std::abs(steps_per_pass(c) - 256);
     }
     if ((c.strategy == BKMA_STRATEGY_COLUMN_PAIR || c.strategy == BKMA_STRATEGY_COLUMN_STREAM) &&
         p.n2 < 64 * (u64)c.vec)  // a wavefront's lanes would mostly idle
@@ -810,6 +876,8 @@ int heuristic_score(const bkma_tuned_config &c, bkma_dtype dt, const bkma_adv_pa
         return 1000000000 - c.smax * 1000000 - std::abs(ns - want) * 100000 + c.vec * 1000 + c.prefetch * 10 +
                c.nontemporal - c.persistent - 100 * c.wide_window;
     }
+    if (c.strategy == BKMA_STRATEGY_LINE_LDS && c.prefetch == kTileRows)
+        return columns_fill(p, dt) ? 1050000000 : 1200000000;
     // LINE_LDS: whole lines; else the longest segment, with 16-wave
     // work-groups where they are offered (the segment fills the LDS)
     return c.seg_rows == 0 ? 500000000 - std::abs(steps_per_pass(c) - 2) * 1000 - c.waves_per_wg
@@ -893,6 +961,22 @@ extern "C" bkma_status bkma_adv_plan_create(const bkma_adv_params *params, bkma_
     auto *pl = new (std::nothrow) bkma_adv_plan();
     if (!pl) return fail(BKMA_ERR_OUT_OF_MEMORY, "plan allocation");
     bkma_status st = build_plan(*params, dtype, best, pl);
+    if (st == BKMA_ERR_OUT_OF_MEMORY && best.strategy == BKMA_STRATEGY_LINE_LDS && best.prefetch == kTileRows) {
+        // no room for the tile's halo snapshot: the best of the other plans
+        (void)hipGetLastError();
+        delete pl;
+        pl = new (std::nothrow) bkma_adv_plan();
+        if (!pl) return fail(BKMA_ERR_OUT_OF_MEMORY, "plan allocation");
+        cands.erase(std::remove_if(cands.begin(), cands.end(),
+                                   [](const auto &c) { return c.strategy == BKMA_STRATEGY_LINE_LDS && c.prefetch == kTileRows; }),
+                    cands.end());
+        if (!cands.empty()) {
+            best = *std::max_element(cands.begin(), cands.end(), [&](const auto &a, const auto &b) {
+                return heuristic_score(a, dtype, *params) < heuristic_score(b, dtype, *params);
+            });
+            st = build_plan(*params, dtype, best, pl);
+        }
+    }
     if (st != BKMA_OK) {
         delete pl;
         return st;
