@@ -170,6 +170,17 @@ template <class T> __global__ void copy_kernel(T *__restrict__ dst, const T *__r
 // ---------------------------------------------------------------------------
 constexpr i64 kMaxWgSize = 1024;
 
+// A solver whose whole-array step has a kernel of its own specialises this:
+// one step of the [n0][n1][n2] array at `data`, with the executor's values.
+// AdaptiveWg (one batch over the array, LDS scratch) and NDRange ask it after
+// their own checks; *done = false leaves the step to the executor's kernel.
+template <class T, class Solver> struct WholeStep {
+    static Status run(T *, const Solver &, i64, i64, i64, hipStream_t, bool *done) {
+        *done = false;
+        return Status{};
+    }
+};
+
 inline Status lds_limit(u64 *bytes) {
     int dev = 0;
     BKMA_EXEC_TRY(hip_status(hipGetDevice(&dev), "hipGetDevice"));
@@ -267,6 +278,11 @@ Status run_adaptivewg(T *data, const Solver &solver, i64 n0, i64 n1, i64 n2, con
                     return error(BKMA_ERR_INVALID_ARGUMENT,
                                  "AdaptiveWg/Local: scratch (w0, w2, nw) of " + std::to_string(lds_bytes) +
                                      " bytes exceeds the work-group LDS limit of " + std::to_string(lds_max));
+                if (i0_base == 0 && d0.n_batch == 1 && d2.n_batch == 1 && bs0 == n0 && bs2 == n2) {
+                    bool done = false;
+                    BKMA_EXEC_TRY((WholeStep<T, Solver>::run(data, solver, n0, n1, n2, stream, &done)));
+                    if (done) continue;
+                }
                 auto kern = adaptivewg_kernel<T, Solver, false>;
                 BKMA_EXEC_TRY(hip_status(hipFuncSetAttribute((const void *)kern,
                                                              hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -303,6 +319,9 @@ Status run_ndrange(T *data, const Solver &solver, i64 n0, i64 n1, i64 n2, hipStr
     BKMA_EXEC_TRY(lds_limit(&lds_max));
     const u64 lds_bytes = (u64)n1 * sizeof(T);
     if (lds_bytes > lds_max) return error(BKMA_ERR_INVALID_ARGUMENT, "NDRange: line does not fit in LDS");
+    bool done = false;
+    BKMA_EXEC_TRY((WholeStep<T, Solver>::run(data, solver, n0, n1, n2, stream, &done)));
+    if (done) return Status{};
     const i64 lines = n0 * n2;
     const i64 max_blocks = 0x7fffffffLL / std::max<i64>(n1, 1);
     for (i64 off = 0; off < lines; off += max_blocks) {

@@ -371,7 +371,8 @@ struct TileShape {
 // The tile of a problem for passes of at most ns steps (ns = 0: chosen here,
 // and returned in a.ns).  False where the tile form does not fit: lines
 // shorter than 16 rows, or whose halos leave too few rows of a segment.
-bool tile_shape(const bkma_adv_params &p, u64 elem_size, int ns, u64 lds_max, TileShape *out);
+// whole_only: whole lines only, which need no snapshot.
+bool tile_shape(const bkma_adv_params &p, u64 elem_size, int ns, u64 lds_max, TileShape *out, bool whole_only = false);
 
 // One pass of ns steps (at most the shape's).  `fused`: fused sums (FP32
 // storage), `rnd`: rounded to FP32 after every step.

@@ -6,15 +6,32 @@
 // bkma/executors.hpp (the reference's work decomposition, generic over the
 // solver) instantiated with AdvSolverDev and ConvSolverDev, which keep the
 // reference's FP64 arithmetic (per-cell foot location and lag_basis), so
-// their results are bit-identical to the FP64 oracle.  They are the baseline
-// the tuned kernels are measured against.
+// their results are bit-identical to the FP64 oracle.  An advection call of
+// AdaptiveWg (LDS scratch, one batch) or NDRange runs the same step through
+// adv_step.hip where that covers it, with the same values.
 #include <algorithm>
 #include <cstdio>
 
+#include "adv_step.hpp"
 #include "bkma/executors.hpp"
 #include "common.hpp"
 
 namespace bkma {
+
+namespace exec {
+
+// The advection solver's whole-array step (adv_step.hip).
+template <class T> struct WholeStep<T, AdvSolverDev> {
+    static Status run(T *data, const AdvSolverDev &solver, i64 n0, i64 n1, i64 n2, hipStream_t stream, bool *done) {
+        *done = false;
+        const AdvDev &p = solver.p;
+        if (n0 != p.n0 || n1 != p.n1 || n2 != p.n2) return Status{};  // a part of the solver's array
+        const bkma_status st = adv_step_whole(p, sizeof(T) == 8 ? BKMA_F64 : BKMA_F32, data, stream, done);
+        return st == BKMA_OK ? Status{} : error(st, bkma_last_error());
+    }
+};
+
+}  // namespace exec
 
 namespace {
 

@@ -86,9 +86,13 @@ int plane_pitch(int rows, int cb) {
 
 }  // namespace
 
-bool tile_shape(const bkma_adv_params &p, u64 elem_size, int ns, u64 lds_max, TileShape *out) {
+bool tile_shape(const bkma_adv_params &p, u64 elem_size, int ns, u64 lds_max, TileShape *out, bool whole_only) {
     if (p.n1 < 16 || p.n0 == 0 || p.n2 == 0) return false;
-    constexpr int kTarget = 512;  // threads per work-group: two work-groups per CU at 128 VGPRs
+    // Threads per work-group.  Whole lines: work-groups of four wavefronts,
+    // five to a CU, keep the LDS and the VALU busy at different times
+    // ([2048][1024][64] FP64, 20 steps: 1436 Gcell/s with 205 threads, 1290
+    // with 410).  Segments: longer ones have fewer halo rows.
+    constexpr int kWhole = 256, kSegment = 512;
     const u64 n0 = p.n0, n1 = p.n1, n2 = p.n2;
     TileShape sh;
     TileArgs &a = sh.a;
@@ -106,10 +110,10 @@ bool tile_shape(const bkma_adv_params &p, u64 elem_size, int ns, u64 lds_max, Ti
         const int rt = (int)rt_line;
         double best = 0;
         for (int v = n2 >= 3 ? 4 : (int)n2; v >= 1; v /= 2) {
-            for (int ct = 1; (ct == 1 || rt * ct <= kTarget) && (u64)(ct - 1) * v < n2; ++ct) {
+            for (int ct = 1; (ct == 1 || rt * ct <= kWhole) && (u64)(ct - 1) * v < n2; ++ct) {
                 const int cols = (int)std::min<u64>((u64)ct * v, n2);
                 const int pitch = plane_pitch((int)n1 + kTileGhost, cols);
-                for (int sb = 1; sb == 1 || ((u64)cols == n2 && rt * ct * sb <= kTarget && (u64)sb <= n0); ++sb) {
+                for (int sb = 1; sb == 1 || ((u64)cols == n2 && rt * ct * sb <= kWhole && (u64)sb <= n0); ++sb) {
                     const u64 b = bytes(sb * cols, pitch, v);
                     if (b > lds_max) break;
                     const u64 units = ceil_div(n0, (u64)sb) * ceil_div(n2, (u64)cols);
@@ -143,20 +147,21 @@ bool tile_shape(const bkma_adv_params &p, u64 elem_size, int ns, u64 lds_max, Ti
         }
         // long lines of many columns: segments of wider rows where only a few
         // columns of a whole line fit
-        if (best >= 0.75 || (best > 0 && n2 < 32)) {
+        if (best >= 0.75 || (best > 0 && (n2 < 32 || whole_only))) {
             *out = sh;
             return true;
         }
         whole = best > 0;
         if (whole) *out = sh;
     }
+    if (whole_only) return false;
     // segments
     sh.wrap = false;
     sh.v = n2 >= 3 ? 4 : (int)n2;
     a.ct = n2 > 4 ? 2 : 1;
     a.nct = (int)ceil_div(n2, (u64)a.ct * sh.v);
     a.cb = (int)ceil_div(n2, (u64)a.nct);
-    a.rt = kTarget / a.ct;
+    a.rt = kSegment / a.ct;
     auto pitch = [&] { return plane_pitch(kTileLow + a.rt * kTileRows + kTileWin, a.cb); };
     while (a.rt > 64 && 2 * bytes(a.cb, pitch(), sh.v) > lds_max) a.rt -= 1;
     a.rows = a.rt * kTileRows;
