@@ -281,10 +281,14 @@ typedef struct bkma_adv_problem {
 
 typedef struct bkma_adv_batch bkma_adv_batch;
 
-/* autotune = 1 times the LDS budgets (32 KB .. the device limit), work-group
- * sizes and steps per pass (1 .. 4) on the problems' own arrays, which the
- * timing steps modify: create the batch before initialising the data.
- * autotune = 0: 64 KB, 256 threads, one step per pass. */
+/* Problems whose lines all have a LINE_LDS register tile (16 rows and more,
+ * moderate shifts) run as groups of such tiles, one launch per group and as
+ * many fused steps as its tiles hold, with the results of one step per pass;
+ * autotune then has nothing to choose.  Otherwise autotune = 1 times the LDS
+ * budgets (32 KB .. the device limit), work-group sizes and steps per pass
+ * (1 .. 4) on the problems' own arrays, which the timing steps modify: create
+ * the batch before initialising the data.  autotune = 0: 64 KB, 256 threads,
+ * one step per pass. */
 bkma_status bkma_adv_batch_create(const bkma_adv_problem *problems, int32_t nproblems, bkma_dtype dtype,
                                   int32_t autotune, void *stream, bkma_adv_batch **out);
 /* A batch with an explicit configuration: LDS budget per work-group (bytes),

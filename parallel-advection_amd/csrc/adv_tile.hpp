@@ -379,4 +379,26 @@ bool tile_shape(const bkma_adv_params &p, u64 elem_size, int ns, u64 lds_max, Ti
 bkma_status launch_tile(const TileShape &sh, bkma_dtype dt, bool fused, bool rnd, void *data, void *halo, int ns,
                         hipStream_t s);
 
+// Several problems in one launch (ragged batches): problems whose tiles have
+// the same columns per thread and kind.
+struct TileProblem {
+    TileArgs a;
+    void *data;
+    void *halo;
+    i64 first;        // first work-group of the problem
+    i64 first_halo;   // SEG: first work-group of its snapshot
+};
+struct TileGroup {
+    int v = 1;
+    bool wrap = true;
+    int threads = 0;
+    u64 lds_bytes = 0;
+    int ns = 1;                     // steps per pass
+    int count = 0;                  // problems
+    i64 units = 0, halo_units = 0;  // work-groups
+    TileProblem *table = nullptr;   // device
+};
+// One pass of ns steps (at most the group's) of every problem of the group.
+bkma_status launch_tile_group(const TileGroup &g, bkma_dtype dt, bool rnd, int ns, hipStream_t s);
+
 }  // namespace bkma

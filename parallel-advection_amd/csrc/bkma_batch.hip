@@ -1,4 +1,11 @@
-// Ragged batches of independent advection problems in one persistent launch.
+// Ragged batches of independent advection problems.
+//
+// Where every problem has a tile of adv_tile.hpp, the batch runs those: the
+// problems whose tiles are of one kind, work-group size and depth share a
+// launch, and a launch fuses as many steps as the depth, the values rounded
+// to FP32 after every step (FP32 storage), so that the results are those of
+// one step per pass.  Otherwise, and for an explicit configuration, one
+// persistent launch per pass:
 //
 // Each problem ([n0][n1][n2], its own dt and velocity grid) is cut into work
 // items of the LINE_LDS kind.  A problem whose slab fits the LDS budget is
@@ -26,6 +33,7 @@
 #include <vector>
 
 #include "adv_lds.hpp"
+#include "adv_tile.hpp"
 #include "common.hpp"
 
 namespace bkma {
@@ -150,8 +158,17 @@ struct AdvBatch {
     std::map<u64, hipGraphExec_t> graphs;  // by step count
     std::vector<bkma_adv_plan *> plans;    // per-problem tuned plans (loop mode)
     u64 cells = 0;
+    // The register tiles of adv_tile.hpp instead of the persistent launch
+    std::vector<TileGroup> groups;  // tables owned
+    u64 tile_units = 0, tile_seg_units = 0;
 
+    void drop_groups() {
+        for (auto &g : groups) (void)hipFree(g.table);
+        groups.clear();
+        tile_units = tile_seg_units = 0;
+    }
     ~AdvBatch() {
+        drop_groups();
         for (auto &g : graphs) (void)hipGraphExecDestroy(g.second);
         for (auto *pl : plans) bkma_adv_plan_destroy(pl);
         for (void *h : halos) (void)hipFree(h);
@@ -184,6 +201,20 @@ template <class T> static bkma_status batch_pass(const AdvBatch &b, hipStream_t 
 
 // nsteps steps: passes of b.ns steps, then one pass of the remainder.
 static bkma_status batch_steps(const AdvBatch &b, u64 nsteps, hipStream_t s) {
+    if (!b.groups.empty()) {
+        // one step per pass in the results (FP32 storage rounds after every
+        // step), as many fused steps as a group's tiles hold in the launches:
+        // equal passes
+        for (const TileGroup &g : b.groups) {
+            const u64 passes = ceil_div(nsteps, (u64)g.ns);
+            for (u64 k = 0, t = 0; k < passes; ++k) {
+                const u64 end = nsteps * (k + 1) / passes;
+                BKMA_TRY(launch_tile_group(g, b.dtype, true, (int)(end - t), s));
+                t = end;
+            }
+        }
+        return BKMA_OK;
+    }
     for (u64 t = 0; t < nsteps;) {
         const int k = (int)std::min<u64>((u64)b.ns, nsteps - t);
         BKMA_TRY(b.dtype == BKMA_F64 ? batch_pass<double>(b, s, k) : batch_pass<float>(b, s, k));
@@ -292,6 +323,88 @@ static bkma_status build_items(AdvBatch &b, u64 budget, int threads, int ns) {
     return BKMA_OK;
 }
 
+// The tile groups of a batch, one step per pass in its results; false (and
+// no groups) where some problem has no tile or there is no room.
+static bool build_groups(AdvBatch &b) {
+    u64 lds_max = 0;
+    if (lds_limit_bytes(&lds_max) != BKMA_OK) return false;
+    const u64 esz = b.dtype == BKMA_F64 ? 8 : 4;
+    const size_t n = b.problems.size();
+    std::vector<TileShape> shapes(n);
+    for (size_t j = 0; j < n; ++j) {
+        const bkma_adv_params &p = b.problems[j].params;
+        if (!std::isfinite(p.minRealVx) || !std::isfinite(p.dvx) || !std::isfinite(p.inv_dx) ||
+            !std::isfinite(p.minRealX) || !std::isfinite(p.realWidthX) || !tile_shape(p, esz, 0, lds_max, &shapes[j]))
+            return false;
+    }
+    for (void *h : b.halos) (void)hipFree(h);
+    b.halos.clear();
+    b.drop_groups();
+    // Problems of one kind, work-group size and depth share a launch (the
+    // largest first: its last work-groups are then the short ones).
+    auto threads = [](const TileShape &t) { return t.threads <= 256 ? 256 : t.threads <= 512 ? 512 : kTileThreads; };
+    auto same = [&](const TileShape &x, const TileShape &y) {
+        return x.v == y.v && x.wrap == y.wrap && threads(x) == threads(y) && x.a.ns == y.a.ns;
+    };
+    std::vector<bool> taken(n, false);
+    std::vector<size_t> order(n);
+    for (size_t j = 0; j < n; ++j) order[j] = j;
+    auto cells = [&](size_t j) { return b.problems[j].params.n0 * b.problems[j].params.n1 * b.problems[j].params.n2; };
+    std::stable_sort(order.begin(), order.end(), [&](size_t x, size_t y) { return cells(x) > cells(y); });
+    bool ok = true;
+    for (size_t f : order) {
+        if (taken[f] || !ok) continue;
+        TileGroup g;
+        g.v = shapes[f].v;
+        g.wrap = shapes[f].wrap;
+        g.ns = shapes[f].a.ns;
+        std::vector<TileProblem> tab;
+        for (size_t j : order) {
+            if (taken[j] || !ok || !same(shapes[f], shapes[j])) continue;
+            const TileShape &t = shapes[j];
+            if ((u64)(g.units + t.a.units) > 0x7fffffffULL) continue;  // a group of its own
+            taken[j] = true;
+            TileProblem pr{};
+            pr.a = t.a;
+            pr.data = b.problems[j].data;
+            if (t.halo_bytes) {
+                ok = hipMalloc(&pr.halo, t.halo_bytes) == hipSuccess;
+                if (ok) b.halos.push_back(pr.halo);
+            }
+            pr.first = g.units;
+            pr.first_halo = g.halo_units;
+            g.units += t.a.units;
+            if (!t.wrap) g.halo_units += t.a.p.n0 * t.a.nseg;
+            g.threads = std::max(g.threads, t.threads);
+            g.lds_bytes = std::max(g.lds_bytes, t.lds_bytes);
+            tab.push_back(pr);
+        }
+        g.count = (int)tab.size();
+        ok = ok && hipMalloc((void **)&g.table, sizeof(TileProblem) * tab.size()) == hipSuccess;
+        if (ok) b.groups.push_back(g);
+        ok = ok && hipMemcpy(g.table, tab.data(), sizeof(TileProblem) * tab.size(), hipMemcpyHostToDevice) == hipSuccess;
+        b.tile_units += (u64)g.units;
+        if (!g.wrap) b.tile_seg_units += (u64)g.units;
+    }
+    if (!ok) {
+        (void)hipGetLastError();
+        b.drop_groups();
+        for (void *h : b.halos) (void)hipFree(h);
+        b.halos.clear();
+        return false;
+    }
+    b.ns = 1;
+    b.lds_budget = 0;
+    b.grid = 0;
+    for (const TileGroup &g : b.groups) {
+        b.lds_budget = std::max(b.lds_budget, g.lds_bytes);
+        b.grid = std::max(b.grid, (unsigned)g.units);
+    }
+    for (auto &g : b.graphs) (void)hipGraphExecDestroy(g.second);
+    b.graphs.clear();
+    return true;
+}
+
 }  // namespace bkma
 
 using namespace bkma;
@@ -374,6 +487,15 @@ extern "C" bkma_status bkma_adv_batch_create(const bkma_adv_problem *problems, i
         if (hipEventRecord(b->ev_in, as_stream(stream)) != hipSuccess ||
             hipStreamWaitEvent(b->stream, b->ev_in, 0) != hipSuccess)
             return bail(fail(BKMA_ERR_DEVICE, "batch: ordering after the caller's stream"));
+    }
+
+    // The register tiles cover lines from 16 rows on; measured on 48 problems
+    // of 16 .. 256 slabs, 64 .. 8192 rows and 1, 8 or 64 columns (345 M cells,
+    // FP32, 32 steps): 0.28 ms per step against 0.94 of the persistent launch
+    // below, whose every step reads and writes HBM and evaluates every foot.
+    if (build_groups(*b)) {
+        *out = b;
+        return BKMA_OK;
     }
 
     // Dynamic LDS budgets per work-group (the kernel adds a few static bytes),
@@ -529,8 +651,8 @@ extern "C" bkma_status bkma_adv_batch_describe(const bkma_adv_batch *b, uint64_t
                                                uint64_t *segmented_items, uint64_t *lds_budget, uint32_t *grid) {
     if (!b) return fail(BKMA_ERR_INVALID_ARGUMENT, "null batch");
     if (cells) *cells = b->cells;
-    if (items) *items = b->host_items.size();
-    if (segmented_items) *segmented_items = b->host_seg_items.size();
+    if (items) *items = b->groups.empty() ? b->host_items.size() : b->tile_units;
+    if (segmented_items) *segmented_items = b->groups.empty() ? b->host_seg_items.size() : b->tile_seg_units;
     if (lds_budget) *lds_budget = b->lds_budget;
     if (grid) *grid = b->grid;
     return BKMA_OK;

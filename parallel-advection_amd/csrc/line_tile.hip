@@ -10,8 +10,8 @@ namespace bkma {
 
 // Consecutive tiles of one memory line (the column tiles of a slab) on one
 // XCD: work-groups go to the 8 XCDs in turn.
-__device__ __forceinline__ i64 tile_of_block(i64 units, int nct) {
-    const i64 b = blockIdx.x, per = units / 8;
+__device__ __forceinline__ i64 tile_of_block(i64 b, i64 units, int nct) {
+    const i64 per = units / 8;
     return nct > 1 && b < per * 8 ? (b % 8) * per + b / 8 : b;
 }
 
@@ -19,13 +19,44 @@ template <class T, bool FUSED, bool RND, int V, bool WRAP>
 __global__ __launch_bounds__(kTileThreads) void adv_tile_kernel(T *__restrict__ data, const T *__restrict__ halo,
                                                                 TileArgs a) {
     extern __shared__ __align__(16) unsigned char tile_lds[];
-    tile_unit<T, FUSED, RND, V, WRAP>(data, halo, a, tile_of_block(a.units, a.nct),
+    tile_unit<T, FUSED, RND, V, WRAP>(data, halo, a, tile_of_block(blockIdx.x, a.units, a.nct),
                                       reinterpret_cast<double *>(tile_lds));
 }
 
 template <class T>
 __global__ void tile_snapshot_kernel(const T *__restrict__ data, T *__restrict__ halo, TileArgs a) {
     tile_snapshot_unit(data, halo, a, blockIdx.x);
+}
+
+// The last problem whose first work-group is not past b.
+template <i64 TileProblem::*FIRST> __device__ __forceinline__ int problem_of_block(const TileProblem *tab, int count, i64 b) {
+    int lo = 0, hi = count;
+    while (hi - lo > 1) {
+        const int mid = (lo + hi) / 2;
+        if (tab[mid].*FIRST <= b) lo = mid;
+        else hi = mid;
+    }
+    return lo;
+}
+
+template <class T, bool FUSED, bool RND, int V, bool WRAP>
+__global__ __launch_bounds__(kTileThreads) void adv_tile_group_kernel(const TileProblem *__restrict__ tab, int count,
+                                                                      int ns) {
+    extern __shared__ __align__(16) unsigned char tile_lds[];
+    const TileProblem &pr = tab[problem_of_block<&TileProblem::first>(tab, count, blockIdx.x)];
+    TileArgs a = pr.a;
+    a.ns = ns;
+    tile_unit<T, FUSED, RND, V, WRAP>((T *)pr.data, (const T *)pr.halo, a,
+                                      tile_of_block((i64)blockIdx.x - pr.first, a.units, a.nct),
+                                      reinterpret_cast<double *>(tile_lds));
+}
+
+template <class T>
+__global__ void tile_group_snapshot_kernel(const TileProblem *__restrict__ tab, int count, int ns) {
+    const TileProblem &pr = tab[problem_of_block<&TileProblem::first_halo>(tab, count, blockIdx.x)];
+    TileArgs a = pr.a;
+    a.ns = ns;
+    tile_snapshot_unit((const T *)pr.data, (T *)pr.halo, a, (i64)blockIdx.x - pr.first_halo);
 }
 
 namespace {
@@ -69,6 +100,32 @@ bkma_status launch_v(const TileShape &sh, const TileArgs &a, void *data, void *h
     if (sh.v == 1) return launch<T, FUSED, RND, 1, false>(sh, a, data, halo, s);
     if (sh.v == 2) return launch<T, FUSED, RND, 2, false>(sh, a, data, halo, s);
     return launch<T, FUSED, RND, 4, false>(sh, a, data, halo, s);
+}
+
+template <class T, bool FUSED, bool RND, int V, bool WRAP>
+bkma_status launch_group(const TileGroup &g, int ns, hipStream_t s) {
+    static std::atomic<unsigned> done{0};
+    auto k = adv_tile_group_kernel<T, FUSED, RND, V, WRAP>;
+    u64 lds_max = 0;
+    BKMA_TRY(lds_limit_bytes(&lds_max));
+    BKMA_HIP_TRY(allow_lds(k, done, lds_max));
+    hipLaunchKernelGGL(k, dim3((unsigned)g.units), dim3((unsigned)g.threads), (size_t)g.lds_bytes, s,
+                       (const TileProblem *)g.table, g.count, ns);
+    return check_launch("adv_tile_group_kernel");
+}
+
+template <class T, bool FUSED, bool RND> bkma_status launch_group_v(const TileGroup &g, int ns, hipStream_t s) {
+    if (g.wrap) {
+        if (g.v == 1) return launch_group<T, FUSED, RND, 1, true>(g, ns, s);
+        if (g.v == 2) return launch_group<T, FUSED, RND, 2, true>(g, ns, s);
+        return launch_group<T, FUSED, RND, 4, true>(g, ns, s);
+    }
+    hipLaunchKernelGGL(tile_group_snapshot_kernel<T>, dim3((unsigned)g.halo_units), dim3(256), 0, s,
+                       (const TileProblem *)g.table, g.count, ns);
+    BKMA_TRY(check_launch("tile_group_snapshot_kernel"));
+    if (g.v == 1) return launch_group<T, FUSED, RND, 1, false>(g, ns, s);
+    if (g.v == 2) return launch_group<T, FUSED, RND, 2, false>(g, ns, s);
+    return launch_group<T, FUSED, RND, 4, false>(g, ns, s);
 }
 
 unsigned magic(u64 d) { return d > 1 ? (unsigned)((((u64)1 << 32) + d - 1) / d) : 0; }
@@ -220,6 +277,13 @@ bkma_status launch_tile(const TileShape &sh, bkma_dtype dt, bool fused, bool rnd
     if (rnd) return launch_v<float, true, true>(sh, a, data, halo, s);
     if (fused) return launch_v<float, true, false>(sh, a, data, halo, s);
     return launch_v<float, false, false>(sh, a, data, halo, s);
+}
+
+bkma_status launch_tile_group(const TileGroup &g, bkma_dtype dt, bool rnd, int ns, hipStream_t s) {
+    if (ns < 1 || ns > g.ns) return fail(BKMA_ERR_RUNTIME, "LINE_LDS tiles: steps per pass out of range");
+    if (dt == BKMA_F64) return launch_group_v<double, false, false>(g, ns, s);
+    if (rnd) return launch_group_v<float, true, true>(g, ns, s);
+    return launch_group_v<float, true, false>(g, ns, s);
 }
 
 }  // namespace bkma

@@ -99,3 +99,36 @@ def test_default_plans(cuda, dtype, shape, dt):
     plan.close()
     assert ",regs5," in name
     _check(shape, dtype, 11, cfg.steps_per_pass, None, dt=dt, minRealVx=-1, maxRealVx=1)
+
+
+# Whole-line and segmented tiles of every width, several problems to a launch; the last two share one.
+BATCH = [(3, 8192, 8, 2e-3), (2, 16384, 1, 1e-3), (4, 640, 64, 1e-3), (5, 100, 1, 2e-3), (3, 6001, 2, 1e-3),
+         (7, 33, 2, 1e-3), (2, 5200, 3, 1e-3), (40, 64, 8, 2e-3), (9, 80, 8, 1e-3)]
+
+
+@pytest.mark.parametrize("graph", [True, False], ids=["graph", "eager"])
+@pytest.mark.parametrize("dtype", [B.F64, B.F32], ids=["f64", "f32"])
+def test_batch_of_tiles_rounds_every_step(cuda, dtype, graph):
+    """The default batch fuses steps in its tiles, with the results of one step per pass, on every run: 37 steps
+    (a graph of 32 and one of 5), then 1, then 37 again."""
+    import torch
+    tdt = torch.float64 if dtype == B.F64 else torch.float32
+    arrays = [torch.empty((n0, n1, n2), dtype=tdt, device="cuda") for n0, n1, n2, _ in BATCH]
+    params = [B.make_params(n0, n1, n2, dt=dt, minRealVx=-1, maxRealVx=1) for n0, n1, n2, dt in BATCH]
+    batch = B.AdvBatch(arrays, params, dtype)
+    assert batch.describe()["steps_per_pass"] == 1
+    for j, a in enumerate(arrays):
+        B.fill_uniform(a, 600 + j)
+    torch.cuda.synchronize()
+    refs = [a.cpu().numpy() for a in arrays]
+    for nsteps in (37, 1, 37):
+        batch.run(nsteps, graph=graph)
+        torch.cuda.synchronize()
+        for j, (n0, n1, n2, dt) in enumerate(BATCH):
+            po = O.make_params(n0, n1, n2, dt=dt, minRealVx=-1, maxRealVx=1)
+            if dtype == B.F64:
+                O.advect_f64(refs[j], po, nsteps)
+            else:
+                O.advect_f32_blocked(refs[j], po, nsteps, 1)
+            assert np.array_equal(arrays[j].cpu().numpy(), refs[j]), (nsteps, BATCH[j])
+    batch.close()
