@@ -6,14 +6,12 @@
 // In-place safety: y[b][:, J] overwrites x[b][:, J], which every output
 // channel still needs.  Every kernel walks columns in increasing tiles
 // [j0, j0+TN): a tile reads columns [j0, j0+TN+K-1) and writes [j0, j0+TN),
-// so reads run ahead of writes.  The direct kernels give one work-group one
-// batch element; the MFMA kernels give one work-group a contiguous chunk of
+// so reads run ahead of writes.  One work-group takes a contiguous chunk of
 // the flattened (batch, tile) sequence, and the K-1 columns past a chunk's
 // last tile are snapshotted first (conv_halo_kernel).
 //
 // Kernels
-//  - conv_direct_kernel<T>: FP64 / FP32 FMA reference kernels (FP64 keeps the
-//    oracle's order: bias, then ic outer, k inner, separate multiply/add).
+//  - the FP64 and FP32 modes: conv_direct.hip.
 //  - conv_mfma_kernel<TIO, NPROD>: implicit GEMM on v_mfma_f32_32x32x16_bf16.
 //    GEMM: Y[oc][j] = sum_r W[oc][r] X[r][j] with r = k*C + ic, so 8
 //    consecutive r are 8 consecutive channels at one tap and one ds_read_b128
@@ -37,6 +35,7 @@
 #include <vector>
 
 #include "common.hpp"
+#include "conv_direct.hpp"
 #include "mfma_ops.hpp"
 
 namespace bkma {
@@ -52,66 +51,6 @@ template <> __device__ __forceinline__ float io_to_f32<__hip_bfloat16>(__hip_bfl
 template <class T> __device__ __forceinline__ T f32_to_io(float v) { return (T)v; }
 template <> __device__ __forceinline__ __hip_bfloat16 f32_to_io<__hip_bfloat16>(float v) {
     return __builtin_bit_cast(__hip_bfloat16, (__bf16)v);  // round to nearest even (v_cvt_pk_bf16_f32)
-}
-
-// ---------------------------------------------------------------------------
-// Direct kernels (FP64 / FP32)
-// ---------------------------------------------------------------------------
-constexpr int kDirTN = 64;   // columns per tile
-constexpr int kDirOC = 4;    // output channels per thread
-constexpr int kDirJ = 8;     // columns per thread
-
-template <class T>
-__global__ __launch_bounds__(256) void conv_direct_kernel(T *__restrict__ x, const T *__restrict__ w,
-                                                          const T *__restrict__ bias, int C, int L, int K) {
-    extern __shared__ __align__(16) unsigned char lds_raw[];
-    T *xs = reinterpret_cast<T *>(lds_raw);  // [C][JW]
-    const int JW = kDirTN + K - 1;
-    const int Lout = L - K + 1;
-    T *xb = x + (i64)blockIdx.x * C * L;
-    const int t = threadIdx.x;
-    const int jb = t % (kDirTN / kDirJ);                 // 8 column blocks
-    const int ob = t / (kDirTN / kDirJ);                 // 32 channel blocks of 4
-    const int oc_groups = (C + kDirOC * 32 - 1) / (kDirOC * 32);
-    for (int j0 = 0; j0 < Lout; j0 += kDirTN) {
-        __syncthreads();
-        for (int e = t; e < C * JW; e += 256) {
-            const int ic = e / JW, jj = e - ic * JW;
-            const int j = j0 + jj;
-            xs[e] = j < L ? xb[(i64)ic * L + j] : (T)0;
-        }
-        __syncthreads();
-        for (int g = 0; g < oc_groups; ++g) {
-            const int oc0 = (g * 32 + ob) * kDirOC;
-            T acc[kDirOC][kDirJ];
-#pragma unroll
-            for (int a = 0; a < kDirOC; ++a)
-#pragma unroll
-                for (int c = 0; c < kDirJ; ++c) acc[a][c] = oc0 + a < C ? bias[oc0 + a] : (T)0;
-            for (int ic = 0; ic < C; ++ic) {
-                const T *xr = xs + ic * JW + jb * kDirJ;
-                for (int k = 0; k < K; ++k) {
-                    T wv[kDirOC];
-#pragma unroll
-                    for (int a = 0; a < kDirOC; ++a) wv[a] = oc0 + a < C ? w[((i64)(oc0 + a) * C + ic) * K + k] : (T)0;
-#pragma unroll
-                    for (int c = 0; c < kDirJ; ++c) {
-                        const T xv = xr[c + k];
-#pragma unroll
-                        for (int a = 0; a < kDirOC; ++a) acc[a][c] = acc[a][c] + wv[a] * xv;
-                    }
-                }
-            }
-            // Stores land in columns [j0, j0+TN), which no later tile reads.
-#pragma unroll
-            for (int a = 0; a < kDirOC; ++a)
-#pragma unroll
-                for (int c = 0; c < kDirJ; ++c) {
-                    const int j = j0 + jb * kDirJ + c;
-                    if (oc0 + a < C && j < Lout) xb[(i64)(oc0 + a) * L + j] = acc[a][c];
-                }
-        }
-    }
 }
 
 // ---------------------------------------------------------------------------
@@ -1142,7 +1081,7 @@ struct ConvPlan {
     bkma_conv_mode mode;
     bkma_dtype io;
     i64 B, C, L, K;
-    void *w = nullptr;      // direct modes: weights in io precision; MFMA: bf16 hi fragments
+    void *w = nullptr;      // MFMA: bf16 hi fragments
     void *wlo = nullptr;    // BF16X3: bf16 lo fragments
     void *bias = nullptr;   // direct: io precision; MFMA: f32
     void *halo = nullptr;   // MFMA: tile-boundary columns, snapshotted before each run
@@ -1150,8 +1089,10 @@ struct ConvPlan {
     float xscale = 1.0f;    // FP8: the input is quantized as x / xscale
     i64 resident_groups = 0;
     u64 lds_bytes = 0;
+    DirectConv direct;      // FP64 and FP32 modes
     std::string name;
     ~ConvPlan() {
+        direct_conv_free(direct);
         if (w) (void)hipFree(w);
         if (wlo) (void)hipFree(wlo);
         if (bias) (void)hipFree(bias);
@@ -1361,13 +1302,12 @@ extern "C" bkma_status bkma_conv1d_plan_create(bkma_conv_mode mode, bkma_dtype i
         if (io_dtype != want || w_dtype != want)
             return bail(fail(BKMA_ERR_UNSUPPORTED, "conv1d plan: F64/F32 modes take data and weights of that type"));
         const size_t esz = want == BKMA_F64 ? 8 : 4;
-        if (hipMalloc(&p->w, nw * esz) != hipSuccess || hipMalloc(&p->bias, C * esz) != hipSuccess)
+        if (hipMalloc(&p->bias, C * esz) != hipSuccess)
             return bail(fail(BKMA_ERR_OUT_OF_MEMORY, "conv1d plan: weight copy"));
-        if (hipMemcpyAsync(p->w, weight, nw * esz, hipMemcpyDeviceToDevice, s) != hipSuccess ||
-            hipMemcpyAsync(p->bias, bias, C * esz, hipMemcpyDeviceToDevice, s) != hipSuccess)
+        const bkma_status st = direct_conv_create(want, (int)B, (int)C, (int)L, (int)K, weight, s, &p->direct);
+        if (st != BKMA_OK) return bail(st);
+        if (hipMemcpyAsync(p->bias, bias, C * esz, hipMemcpyDeviceToDevice, s) != hipSuccess)
             return bail(fail(BKMA_ERR_DEVICE, "conv1d plan: weight copy"));
-        p->lds_bytes = (u64)C * (u64)(kDirTN + K - 1) * esz;
-        if (p->lds_bytes > lds_max) return bail(fail(BKMA_ERR_UNSUPPORTED, "conv1d plan: C too large for the LDS tile"));
         p->name = want == BKMA_F64 ? "conv_direct<f64>" : "conv_direct<f32>";
     } else if (mode == BKMA_CONV_BF16 || mode == BKMA_CONV_BF16X3) {
         const int nprod = mode == BKMA_CONV_BF16 ? 1 : 3;
@@ -1461,20 +1401,9 @@ extern "C" bkma_status bkma_conv1d_plan_run(bkma_conv1d_plan *p, void *x, void *
     if (!p || !x) return fail(BKMA_ERR_INVALID_ARGUMENT, "conv1d run: null argument");
     hipStream_t s = as_stream(stream);
     switch (p->mode) {
-        case BKMA_CONV_F64: {
-            auto k = conv_direct_kernel<double>;
-            BKMA_HIP_TRY(hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)p->lds_bytes));
-            hipLaunchKernelGGL(k, dim3((unsigned)p->B), dim3(256), (size_t)p->lds_bytes, s, (double *)x,
-                               (const double *)p->w, (const double *)p->bias, (int)p->C, (int)p->L, (int)p->K);
-            break;
-        }
-        case BKMA_CONV_F32: {
-            auto k = conv_direct_kernel<float>;
-            BKMA_HIP_TRY(hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)p->lds_bytes));
-            hipLaunchKernelGGL(k, dim3((unsigned)p->B), dim3(256), (size_t)p->lds_bytes, s, (float *)x,
-                               (const float *)p->w, (const float *)p->bias, (int)p->C, (int)p->L, (int)p->K);
-            break;
-        }
+        case BKMA_CONV_F64:
+        case BKMA_CONV_F32:
+            return direct_conv_run(p->direct, x, p->bias, s);
         case BKMA_CONV_BF16:
         case BKMA_CONV_BF16X3: {
             const MfmaVariant *v = find_mfma(p->io, p->mode == BKMA_CONV_BF16 ? 1 : 3, p->C, p->K, p->L);
