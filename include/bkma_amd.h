@@ -226,14 +226,15 @@ typedef struct bkma_tuned_config {
     int32_t vec;          /* consecutive i2 cells per lane (LINE_SHFL: consecutive i1 cells per lane) */
     int32_t smax;         /* largest |v*dt/dx| the stencil window covers */
     int32_t prefetch;     /* rows loaded ahead of the stencil window (LINE_LDS: 5 = five rows per thread with their
-                             coefficients in registers, lines from 16 rows on, the segment length chosen by the
-                             plan; else the coefficients are computed at every step) */
+                             coefficients in registers, 6 = strips of rows, several steps of which stay in a
+                             wavefront's registers, for the slabs with shifts -5..6; both for lines from 16 rows
+                             on, shape chosen by the plan; else the coefficients are computed at every step) */
     int32_t waves_per_wg; /* wavefronts per work-group (LINE_LDS: 4, 8 or 16; 0 = 4) */
     int32_t nontemporal;  /* 1: non-temporal global loads/stores */
     int32_t persistent;   /* 1: grid capped at the resident work-groups, waves loop over units */
     int32_t seg_rows;     /* LINE_LDS: rows per segment (0 = whole line in LDS); PLAIN, HYBRID: pref_wg_size */
     int32_t wide_window;  /* COLUMN_STREAM, F32 storage: 1 = FP64 register window (rows widened once) */
-    int32_t steps_per_pass; /* COLUMN_STREAM, COLUMN_PAIR, LINE_LDS (at most 4; 256 with prefetch = 5), LINE_SHFL (at most 256): time
+    int32_t steps_per_pass; /* COLUMN_STREAM, COLUMN_PAIR, LINE_LDS (at most 4; 256 with prefetch = 5 or 6), LINE_SHFL (at most 256): time
                                steps fused into one pass over HBM (0 or 1: one) */
     int32_t chunk_segs;   /* LINE_LDS segmented: consecutive segments one work-group walks in order (0 or 1: one);
                              LINE_LDS whole line: consecutive slabs one work-group stages together;

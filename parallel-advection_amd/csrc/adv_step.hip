@@ -110,7 +110,7 @@ const StepShape &step_shape(const AdvDev &p, u64 esz, u64 lds_max) {
         q.n0 = (u64)p.n0;
         q.n1 = (u64)p.n1;
         q.n2 = (u64)p.n2;
-        k.fits = p.n1 <= kTileRows * kTileThreads && tile_shape(q, esz, 1, lds_max, &k.tile, true);
+        k.fits = p.n1 <= kTileRows * kTileThreads && tile_shape(q, 0, q.n0, esz, 1, lds_max, &k.tile, true);
     }
     return k;
 }

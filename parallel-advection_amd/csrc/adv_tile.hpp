@@ -40,12 +40,16 @@
 // step each.
 #pragma once
 
+#include <atomic>
+#include <vector>
+
 #include "common.hpp"
 
 namespace bkma {
 
 constexpr int kTileRows = 5;               // rows per thread
 constexpr int kTileWin = kTileRows + 5;    // rows a thread's step reads
+constexpr int kStripForm = 6;  // bkma_tuned_config::prefetch of the strip form (kTileRows: of the LDS form)
 constexpr int kTileGhost = 2 * kTileRows;  // rows repeated after a whole line
 constexpr int kTileLow = kTileRows;        // SEG: rows a thread's window may start before the buffer
 constexpr int kTileThreads = 1024;         // largest work-group
@@ -62,15 +66,27 @@ struct TileArgs {
     int hb_max, ha_max;  // SEG: largest halo rows per step before and after a segment
     int hrows;           // SEG: snapshot rows per (slab, segment)
     unsigned mcb, mn1;   // ceil(2^32 / cb) (cb > 1), ceil(2^32 / n1): quotients of tile indexes (below 2^16)
+    unsigned mcw;        // ceil(2^32 / (cb / W)), W elements of 16 bytes
+    int wide;            // staged and stored 16 bytes at a time: columns and addresses allow it
+    int strips, sr;      // strip form: wavefronts per plane, rows of a strip that are its own
+    i64 s0, s1;          // the launch's slabs
     i64 units;
 };
 
+// Smallest and largest shift of slab i0: d = i1 - leftNode is ceil(s),
+// s = v dt / dx, up to the rounding of the foot (some ulps of the coordinates).
+__host__ __device__ __forceinline__ void tile_shifts(const AdvDev &p, i64 i0, double &dlo, double &dhi) {
+    const double s = (p.minRealVx + (double)(int)i0 * p.dvx) * p.dt * p.inv_dx;
+    const double e = 1e-6 + 1e-15 * (fabs(p.minRealX) + 2.0 * p.realWidthX) * p.inv_dx;
+    dlo = ceil(s - e);
+    dhi = ceil(s + e);
+}
+
 // Halo rows per step of slab i0 before and after a segment (the stencil of
-// row i1 reads rows i1-d-2 .. i1-d+3, d in [floor(s), floor(s)+1]).
+// row i1 reads rows i1-d-2 .. i1-d+3).
 __host__ __device__ __forceinline__ void tile_halo(const AdvDev &p, i64 i0, int hb_max, int ha_max, int &hb, int &ha) {
-    const double v = p.minRealVx + (double)(int)i0 * p.dvx;
-    const double s = v * p.dt * p.inv_dx;
-    const double dlo = floor(s - 1e-6), dhi = floor(s + 1e-6) + 1.0;
+    double dlo, dhi;
+    tile_shifts(p, i0, dlo, dhi);
     const double b = dhi + 2.0 > 0.0 ? dhi + 2.0 : 0.0, a = 3.0 - dlo > 0.0 ? 3.0 - dlo : 0.0;
     hb = b < (double)hb_max ? (int)b : hb_max;
     ha = a < (double)ha_max ? (int)a : ha_max;
@@ -97,8 +113,8 @@ __device__ __forceinline__ TileSeg tile_segment(const TileArgs &a, i64 i0, int s
 template <class T>
 __device__ __forceinline__ void tile_snapshot_unit(const T *__restrict__ data, T *__restrict__ halo, const TileArgs &a,
                                                    i64 unit) {
-    const i64 i0 = unit / a.nseg;
-    const TileSeg s = tile_segment(a, i0, (int)(unit - i0 * a.nseg));
+    const i64 i0 = a.s0 + unit / a.nseg;
+    const TileSeg s = tile_segment(a, i0, (int)(unit % a.nseg));
     if (s.nr <= 0) return;
     const i64 n2 = a.p.n2, line = a.p.n1 * n2;
     const T *slab = data + i0 * line;
@@ -127,6 +143,121 @@ __device__ __forceinline__ int tile_foot(const AdvDev &p, int i0, int i1, double
     return leftNode;
 }
 
+// W elements of T in one access of 16 bytes (W = 1: one element).
+template <class T, int W> struct alignas(W == 1 ? alignof(T) : 16) TilePack {
+    T v[W];
+};
+
+// Stages the tile's rows as FP64, about U elements in flight per thread.
+// WRAP: whole lines of all slabs of the tile, their first kTileGhost rows also
+// after the last; SEG: hbn halo rows, nr rows from line row r0 on, the other
+// halo rows.  W > 1: rows of 16-byte accesses, a.cb and n2 multiples of W.
+// Index arithmetic is most of what an element costs here (strips, [512][1024][512],
+// one step: FP32 0.98 ms with W = 1, 0.88 with W = 4; FP64 1.29 and 1.13 ms).
+template <class T, int U, int W, bool WRAP>
+__device__ __forceinline__ void tile_stage_w(const T *base, const T *__restrict__ hsrc, double *__restrict__ lds,
+                                             const TileArgs &a, int nrow, int cbw, int hbn, int r0, int nr) {
+    constexpr int UW = W == 1 ? U : U / 2;  // accesses in flight
+    const int n1 = (int)a.p.n1, tid = (int)threadIdx.x, nthr = (int)blockDim.x, cb = a.cb;
+    const unsigned cq = (unsigned)(cb / W), mq = W == 1 ? a.mcb : a.mcw;
+    const i64 n2 = a.p.n2;
+    const int total = nrow * (int)cq;
+#pragma unroll 1
+    for (int q0 = tid; q0 < total; q0 += UW * nthr) {
+        TilePack<T, W> ld[UW];
+#pragma unroll
+        for (int i = 0; i < UW; ++i) {
+            const unsigned q = (unsigned)(q0 + i * nthr);
+            const unsigned row = cq == 1 ? q : __umulhi(q, mq);
+            const unsigned col = (q - row * cq) * W;
+#pragma unroll
+            for (int k = 0; k < W; ++k) ld[i].v[k] = (T)0;
+            if ((int)row < nrow && (int)col < cbw) {
+                const T *src;
+                if constexpr (WRAP) {
+                    src = base + (i64)row * n2;
+                } else {
+                    const int b = (int)row - hbn;
+                    src = b >= 0 && b < nr ? base + (i64)(r0 + b) * n2 : hsrc + (i64)(b < 0 ? (int)row : (int)row - nr) * n2;
+                }
+                ld[i] = *reinterpret_cast<const TilePack<T, W> *>(src + col);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < UW; ++i) {
+            const unsigned q = (unsigned)(q0 + i * nthr);
+            unsigned row = cq == 1 ? q : __umulhi(q, mq);
+            const unsigned col = (q - row * cq) * W;
+            if ((int)row < nrow && (int)col < cbw) {
+                unsigned s = 0;
+                if constexpr (WRAP) {
+                    s = __umulhi(row, a.mn1);
+                    row -= s * (unsigned)n1;
+                }
+                double *dst = lds + (int)(s * (unsigned)cb + col) * a.pl + (int)row;
+#pragma unroll
+                for (int k = 0; k < W; ++k) dst[k * a.pl] = (double)ld[i].v[k];
+                if constexpr (WRAP) {
+                    if ((int)row < kTileGhost) {
+#pragma unroll
+                        for (int k = 0; k < W; ++k) dst[k * a.pl + n1] = (double)ld[i].v[k];
+                    }
+                }
+            }
+        }
+    }
+}
+
+// The tile's nout rows (WRAP: of all slabs; SEG: after the hbn halo rows) to
+// the array.
+template <class T, int U, int W, bool WRAP>
+__device__ __forceinline__ void tile_store_w(T *base, const double *__restrict__ src, const TileArgs &a, int nout,
+                                             int cbw, int hbn, int r0) {
+    constexpr int UW = W == 1 ? U : U / 2;
+    const int n1 = (int)a.p.n1, tid = (int)threadIdx.x, nthr = (int)blockDim.x, cb = a.cb;
+    const unsigned cq = (unsigned)(cb / W), mq = W == 1 ? a.mcb : a.mcw;
+    const i64 n2 = a.p.n2;
+    const int total = nout * (int)cq;
+#pragma unroll 1
+    for (int q0 = tid; q0 < total; q0 += UW * nthr) {
+#pragma unroll
+        for (int i = 0; i < UW; ++i) {
+            const unsigned q = (unsigned)(q0 + i * nthr);
+            const unsigned row = cq == 1 ? q : __umulhi(q, mq);
+            const unsigned col = (q - row * cq) * W;
+            if ((int)row < nout && (int)col < cbw) {
+                const double *w;
+                T *dst;
+                if constexpr (WRAP) {
+                    const unsigned s = __umulhi(row, a.mn1);
+                    w = src + (int)(s * (unsigned)cb + col) * a.pl + (int)(row - s * (unsigned)n1);
+                    dst = base + (i64)row * n2;
+                } else {
+                    w = src + (int)col * a.pl + hbn + (int)row;
+                    dst = base + (i64)(r0 + (int)row) * n2;
+                }
+                TilePack<T, W> st;
+#pragma unroll
+                for (int k = 0; k < W; ++k) st.v[k] = (T)w[k * a.pl];
+                *reinterpret_cast<TilePack<T, W> *>(dst + col) = st;
+            }
+        }
+    }
+}
+
+template <class T, int U, bool WRAP>
+__device__ __forceinline__ void tile_stage(const T *base, const T *__restrict__ hsrc, double *__restrict__ lds,
+                                           const TileArgs &a, int nrow, int cbw, int hbn, int r0, int nr) {
+    if (a.wide) tile_stage_w<T, U, 16 / sizeof(T), WRAP>(base, hsrc, lds, a, nrow, cbw, hbn, r0, nr);
+    else tile_stage_w<T, U, 1, WRAP>(base, hsrc, lds, a, nrow, cbw, hbn, r0, nr);
+}
+template <class T, int U, bool WRAP>
+__device__ __forceinline__ void tile_store(T *base, const double *__restrict__ src, const TileArgs &a, int nout, int cbw,
+                                           int hbn, int r0) {
+    if (a.wide) tile_store_w<T, U, 16 / sizeof(T), WRAP>(base, src, a, nout, cbw, hbn, r0);
+    else tile_store_w<T, U, 1, WRAP>(base, src, a, nout, cbw, hbn, r0);
+}
+
 // Six-tap sum over w[0..5].
 template <bool FUSED> __device__ __forceinline__ double tile_taps(const double (&c)[6], const double *w) {
     double acc = c[0] * w[0];
@@ -147,7 +278,7 @@ __device__ __forceinline__ void tile_unit(T *__restrict__ data, const T *__restr
     if constexpr (!WRAP) lds += kTileLow;
     const int n1 = (int)a.p.n1;
     const i64 n2 = a.p.n2;
-    const int tid = (int)threadIdx.x, nthr = (int)blockDim.x;
+    const int tid = (int)threadIdx.x;
     const int cb = a.cb, pl = a.pl, ns = a.ns;
 
     // ---- the tile ----
@@ -160,12 +291,12 @@ __device__ __forceinline__ void tile_unit(T *__restrict__ data, const T *__restr
     int hbn = 0, r0 = 0, nr = 0;
     const T *hsrc = nullptr;
     if constexpr (WRAP) {
-        i0b = grp * a.sb;
-        nsl = (int)min((i64)a.sb, a.p.n0 - i0b);
+        i0b = a.s0 + grp * a.sb;
+        nsl = (int)min((i64)a.sb, a.s1 - i0b);
         nrow = nsl * n1;
     } else {
-        i0b = grp / a.nseg;
-        const TileSeg s = tile_segment(a, i0b, (int)(grp - i0b * a.nseg));
+        i0b = a.s0 + grp / a.nseg;
+        const TileSeg s = tile_segment(a, i0b, (int)(grp % a.nseg));
         if (s.nr <= 0) return;  // uniform over the work-group
         hbn = ns * s.hb;
         r0 = s.r0;
@@ -175,46 +306,7 @@ __device__ __forceinline__ void tile_unit(T *__restrict__ data, const T *__restr
     }
     T *base = data + i0b * n1 * n2 + col0;
 
-    // ---- stage, kTileRows loads in flight per thread ----
-#pragma unroll 1
-    for (int u = 0; u < V; ++u) {
-        const int q0 = tid + u * E * nthr;
-        T ld[E];
-#pragma unroll
-        for (int i = 0; i < E; ++i) {
-            const unsigned q = (unsigned)(q0 + i * nthr);
-            const unsigned row = cb == 1 ? q : __umulhi(q, a.mcb);
-            const unsigned col = q - row * (unsigned)cb;
-            ld[i] = (T)0;
-            if ((int)row < nrow && (int)col < cbw) {
-                if constexpr (WRAP) {
-                    ld[i] = base[(i64)row * n2 + col];
-                } else {
-                    const int b = (int)row - hbn;
-                    const T *src = b >= 0 && b < nr ? base + (i64)(r0 + b) * n2 : hsrc + (i64)(b < 0 ? (int)row : (int)row - nr) * n2;
-                    ld[i] = src[col];
-                }
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < E; ++i) {
-            const unsigned q = (unsigned)(q0 + i * nthr);
-            unsigned row = cb == 1 ? q : __umulhi(q, a.mcb);
-            const unsigned col = q - row * (unsigned)cb;
-            if ((int)row < nrow && (int)col < cbw) {
-                unsigned s = 0;
-                if constexpr (WRAP) {
-                    s = __umulhi(row, a.mn1);
-                    row -= s * (unsigned)n1;
-                }
-                double *dst = lds + (int)(s * (unsigned)cb + col) * pl + (int)row;
-                dst[0] = (double)ld[i];
-                if constexpr (WRAP) {
-                    if ((int)row < kTileGhost) dst[n1] = (double)ld[i];
-                }
-            }
-        }
-    }
+    tile_stage<T, E, WRAP>(base, hsrc, lds, a, nrow, cbw, hbn, r0, nr);
     __builtin_amdgcn_sched_barrier(0);
 
     // ---- this thread's rows: feet, coefficients, window position ----
@@ -337,30 +429,13 @@ __device__ __forceinline__ void tile_unit(T *__restrict__ data, const T *__restr
     }
     if constexpr (V > 1) __syncthreads();
 
-    // ---- store ----
-    const int nout = WRAP ? nrow : nr;
-#pragma unroll 1
-    for (int u = 0; u < V; ++u) {
-#pragma unroll
-        for (int i = 0; i < E; ++i) {
-            const unsigned q = (unsigned)(tid + (u * E + i) * nthr);
-            const unsigned row = cb == 1 ? q : __umulhi(q, a.mcb);
-            const unsigned col = q - row * (unsigned)cb;
-            if ((int)row < nout && (int)col < cbw) {
-                if constexpr (WRAP) {
-                    const unsigned s = __umulhi(row, a.mn1);
-                    base[(i64)row * n2 + col] = (T)src[(int)(s * (unsigned)cb + col) * pl + (int)(row - s * (unsigned)n1)];
-                } else {
-                    base[(i64)(r0 + (int)row) * n2 + col] = (T)src[(int)col * pl + hbn + (int)row];
-                }
-            }
-        }
-    }
+    tile_store<T, E, WRAP>(base, src, a, WRAP ? nrow : nr, cbw, hbn, r0);
 }
 
-// Launch shape of one problem (host side).
+// Launch shape of the slabs [a.s0, a.s1) of one problem (host side).
 struct TileShape {
     TileArgs a{};
+    int e = 0;  // 0: the LDS form (below: V columns per thread); else the strip form with e rows per lane
     int v = 1;
     bool wrap = true;
     int threads = 0;
@@ -368,19 +443,26 @@ struct TileShape {
     u64 halo_bytes = 0;  // SEG: snapshot buffer
 };
 
-// The tile of a problem for passes of at most ns steps (ns = 0: chosen here,
-// and returned in a.ns).  False where the tile form does not fit: lines
-// shorter than 16 rows, or whose halos leave too few rows of a segment.
-// whole_only: whole lines only, which need no snapshot.
-bool tile_shape(const bkma_adv_params &p, u64 elem_size, int ns, u64 lds_max, TileShape *out, bool whole_only = false);
+// The LDS tile of the slabs [s0, s1) of a problem for passes of at most ns
+// steps (ns = 0: chosen here, and returned in a.ns).  False where it does not
+// fit: lines shorter than 16 rows, or whose halos leave too few rows of a
+// segment.  whole_only: whole lines only, which need no snapshot.
+bool tile_shape(const bkma_adv_params &p, u64 s0, u64 s1, u64 elem_size, int ns, u64 lds_max, TileShape *out,
+                bool whole_only = false);
+// The strip tile (adv_strip.hpp) of slabs whose shifts it covers.
+bool strip_shape(const bkma_adv_params &p, u64 s0, u64 s1, u64 elem_size, int ns, u64 lds_max, TileShape *out);
+// A problem's tiles for passes of ns steps (0: chosen here; the same for all
+// parts, in parts[0].a.ns): with `strips`, strips for the slabs whose shifts
+// they cover (first in the list, if there are any) and LDS tiles for the
+// others.  Empty where there are none.
+std::vector<TileShape> tile_parts(const bkma_adv_params &p, u64 elem_size, int ns, u64 lds_max, bool strips);
 
 // One pass of ns steps (at most the shape's).  `fused`: fused sums (FP32
 // storage), `rnd`: rounded to FP32 after every step.
 bkma_status launch_tile(const TileShape &sh, bkma_dtype dt, bool fused, bool rnd, void *data, void *halo, int ns,
                         hipStream_t s);
 
-// Several problems in one launch (ragged batches): problems whose tiles have
-// the same columns per thread and kind.
+// Several problems' parts in one launch (ragged batches): tiles of one kind.
 struct TileProblem {
     TileArgs a;
     void *data;
@@ -389,7 +471,7 @@ struct TileProblem {
     i64 first_halo;   // SEG: first work-group of its snapshot
 };
 struct TileGroup {
-    int v = 1;
+    int e = 0, v = 1;
     bool wrap = true;
     int threads = 0;
     u64 lds_bytes = 0;
@@ -400,5 +482,44 @@ struct TileGroup {
 };
 // One pass of ns steps (at most the group's) of every problem of the group.
 bkma_status launch_tile_group(const TileGroup &g, bkma_dtype dt, bool rnd, int ns, hipStream_t s);
+
+// The strip kernels (strip_f64.hip, strip_f32.hip, strip_f32_round.hip).
+bkma_status launch_strip_f64(const TileShape &sh, const TileArgs &a, void *data, void *halo, hipStream_t s);
+bkma_status launch_strip_f32(const TileShape &sh, const TileArgs &a, void *data, void *halo, hipStream_t s);
+bkma_status launch_strip_f32_round(const TileShape &sh, const TileArgs &a, void *data, void *halo, hipStream_t s);
+bkma_status launch_strip_group_f64(const TileGroup &g, int ns, hipStream_t s);
+bkma_status launch_strip_group_f32(const TileGroup &g, int ns, hipStream_t s);
+bkma_status launch_strip_group_f32_round(const TileGroup &g, int ns, hipStream_t s);
+
+// Consecutive tiles of one memory line (the column tiles of a slab) on one
+// XCD: work-groups go to the 8 XCDs in turn.
+__device__ __forceinline__ i64 tile_of_block(i64 b, i64 units, int nct) {
+    const i64 per = units / 8;
+    return nct > 1 && b < per * 8 ? (b % 8) * per + b / 8 : b;
+}
+
+// The last problem whose first work-group is not past b.
+template <i64 TileProblem::*FIRST> __device__ __forceinline__ int problem_of_block(const TileProblem *tab, int count, i64 b) {
+    int lo = 0, hi = count;
+    while (hi - lo > 1) {
+        const int mid = (lo + hi) / 2;
+        if (tab[mid].*FIRST <= b) lo = mid;
+        else hi = mid;
+    }
+    return lo;
+}
+
+// Allows the whole LDS to the kernel, once per device.
+template <class K> bkma_status allow_lds(K kernel, std::atomic<unsigned> &done) {
+    int dev = 0;
+    BKMA_HIP_TRY(hipGetDevice(&dev));
+    const unsigned bit = 1u << (dev & 31);
+    if (done.load(std::memory_order_relaxed) & bit) return BKMA_OK;
+    u64 lds_max = 0;
+    BKMA_TRY(lds_limit_bytes(&lds_max));
+    BKMA_HIP_TRY(hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_max));
+    done.fetch_or(bit, std::memory_order_relaxed);
+    return BKMA_OK;
+}
 
 }  // namespace bkma

@@ -330,43 +330,49 @@ static bool build_groups(AdvBatch &b) {
     if (lds_limit_bytes(&lds_max) != BKMA_OK) return false;
     const u64 esz = b.dtype == BKMA_F64 ? 8 : 4;
     const size_t n = b.problems.size();
-    std::vector<TileShape> shapes(n);
+    struct Part {
+        size_t prob;
+        TileShape t;
+    };
+    std::vector<Part> parts;
     for (size_t j = 0; j < n; ++j) {
         const bkma_adv_params &p = b.problems[j].params;
         if (!std::isfinite(p.minRealVx) || !std::isfinite(p.dvx) || !std::isfinite(p.inv_dx) ||
-            !std::isfinite(p.minRealX) || !std::isfinite(p.realWidthX) || !tile_shape(p, esz, 0, lds_max, &shapes[j]))
+            !std::isfinite(p.minRealX) || !std::isfinite(p.realWidthX))
             return false;
+        const std::vector<TileShape> ts = tile_parts(p, esz, 0, lds_max, true);
+        if (ts.empty()) return false;
+        for (const TileShape &t : ts) parts.push_back(Part{j, t});
     }
     for (void *h : b.halos) (void)hipFree(h);
     b.halos.clear();
     b.drop_groups();
-    // Problems of one kind, work-group size and depth share a launch (the
-    // largest first: its last work-groups are then the short ones).
+    // Parts of one kind, work-group size and depth share a launch (the largest
+    // first: its last work-groups are then the short ones).
     auto threads = [](const TileShape &t) { return t.threads <= 256 ? 256 : t.threads <= 512 ? 512 : kTileThreads; };
     auto same = [&](const TileShape &x, const TileShape &y) {
-        return x.v == y.v && x.wrap == y.wrap && threads(x) == threads(y) && x.a.ns == y.a.ns;
+        return x.e == y.e && (x.e || x.v == y.v) && x.wrap == y.wrap && threads(x) == threads(y) && x.a.ns == y.a.ns;
     };
-    std::vector<bool> taken(n, false);
-    std::vector<size_t> order(n);
-    for (size_t j = 0; j < n; ++j) order[j] = j;
-    auto cells = [&](size_t j) { return b.problems[j].params.n0 * b.problems[j].params.n1 * b.problems[j].params.n2; };
-    std::stable_sort(order.begin(), order.end(), [&](size_t x, size_t y) { return cells(x) > cells(y); });
+    auto cells = [](const Part &x) { return (double)(x.t.a.s1 - x.t.a.s0) * (double)x.t.a.p.n1 * (double)x.t.a.p.n2; };
+    std::stable_sort(parts.begin(), parts.end(), [&](const Part &x, const Part &y) { return cells(x) > cells(y); });
+    std::vector<bool> taken(parts.size(), false);
     bool ok = true;
-    for (size_t f : order) {
+    for (size_t f = 0; f < parts.size(); ++f) {
         if (taken[f] || !ok) continue;
         TileGroup g;
-        g.v = shapes[f].v;
-        g.wrap = shapes[f].wrap;
-        g.ns = shapes[f].a.ns;
+        g.e = parts[f].t.e;
+        g.v = parts[f].t.v;
+        g.wrap = parts[f].t.wrap;
+        g.ns = parts[f].t.a.ns;
         std::vector<TileProblem> tab;
-        for (size_t j : order) {
-            if (taken[j] || !ok || !same(shapes[f], shapes[j])) continue;
-            const TileShape &t = shapes[j];
+        for (size_t j = f; j < parts.size(); ++j) {
+            if (taken[j] || !ok || !same(parts[f].t, parts[j].t)) continue;
+            const TileShape &t = parts[j].t;
             if ((u64)(g.units + t.a.units) > 0x7fffffffULL) continue;  // a group of its own
             taken[j] = true;
             TileProblem pr{};
             pr.a = t.a;
-            pr.data = b.problems[j].data;
+            pr.data = b.problems[parts[j].prob].data;
             if (t.halo_bytes) {
                 ok = hipMalloc(&pr.halo, t.halo_bytes) == hipSuccess;
                 if (ok) b.halos.push_back(pr.halo);
@@ -374,7 +380,7 @@ static bool build_groups(AdvBatch &b) {
             pr.first = g.units;
             pr.first_halo = g.halo_units;
             g.units += t.a.units;
-            if (!t.wrap) g.halo_units += t.a.p.n0 * t.a.nseg;
+            if (!t.wrap) g.halo_units += (t.a.s1 - t.a.s0) * t.a.nseg;
             g.threads = std::max(g.threads, t.threads);
             g.lds_bytes = std::max(g.lds_bytes, t.lds_bytes);
             tab.push_back(pr);

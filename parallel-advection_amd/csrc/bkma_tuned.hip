@@ -23,6 +23,7 @@
 #include <cstring>
 #include <new>
 #include <string>
+#include <memory>
 #include <vector>
 
 #include <climits>
@@ -94,6 +95,11 @@ const std::vector<StreamVariant> &stream_variants(bkma_dtype dt) {
     return dt == BKMA_F32 ? f32 : dt == BKMA_F64 ? f64 : none;
 }
 
+// LINE_LDS with the coefficients in registers (adv_tile.hpp).
+bool is_tile(const bkma_tuned_config &c) {
+    return c.strategy == BKMA_STRATEGY_LINE_LDS && (c.prefetch == kTileRows || c.prefetch == kStripForm);
+}
+
 int steps_per_pass(const bkma_tuned_config &c) { return c.steps_per_pass > 1 ? c.steps_per_pass : 1; }
 
 // Range of the backward shift d = i1 - leftNode over the velocity grid.
@@ -139,11 +145,19 @@ struct TunedPlan {
     LdsArgs lds{};
     u64 lds_bytes = 0;
     int lds_threads = 256;  // threads per work-group: 256, 512 or 1024
-    bool tiled = false;     // LINE_LDS with the coefficients in registers (adv_tile.hpp)
-    TileShape tile{};
+    // LINE_LDS with the coefficients in registers (adv_tile.hpp, adv_strip.hpp):
+    // the tiles of consecutive slabs and their snapshot buffers (owned)
+    std::vector<TileShape> tiles;
+    std::vector<void *> tile_halos;
+    // Runs of at most few_steps steps (default plans; owned): the column pair,
+    // whose results are the same
+    std::unique_ptr<TunedPlan> few;
+    u64 few_steps = 0;
     void *halo = nullptr;  // segmented mode: halo snapshot buffer (owned)
     ~TunedPlan() {
         if (halo) (void)hipFree(halo);
+        for (void *h : tile_halos)
+            if (h) (void)hipFree(h);
         if (slab_shift) (void)hipFree(slab_shift);
         if (gscratch.data) (void)hipFree(gscratch.data);
         if (fork) (void)hipEventDestroy(fork);
@@ -445,7 +459,11 @@ bkma_status plan_launch(const TunedPlan &pl, void *data, hipStream_t s, int ns) 
         BKMA_HIP_TRY(hipStreamWaitEvent(s, pl.join, 0));
         return st;
     }
-    if (pl.tiled) return launch_tile(pl.tile, pl.dtype, true, false, data, pl.halo, ns, s);
+    if (!pl.tiles.empty()) {
+        for (size_t k = 0; k < pl.tiles.size(); ++k)
+            BKMA_TRY(launch_tile(pl.tiles[k], pl.dtype, true, false, data, pl.tile_halos[k], ns, s));
+        return BKMA_OK;
+    }
     if (pl.cfg.strategy == BKMA_STRATEGY_LINE_LDS)
         return pl.dtype == BKMA_F64 ? launch_lds<double>(pl, data, s, ns) : launch_lds<float>(pl, data, s, ns);
     if (pl.cfg.strategy == BKMA_STRATEGY_LINE_SHFL) {
@@ -475,10 +493,11 @@ bkma_status plan_launch(const TunedPlan &pl, void *data, hipStream_t s, int ns) 
 
 // nsteps steps: full passes of the plan's steps per pass, then the rest.
 bkma_status plan_steps(const TunedPlan &pl, void *data, u64 nsteps, hipStream_t s) {
+    if (pl.few && nsteps <= pl.few_steps) return plan_steps(*pl.few, data, nsteps, s);
     u64 ns = (u64)pl.ns;
     // FP64 storage of the register tiles: equal passes (the split does not
     // change the results, and a short last pass pays a whole staging)
-    if (pl.tiled && pl.dtype == BKMA_F64 && nsteps > ns) ns = ceil_div(nsteps, ceil_div(nsteps, ns));
+    if (!pl.tiles.empty() && pl.dtype == BKMA_F64 && nsteps > ns) ns = ceil_div(nsteps, ceil_div(nsteps, ns));
     for (u64 t = 0; t + ns <= nsteps; t += ns) BKMA_TRY(plan_launch(pl, data, s, (int)ns));
     if (nsteps % ns) BKMA_TRY(plan_launch(pl, data, s, (int)(nsteps % ns)));
     return BKMA_OK;
@@ -500,11 +519,15 @@ std::string lds_name(bkma_dtype dt, const LdsArgs &a, int threads) {
            (threads != 256 ? ",wg" + std::to_string(threads) : "") + ">";
 }
 
-std::string tile_name(bkma_dtype dt, const TileShape &t) {
-    return std::string("line_lds<") + (dt == BKMA_F64 ? "f64" : "f32") + ",regs" + std::to_string(kTileRows) +
-           (t.wrap ? std::string(",whole_line") + (t.a.sb > 1 ? ",slabs" + std::to_string(t.a.sb) : "")
-                   : ",seg" + std::to_string(t.a.rows - t.a.hrows)) +
-           ",cols" + std::to_string(t.a.cb) + ",steps" + std::to_string(t.a.ns) + ",wg" + std::to_string(t.threads) + ">";
+std::string tile_name(bkma_dtype dt, const std::vector<TileShape> &parts) {
+    std::string n = std::string("line_lds<") + (dt == BKMA_F64 ? "f64" : "f32") + ",steps" + std::to_string(parts[0].a.ns);
+    for (const TileShape &t : parts)
+        n += (&t == &parts[0] ? "," : "|") + std::string(t.e ? "strip" + std::to_string(t.e) + "x" + std::to_string(t.a.strips)
+                                                            : "regs" + std::to_string(kTileRows)) +
+             (t.wrap ? std::string(",whole_line") + (t.a.sb > 1 ? ",slabs" + std::to_string(t.a.sb) : "")
+                     : ",seg" + std::to_string(t.a.rows - t.a.hrows)) +
+             ",cols" + std::to_string(t.a.cb) + ",wg" + std::to_string(t.threads);
+    return n + ">";
 }
 
 // Resident work-groups on the whole device for a variant (persistent grid).
@@ -610,23 +633,27 @@ bkma_status build_plan(const bkma_adv_params &p, bkma_dtype dt, const bkma_tuned
                    std::to_string(cfg.chunk_segs) + "%>";
         return BKMA_OK;
     }
-    if (cfg.strategy == BKMA_STRATEGY_LINE_LDS && cfg.prefetch == kTileRows) {
+    if (is_tile(cfg)) {
         // coefficients in registers, where that form fits (else below)
         u64 lds_max = 0;
         BKMA_TRY(lds_limit_bytes(&lds_max));
         const int ns = steps_per_pass(cfg);
-        if (ns <= kTileMaxSteps && shift_supported(p, &why) && tile_shape(p, dt == BKMA_F64 ? 8 : 4, ns, lds_max, &pl->tile)) {
-            if (pl->tile.halo_bytes && hipMalloc(&pl->halo, pl->tile.halo_bytes) != hipSuccess) {
-                pl->halo = nullptr;
-                return fail(BKMA_ERR_OUT_OF_MEMORY, "tuned advection: halo buffer allocation failed");
+        if (ns <= kTileMaxSteps && shift_supported(p, &why)) pl->tiles = tile_parts(p, dt == BKMA_F64 ? 8 : 4, ns, lds_max, cfg.prefetch == kStripForm);
+        if (!pl->tiles.empty()) {
+            for (const TileShape &t : pl->tiles) {
+                pl->tile_halos.push_back(nullptr);
+                if (t.halo_bytes && hipMalloc(&pl->tile_halos.back(), t.halo_bytes) != hipSuccess) {
+                    pl->tile_halos.back() = nullptr;
+                    return fail(BKMA_ERR_OUT_OF_MEMORY, "tuned advection: halo buffer allocation failed");
+                }
             }
-            pl->tiled = true;
+            const TileShape &t = pl->tiles[0];
             pl->ns = ns;
             pl->cfg.steps_per_pass = ns;
-            pl->cfg.seg_rows = pl->tile.wrap ? 0 : pl->tile.a.rows - pl->tile.a.hrows;
-            pl->cfg.chunk_segs = pl->tile.a.sb;
-            pl->cfg.waves_per_wg = pl->tile.threads / 64;
-            pl->name = tile_name(dt, pl->tile);
+            pl->cfg.seg_rows = t.wrap ? 0 : t.a.rows - t.a.hrows;
+            pl->cfg.chunk_segs = t.a.sb;
+            pl->cfg.waves_per_wg = t.threads / 64;
+            pl->name = tile_name(dt, pl->tiles);
             return BKMA_OK;
         }
     }
@@ -738,13 +765,15 @@ std::vector<bkma_tuned_config> candidates(const bkma_adv_params &p, bkma_dtype d
     u64 bytes, lds_max = 0;
     if (lds_limit_bytes(&lds_max) != BKMA_OK) lds_max = 0;
     // the LDS tile with register coefficients, at its own steps per pass
-    TileShape ts;
-    if (shift_supported(p, nullptr) && tile_shape(p, esz, 0, lds_max, &ts)) {
+    for (const bool strips : {false, true}) {
+        std::vector<TileShape> ts;
+        if (shift_supported(p, nullptr)) ts = tile_parts(p, esz, 0, lds_max, strips);
+        if (ts.empty() || (strips && !ts[0].e)) continue;
         bkma_tuned_config c;
         std::memset(&c, 0, sizeof(c));
         c.strategy = BKMA_STRATEGY_LINE_LDS;
-        c.prefetch = kTileRows;
-        c.steps_per_pass = ts.a.ns;
+        c.prefetch = strips ? kStripForm : kTileRows;
+        c.steps_per_pass = ts[0].a.ns;
         out.push_back(c);
     }
     int dlo = 0, dhi = 0;
@@ -819,33 +848,70 @@ std::vector<bkma_tuned_config> candidates(const bkma_adv_params &p, bkma_dtype d
     return out;
 }
 
-// Whether the column kernels keep the GPU busy on a shape: they run one
-// wavefront per 64*VEC columns of a slab (VEC = 2 from 128 columns on), a
-// serial walk along the line, and a tile that the columns do not fill runs
-// their slow body with range checks.  Both sides measured at 1, 5 and 20
-// steps (time of the column pair over that of the LINE_LDS register tiles):
+// Part of the column tiles' lanes that are columns: one wavefront per 64*VEC
+// columns of a slab (VEC = 2 from 128 columns on), and a tile that the columns
+// do not fill runs its slow body with range checks.
+double columns_full(const bkma_adv_params &p) {
+    const u64 width = p.n2 >= 128 ? 128 : 64;
+    return (double)p.n2 / (double)(ceil_div(p.n2, width) * width);
+}
+
+// Whether the column kernels, a serial walk along the line per wavefront, keep
+// the GPU busy.  Measured at 1, 5 and 20 steps (time of the column pair over
+// that of the LINE_LDS register tiles):
 //   FP64 [n0][1000][128]: 512 wavefronts 0.8 / 1.5 / 1.9, 1024 0.8 / 1.2 / 1.2;
 //   FP64 [n0][1000][300] (a tile in three not full): 1023 wavefronts
 //     1.7 / 2.3 / 2.2, 2046 1.2 / 1.8 / 1.8;
 //   FP32 [n0][1000][128]: 256 wavefronts 0.9 / 1.4 / 2.2, 512 0.6 / 0.8 / 1.3;
 //   FP32 [n0][1000][300]: 510 wavefronts 3.2 / 1.5 / 2.3, 1023 1.7 / 0.9 / 1.4;
-// lines of 3000 rows, with narrower register tiles, move the lines down by
-// about a factor of two.
+//   FP32 [64][4096][512] (256 wavefronts), 5 and 20 steps: 1.5 / 2.3.
 bool columns_fill(const bkma_adv_params &p, bkma_dtype dt) {
     if (p.n2 < (dt == BKMA_F64 ? 64 : 128)) return false;
-    const u64 width = p.n2 >= 128 ? 128 : 64;
-    const bool even = p.n2 % width == 0;
-    u64 enough = dt == BKMA_F64 ? (even ? 1024 : 4096) : (even ? 384 : 768);
-    if (p.n1 > 2500) enough /= 2;
-    return p.n0 * ceil_div(p.n2, width) >= enough;
+    const bool even = columns_full(p) == 1.0;
+    const u64 enough = dt == BKMA_F64 ? (even ? 1024 : 4096) : (even ? 384 : 768);
+    return p.n0 * ceil_div(p.n2, p.n2 >= 128 ? 128 : 64) >= enough;
+}
+
+// Whether strips (adv_strip.hpp) beat the column pair on runs of more steps
+// than pair_steps: one pass of up to 64 steps against one per 4 (FP64) or 5
+// (FP32) steps.  Time of the pair over that of the strips at 5, 12, 20 and 50
+// steps:
+//   FP64 [512][1024][512] 1.2 / 1.2 / 1.4 / 1.6, [512][300][1000]
+//     1.5 / 1.5 / 1.7 / 2.0, [1400][1000][300] 1.8 / 1.8 / 2.1 / 2.7,
+//     [64][8192][2048] (segments) 1.1 / 1.0 / 1.2 / 1.3;
+//   FP32 [512][1024][512] 0.45 / 0.9 / 0.9 / 1.0, [128][1024][512]
+//     0.9 / - / 1.7 / 2.2, [512][300][1000] 0.7 / 1.5 / 1.4 / 1.6,
+//     [1400][1000][300] 0.8 / 1.6 / 1.6 / 1.9, [128][4096][1024] (segments)
+//     0.5 / 0.8 / 0.8 / 0.9;
+// lines that fill little of their strips' 64 E rows (E >= 4) stay with the
+// pair (FP64 [4096][100][256]: 0.8 / 0.8 / 0.9 / 1.0).
+bool strips_pay(const bkma_adv_params &p, bkma_dtype dt) {
+    if (p.n1 < 160) return false;
+    if (dt == BKMA_F64 || columns_full(p) < 1.0) return true;
+    return p.n0 * (p.n2 / 128) < 768;
+}
+
+// Steps up to which a plan of strips runs the column pair instead (results are
+// the same: FP64 whatever the passes, FP32 within one pass of the pair).  Time
+// of the pair over that of the strips at 1, 4, 5 and 8 steps: FP64
+// [512][1024][512] 0.7 / 0.7 / 1.2 / 1.0, [1024][2048][128] 0.6 / 0.6 / 1.1 /
+// 0.9, [512][300][1000] (0.98 full) 1.0 / 0.8 / 1.5 / 1.2, [1400][1000][300]
+// (0.78 full) 1.1 / 1.0 / 1.8 / 1.6; FP32 [512][300][1000] 0.8 / 0.8 / 0.7 /
+// 1.3, [1400][1000][300] 1.0 / 0.9 / 0.8 / 1.4.
+u64 pair_steps(const bkma_adv_params &p, bkma_dtype dt, const bkma_tuned_config &pair) {
+    if (!columns_fill(p, dt)) return 0;
+    const double full = columns_full(p);
+    const u64 ns = (u64)steps_per_pass(pair);
+    if (dt == BKMA_F32) return ns;
+    return full == 1.0 ? 2 * ns : full >= 0.9 ? ns : 0;
 }
 
 // Heuristic: contiguous lines that fit LINE_SHFL, with 256 steps per pass, 8
 // cells per lane from 4096 lines on (measured on [2^21][1024][1]), else 4 (on
-// [256][1024][1]); where the column kernels fill the GPU, column pair when
-// every slab has at most two shifts (FP32 with the DPP broadcast at 5, FP64
-// at 4 steps per pass), else LINE_LDS register tiles, which take every other
-// shape of lines from 16 rows on; then the column stream with the smallest
+// [256][1024][1]); where the column kernels fill the GPU and strips do not pay,
+// column pair when every slab has at most two shifts (FP32 with the DPP
+// broadcast at 5, FP64 at 4 steps per pass), else LINE_LDS register tiles,
+// which take every other shape of lines from 16 rows on; then the column stream with the smallest
 // window, the reference's executor for short lines, and LINE_LDS whole lines
 // or the longest segment.
 int heuristic_score(const bkma_tuned_config &c, bkma_dtype dt, const bkma_adv_params &p) {
@@ -876,8 +942,10 @@ int heuristic_score(const bkma_tuned_config &c, bkma_dtype dt, const bkma_adv_pa
         return 1000000000 - c.smax * 1000000 - std::abs(ns - want) * 100000 + c.vec * 1000 + c.prefetch * 10 +
                c.nontemporal - c.persistent - 100 * c.wide_window;
     }
-    if (c.strategy == BKMA_STRATEGY_LINE_LDS && c.prefetch == kTileRows)
-        return columns_fill(p, dt) ? 1050000000 : 1200000000;
+    if (is_tile(c)) {
+        const int base = c.prefetch == kStripForm ? 10000000 : 0;
+        return base + (columns_fill(p, dt) && !(base && strips_pay(p, dt)) ? 1050000000 : 1200000000);
+    }
     // LINE_LDS: whole lines; else the longest segment, with 16-wave
     // work-groups where they are offered (the segment fills the LDS)
     return c.seg_rows == 0 ? 500000000 - std::abs(steps_per_pass(c) - 2) * 1000 - c.waves_per_wg
@@ -961,15 +1029,13 @@ extern "C" bkma_status bkma_adv_plan_create(const bkma_adv_params *params, bkma_
     auto *pl = new (std::nothrow) bkma_adv_plan();
     if (!pl) return fail(BKMA_ERR_OUT_OF_MEMORY, "plan allocation");
     bkma_status st = build_plan(*params, dtype, best, pl);
-    if (st == BKMA_ERR_OUT_OF_MEMORY && best.strategy == BKMA_STRATEGY_LINE_LDS && best.prefetch == kTileRows) {
+    if (st == BKMA_ERR_OUT_OF_MEMORY && is_tile(best)) {
         // no room for the tile's halo snapshot: the best of the other plans
         (void)hipGetLastError();
         delete pl;
         pl = new (std::nothrow) bkma_adv_plan();
         if (!pl) return fail(BKMA_ERR_OUT_OF_MEMORY, "plan allocation");
-        cands.erase(std::remove_if(cands.begin(), cands.end(),
-                                   [](const auto &c) { return c.strategy == BKMA_STRATEGY_LINE_LDS && c.prefetch == kTileRows; }),
-                    cands.end());
+        cands.erase(std::remove_if(cands.begin(), cands.end(), is_tile), cands.end());
         if (!cands.empty()) {
             best = *std::max_element(cands.begin(), cands.end(), [&](const auto &a, const auto &b) {
                 return heuristic_score(a, dtype, *params) < heuristic_score(b, dtype, *params);
@@ -980,6 +1046,23 @@ extern "C" bkma_status bkma_adv_plan_create(const bkma_adv_params *params, bkma_
     if (st != BKMA_OK) {
         delete pl;
         return st;
+    }
+    if (!pl->tiles.empty()) {
+        cands.erase(std::remove_if(cands.begin(), cands.end(),
+                                   [](const auto &c) { return c.strategy != BKMA_STRATEGY_COLUMN_PAIR; }),
+                    cands.end());
+        if (!cands.empty()) {
+            const bkma_tuned_config pair = *std::max_element(cands.begin(), cands.end(), [&](const auto &a, const auto &b) {
+                return heuristic_score(a, dtype, *params) < heuristic_score(b, dtype, *params);
+            });
+            const u64 n = pair_steps(*params, dtype, pair);
+            if (n) {
+                pl->few.reset(new (std::nothrow) TunedPlan());
+                if (pl->few && build_plan(*params, dtype, pair, pl->few.get()) == BKMA_OK) pl->few_steps = n;
+                else pl->few.reset();
+                (void)hipGetLastError();
+            }
+        }
     }
     *out = pl;
     return BKMA_OK;
