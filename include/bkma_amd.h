@@ -285,7 +285,9 @@ typedef struct bkma_adv_batch bkma_adv_batch;
 /* Problems whose lines all have a LINE_LDS register tile (16 rows and more,
  * moderate shifts) run as groups of such tiles, one launch per group and as
  * many fused steps as its tiles hold, with the results of one step per pass;
- * autotune then has nothing to choose.  Otherwise autotune = 1 times the LDS
+ * long runs launch the groups on up to four streams between the caller's
+ * earlier and later work, and use_graph makes no difference (there are few
+ * launches).  autotune then has nothing to choose.  Otherwise autotune = 1 times the LDS
  * budgets (32 KB .. the device limit), work-group sizes and steps per pass
  * (1 .. 4) on the problems' own arrays, which the timing steps modify: create
  * the batch before initialising the data.  autotune = 0: 64 KB, 256 threads,

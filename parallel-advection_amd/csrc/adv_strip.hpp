@@ -144,7 +144,8 @@ __device__ __forceinline__ void strip_unit(T *data, const T *__restrict__ halo, 
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int pc = wave / a.strips, st = wave - pc * a.strips;
     const int sl = pc / a.ct, cc = pc - sl * a.ct;
-    const bool act = sl < nsl;                 // wave-uniform
+    // wave-uniform; a segment's last strips may be beyond its rows
+    const bool act = sl < nsl && (WRAP || st * R < nrow);
     if constexpr (WRAP) {
         int f;
         tile_halo(a.p, i0b + (act ? sl : 0), a.hb_max, a.ha_max, hb, f);
@@ -160,23 +161,25 @@ __device__ __forceinline__ void strip_unit(T *data, const T *__restrict__ halo, 
     int d0 = 0;
     unsigned differ = 0;  // rows whose shift is not the wave's first
     const int half = n1 / 2;
+    if (act) {
 #pragma unroll
-    for (int e = 0; e < E; ++e) {
-        int lr = r + e;
-        if constexpr (!WRAP) {
-            lr += r0 - hbn;
-            if (lr < 0) lr += n1;
+        for (int e = 0; e < E; ++e) {
+            int lr = r + e;
+            if constexpr (!WRAP) {
+                lr += r0 - hbn;
+                if (lr < 0) lr += n1;
+            }
+            if (lr >= n1) lr -= n1;
+            lr = min(max(lr, 0), n1 - 1);  // rows far outside a segment's buffer: margin
+            double d_prev1;
+            int d = lr - tile_foot(a.p, (int)(i0b + sl), lr, d_prev1);
+            adv_lag_basis(d_prev1, c[e]);
+            if (d > half) d -= n1;
+            if (d < -half) d += n1;
+            if (e == 0) d0 = __builtin_amdgcn_readfirstlane(d);
+            differ |= (unsigned)(d != d0) << e | (unsigned)(d > d0) << (16 + e);
+            __builtin_amdgcn_sched_barrier(0);  // one row's temporaries at a time
         }
-        if (lr >= n1) lr -= n1;
-        lr = min(max(lr, 0), n1 - 1);  // rows far outside a segment's buffer: margin
-        double d_prev1;
-        int d = lr - tile_foot(a.p, (int)(i0b + (act ? sl : 0)), lr, d_prev1);
-        adv_lag_basis(d_prev1, c[e]);
-        if (d > half) d -= n1;
-        if (d < -half) d += n1;
-        if (e == 0) d0 = __builtin_amdgcn_readfirstlane(d);
-        differ |= (unsigned)(d != d0) << e | (unsigned)(d > d0) << (16 + e);
-        __builtin_amdgcn_sched_barrier(0);  // one row's temporaries at a time
     }
     // two adjacent shifts at most: the window starts at the larger one's, the
     // rows of the smaller start one cell later

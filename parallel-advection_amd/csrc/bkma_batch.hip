@@ -140,6 +140,8 @@ void shift_bounds(const bkma_adv_params &p, int *dlo, int *dhi) {
 
 }  // namespace
 
+constexpr int kBatchSides = 3;  // streams beside the internal one
+
 struct AdvBatch {
     bkma_dtype dtype = BKMA_F32;
     std::vector<bkma_adv_problem> problems;
@@ -159,12 +161,16 @@ struct AdvBatch {
     std::vector<bkma_adv_plan *> plans;    // per-problem tuned plans (loop mode)
     u64 cells = 0;
     // The register tiles of adv_tile.hpp instead of the persistent launch
-    std::vector<TileGroup> groups;  // tables owned
+    std::vector<TileGroup> groups;  // tables owned; the largest first
+    std::vector<int> lane;          // stream of each group: 0 the internal stream, k side[k - 1]
+    hipStream_t side[kBatchSides] = {};  // owned, created when groups use them
+    hipEvent_t ev_fork = nullptr, ev_join[kBatchSides] = {};
     u64 tile_units = 0, tile_seg_units = 0;
 
     void drop_groups() {
         for (auto &g : groups) (void)hipFree(g.table);
         groups.clear();
+        lane.clear();
         tile_units = tile_seg_units = 0;
     }
     ~AdvBatch() {
@@ -179,6 +185,11 @@ struct AdvBatch {
         if (ev_in) (void)hipEventDestroy(ev_in);
         if (ev_out) (void)hipEventDestroy(ev_out);
         if (stream) (void)hipStreamDestroy(stream);
+        if (ev_fork) (void)hipEventDestroy(ev_fork);
+        for (hipEvent_t e : ev_join)
+            if (e) (void)hipEventDestroy(e);
+        for (hipStream_t st : side)
+            if (st) (void)hipStreamDestroy(st);
     }
 };
 
@@ -205,15 +216,34 @@ static bkma_status batch_steps(const AdvBatch &b, u64 nsteps, hipStream_t s) {
         // one step per pass in the results (FP32 storage rounds after every
         // step), as many fused steps as a group's tiles hold in the launches:
         // equal passes
-        for (const TileGroup &g : b.groups) {
+        // The groups are independent: in long runs they take turns on a few
+        // streams, so that the tails and the small groups do not leave the GPU
+        // idle (one stream -> four: 6550 -> 6240 us for 48 problems and 32
+        // steps, 400 -> 350 us for 44 small ones and 30 steps); forking and
+        // joining costs 10 to 20 us, so shorter runs stay in one (117 us against
+        // 140 for 16 problems and 9 steps).
+        const double esz = b.dtype == BKMA_F64 ? 8.0 : 4.0;
+        const double us = (double)b.cells * ((double)nsteps / 1.5e6 + 2.0 * esz / 3e6);  // at 1500 Gcell/s, 3 TB/s
+        int lanes = 1;
+        if (us > 200.0)
+            for (int l : b.lane) lanes = std::max(lanes, l + 1);
+        if (lanes > 1) BKMA_HIP_TRY(hipEventRecord(b.ev_fork, s));
+        for (int l = 1; l < lanes; ++l) BKMA_HIP_TRY(hipStreamWaitEvent(b.side[l - 1], b.ev_fork, 0));
+        bkma_status st = BKMA_OK;
+        for (size_t i = 0; i < b.groups.size() && st == BKMA_OK; ++i) {
+            const TileGroup &g = b.groups[i];
             const u64 passes = ceil_div(nsteps, (u64)g.ns);
-            for (u64 k = 0, t = 0; k < passes; ++k) {
+            for (u64 k = 0, t = 0; k < passes && st == BKMA_OK; ++k) {
                 const u64 end = nsteps * (k + 1) / passes;
-                BKMA_TRY(launch_tile_group(g, b.dtype, true, (int)(end - t), s));
+                st = launch_tile_group(g, b.dtype, true, (int)(end - t), lanes > 1 && b.lane[i] ? b.side[b.lane[i] - 1] : s);
                 t = end;
             }
         }
-        return BKMA_OK;
+        for (int l = 1; l < lanes; ++l) {  // also after an error: a capture has to be joined
+            BKMA_HIP_TRY(hipEventRecord(b.ev_join[l - 1], b.side[l - 1]));
+            BKMA_HIP_TRY(hipStreamWaitEvent(s, b.ev_join[l - 1], 0));
+        }
+        return st;
     }
     for (u64 t = 0; t < nsteps;) {
         const int k = (int)std::min<u64>((u64)b.ns, nsteps - t);
@@ -348,8 +378,10 @@ static bool build_groups(AdvBatch &b) {
     b.halos.clear();
     b.drop_groups();
     // Parts of one kind, work-group size and depth share a launch (the largest
-    // first: its last work-groups are then the short ones).
-    auto threads = [](const TileShape &t) { return t.threads <= 256 ? 256 : t.threads <= 512 ? 512 : kTileThreads; };
+    // first: its last work-groups are then the short ones).  Strips of one
+    // work-group size exactly: a wavefront without a strip holds registers (FP32
+    // batch of 44, 30 steps: 550 us with sizes up to 256 together, 410 apart).
+    auto threads = [](const TileShape &t) { return t.e ? t.threads : t.threads <= 256 ? 256 : t.threads <= 512 ? 512 : kTileThreads; };
     auto same = [&](const TileShape &x, const TileShape &y) {
         return x.e == y.e && (x.e || x.v == y.v) && x.wrap == y.wrap && threads(x) == threads(y) && x.a.ns == y.a.ns;
     };
@@ -357,6 +389,7 @@ static bool build_groups(AdvBatch &b) {
     std::stable_sort(parts.begin(), parts.end(), [&](const Part &x, const Part &y) { return cells(x) > cells(y); });
     std::vector<bool> taken(parts.size(), false);
     bool ok = true;
+    std::vector<std::pair<double, TileGroup>> built;  // with its cells
     for (size_t f = 0; f < parts.size(); ++f) {
         if (taken[f] || !ok) continue;
         TileGroup g;
@@ -365,6 +398,7 @@ static bool build_groups(AdvBatch &b) {
         g.wrap = parts[f].t.wrap;
         g.ns = parts[f].t.a.ns;
         std::vector<TileProblem> tab;
+        double sum = 0;
         for (size_t j = f; j < parts.size(); ++j) {
             if (taken[j] || !ok || !same(parts[f].t, parts[j].t)) continue;
             const TileShape &t = parts[j].t;
@@ -384,13 +418,26 @@ static bool build_groups(AdvBatch &b) {
             g.threads = std::max(g.threads, t.threads);
             g.lds_bytes = std::max(g.lds_bytes, t.lds_bytes);
             tab.push_back(pr);
+            sum += cells(parts[j]);
         }
         g.count = (int)tab.size();
         ok = ok && hipMalloc((void **)&g.table, sizeof(TileProblem) * tab.size()) == hipSuccess;
-        if (ok) b.groups.push_back(g);
+        if (ok) built.emplace_back(sum, g);
         ok = ok && hipMemcpy(g.table, tab.data(), sizeof(TileProblem) * tab.size(), hipMemcpyHostToDevice) == hipSuccess;
         b.tile_units += (u64)g.units;
         if (!g.wrap) b.tile_seg_units += (u64)g.units;
+    }
+    std::stable_sort(built.begin(), built.end(), [](const auto &x, const auto &y) { return x.first > y.first; });
+    double load[1 + kBatchSides] = {};
+    for (const auto &g : built) {
+        b.groups.push_back(g.second);
+        const int l = (int)(std::min_element(load, load + 1 + kBatchSides) - load);
+        load[l] += g.first;
+        b.lane.push_back(l);
+        if (l == 0 || b.side[l - 1]) continue;
+        ok = ok && hipStreamCreateWithFlags(&b.side[l - 1], hipStreamNonBlocking) == hipSuccess &&
+             hipEventCreateWithFlags(&b.ev_join[l - 1], hipEventDisableTiming) == hipSuccess &&
+             (b.ev_fork || hipEventCreateWithFlags(&b.ev_fork, hipEventDisableTiming) == hipSuccess);
     }
     if (!ok) {
         (void)hipGetLastError();
@@ -600,7 +647,7 @@ extern "C" bkma_status bkma_adv_batch_run(bkma_adv_batch *b, uint64_t nsteps, in
     // Order the internal stream after the caller's stream, and back.
     BKMA_HIP_TRY(hipEventRecord(b->ev_in, cs));
     BKMA_HIP_TRY(hipStreamWaitEvent(b->stream, b->ev_in, 0));
-    if (use_graph) {
+    if (use_graph && b->groups.empty()) {  // a group's pass fuses many steps: few launches, no graph
         // Graphs of kGraphSteps steps and of the remainder: at most
         // kGraphSteps graphs per batch, each captured on first use.
         const u64 full = nsteps / kGraphSteps, rem = nsteps % kGraphSteps;

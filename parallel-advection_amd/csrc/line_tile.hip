@@ -130,7 +130,7 @@ int segment_steps(const TileArgs &a, int rows, int hmax, double over) {
     int ns = 0;
     double best = 0;
     const i64 stride = std::max<i64>(1, (a.s1 - a.s0) / 256);
-    for (int k : {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64}) {
+    for (int k : {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 64}) {
         if ((i64)k * hmax * 4 > (i64)rows * 3) break;
         double cost = 0;
         for (i64 i0 = a.s0; i0 < a.s1; i0 += stride) {
@@ -269,26 +269,71 @@ bool strip_shape(const bkma_adv_params &p, u64 s0, u64 s1, u64 elem_size, int ns
     a.nseg = 1;
     a.mn1 = magic(n1);
     const int hmax = halo_bounds(a);
-    // Whole lines.  Rows per lane, strips, columns and slabs that keep the
-    // most lanes at useful rows and the most wavefronts resident: a strip's
-    // margins, the exchange after m steps (about one step), two DPP moves per
-    // neighbour cell (10 per lane and step), the feet (shared by a wave's
-    // columns), SIMDs with one or two wavefronts (latency), work-groups too few
-    // to be in different phases.  Over all shapes of eleven problems of 64 to
-    // 3000 rows the choice is within 6% of the fastest, save [1000][300][1] (24
-    // us; two 256-row strips of two slabs 17).
+    // What a shape is worth: the part of the lanes' rows that are rows of the
+    // line, and the time lost to the exchange after m steps (a step or two,
+    // eight where no other work-group runs beside it), the two DPP moves per
+    // neighbour cell (10 per lane and step), the feet (shared by the `cols / ct`
+    // columns of a wave), SIMDs with one or two wavefronts (latency),
+    // work-groups too few to be in different phases, wavefronts that the SIMDs
+    // do not share evenly, idle CUs of the last round, narrow rows.
+    auto worth = [&](int e, int strips, double rows, int m, int cols, int ct, int sb, u64 units, u64 lds) {
+        const double taps = elem_size == 8 ? 11.0 : 6.0;
+        const int waves = sb * strips * ct, resident = e == 8 ? 12 : e == 6 ? 16 : 20;
+        const u64 groups = std::max<u64>(std::min<u64>({lds_max / lds, (u64)(resident / waves), ceil_div(units, 256)}), 1);
+        const double per_simd = (double)groups * waves / 4.0, depth = std::ceil(per_simd);
+        const double busy = (depth <= 1 ? 0.6 : depth <= 2 ? 0.74 : depth <= 3 ? 0.86 : depth <= 4 ? 0.95 : 1.0) * per_simd / depth;
+        const double apart = 1.0 - 0.25 / (double)groups - 0.01 * (waves - 1) - (groups <= 2 && waves % 4 ? 0.15 : 0.0);
+        const double fill = (double)n2 / ((double)ceil_div(n2, (u64)cols) * ct * ceil_div((u64)cols, (u64)ct));
+        const double line = (u64)cols == n2 ? 1.0 : std::min(1.0, 0.9 + 0.1 * cols * (double)elem_size / 32.0);
+        const double cus = (double)units / (256.0 * ceil_div(units, 256));
+        const bool wide = cols % (16 / (int)elem_size) == 0 && n2 % (16 / elem_size) == 0;
+        return rows * m / (m + 0.5 + 8.0 / (double)groups) * taps / (taps + 10.0 / e) * busy * apart * fill * line * cus *
+               (wide || n2 == 1 ? 1.0 : 0.93) / (1.0 + 0.2 * ct / cols);
+    };
     double best = 0;
+    // Segments: four strips of 384 rows with four steps between exchanges, up
+    // to four columns one after the other (best or within 3% of it on five
+    // problems, over 2 to 8 strips of 256 to 512 rows, 2 to 12 steps, 1 to 8
+    // columns).  The rows of all steps' halos are computed too.
+    const int sr = 64 * kStripSegE - 4 * hmax;
+    if ((u64)(4 * sr) < n1) {
+        sh.wrap = false;
+        sh.e = kStripSegE;
+        a.ct = 1;
+        a.strips = 4;
+        a.nct = (int)ceil_div(n2, (u64)4);
+        a.cb = (int)ceil_div(n2, (u64)a.nct);
+        a.sr = sr;
+        a.rows = 4 * sr;
+        a.pl = plane_pitch(a.rows + 2 * 4 * hmax, a.cb);
+        set_columns(a, (u64)a.cb, elem_size);
+        sh.threads = 64 * a.strips;
+        sh.lds_bytes = ((u64)a.cb * a.pl + 4 * (u64)hmax) * 8;
+        if (sh.lds_bytes <= lds_max && set_segments(sh, ns > 0 ? ns : segment_steps(a, a.rows, hmax, 16.0), hmax, elem_size)) {
+            const u64 len = ceil_div(n1, (u64)a.nseg) + (u64)a.hrows;
+            const double rows = (double)n1 / ((double)a.nseg * ceil_div(len, (u64)sr) * 64 * kStripSegE);
+            best = 0.95 * worth(sh.e, 4, rows, 4, a.cb, 1, 1, (u64)a.units, sh.lds_bytes);  // the snapshot
+            *out = sh;
+        }
+    }
+    // Whole lines.  Over all shapes of eleven problems of 64 to 3000 rows the
+    // choice is within 6% of the fastest, save [1000][300][1] (24 us; two
+    // 256-row strips of two slabs 17).  Segments win from about 2500 rows on: at
+    // 20 steps and [n][n1][8], FP64, whole 0.55 ms and segments 0.61 with 2000
+    // rows, 0.80 and 0.52 with 2500, 0.65 and 0.55 with 3500.
+    sh.wrap = true;
+    sh.halo_bytes = 0;
+    a.nseg = 1;
+    a.hrows = 0;
     for (int e : {8, 6, 4}) {
         const int reach = 64 * e;
-        const int resident_waves = e == 8 ? 12 : e == 6 ? 16 : 20;
         if (reach <= hmax) continue;
         const int least = (int)std::min<u64>(ceil_div(n1, (u64)(reach - hmax)), 99);
         for (int strips = least; strips <= std::min(least + 2, kStripMaxThreads / 64); ++strips) {
-            const int sr = (int)ceil_div(n1, (u64)strips);
-            const int m = (reach - sr) / hmax;
+            const int own = (int)ceil_div(n1, (u64)strips);
+            const int m = (reach - own) / hmax;
             if (m < 1) continue;
-            const double taps = elem_size == 8 ? 11.0 : 6.0;
-            const double rows = (double)n1 / ((double)strips * reach) * m / (m + 1.0) * taps / (taps + 10.0 / e);
+            if (strips > least && (reach - (int)ceil_div(n1, (u64)least)) / hmax >= 16) break;  // few exchanges already
             for (int ct = 1; strips * ct * 64 <= kStripMaxThreads && (u64)ct <= n2; ++ct) {
                 for (int v = 1; v <= 4 && (u64)(v - 1) * ct < n2; ++v) {
                     const u64 nct = ceil_div(n2, (u64)ct * v);
@@ -298,22 +343,12 @@ bool strip_shape(const bkma_adv_params &p, u64 s0, u64 s1, u64 elem_size, int ns
                         const u64 b = (u64)sb * cols * pitch * 8;
                         const u64 units = ceil_div(n0, (u64)sb) * nct;
                         if (b > lds_max || units > 0x7fffffffULL) continue;
-                        const int waves = sb * strips * ct;
-                        const u64 groups = std::max<u64>(std::min<u64>({lds_max / b, (u64)(resident_waves / waves), ceil_div(units, 256)}), 1);
-                        const double per_simd = (double)groups * waves / 4.0, depth = std::ceil(per_simd);
-                        const double busy = (depth <= 1 ? 0.6 : depth <= 2 ? 0.8 : depth <= 3 ? 0.93 : 1.0) * per_simd / depth;
-                        const double apart = 1.0 - 0.25 / (double)groups - 0.01 * (waves - 1);  // phases that overlap
-                        const double fill = (double)n2 / ((double)nct * ct * ceil_div((u64)cols, (u64)ct));
-                        const double line = (u64)cols == n2 ? 1.0 : std::min(1.0, 0.9 + 0.1 * cols * (double)elem_size / 32.0);
-                        const double cus = (double)units / (256.0 * ceil_div(units, 256));  // idle CUs of the last round
-                        const bool wide = cols % (16 / (int)elem_size) == 0 && n2 % (16 / elem_size) == 0;
-                        const double score = (wide || n2 == 1 ? 1.0 : 0.93) * cus * rows * busy * apart * fill * line / (1.0 + 0.2 / v);
+                        const double score = worth(e, strips, (double)n1 / ((double)strips * reach), m, cols, ct, sb, units, b);
                         if (score <= best * 1.001) continue;
                         best = score;
                         sh.e = e;
-                        sh.wrap = true;
                         a.strips = strips;
-                        a.sr = sr;
+                        a.sr = own;
                         a.ct = ct;
                         a.sb = sb;
                         a.cb = cols;
@@ -323,40 +358,15 @@ bool strip_shape(const bkma_adv_params &p, u64 s0, u64 s1, u64 elem_size, int ns
                         a.ns = ns > 0 ? ns : 64;
                         a.units = (i64)units;
                         set_columns(a, (u64)cols, elem_size);
-                        sh.threads = 64 * waves;
+                        sh.threads = 64 * sb * strips * ct;
                         sh.lds_bytes = b;
+                        *out = sh;
                     }
                 }
             }
         }
     }
-    if (best > 0) {
-        *out = sh;
-        return true;
-    }
-    // Segments: four strips of 384 rows with four steps between exchanges, up
-    // to four columns one after the other (best or within 3% of it on five
-    // problems, over 2 to 8 strips of 256 to 512 rows, 2 to 12 steps, 1 to 8
-    // columns).
-    sh.wrap = false;
-    sh.e = kStripSegE;
-    a.sb = 1;
-    a.ct = 1;
-    a.strips = 4;
-    a.nct = (int)ceil_div(n2, (u64)4);
-    a.cb = (int)ceil_div(n2, (u64)a.nct);
-    a.sr = 64 * sh.e - 4 * hmax;
-    const int slack = 64 * sh.e - a.sr;
-    a.rows = a.strips * a.sr;
-    a.pl = plane_pitch(a.rows + 2 * slack, a.cb);
-    set_columns(a, (u64)a.cb, elem_size);
-    sh.threads = 64 * a.strips * a.ct;
-    sh.lds_bytes = (u64)a.cb * a.pl * 8 + (u64)slack * 8;
-    if ((u64)a.rows >= n1 || sh.lds_bytes > lds_max) return false;
-    if (ns <= 0) ns = segment_steps(a, a.rows, hmax, 12.0);
-    if (!set_segments(sh, ns, hmax, elem_size)) return false;
-    *out = sh;
-    return true;
+    return best > 0;
 }
 
 std::vector<TileShape> tile_parts(const bkma_adv_params &p, u64 elem_size, int ns, u64 lds_max, bool strips) {

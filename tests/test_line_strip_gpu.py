@@ -117,3 +117,38 @@ def test_step_on_an_address_between_16_bytes(cuda, dtype):
     torch.cuda.synchronize()
     (O.advect_f32_plain if dtype == B.F32 else O.advect_f64)(host, po, 1)
     assert np.array_equal(d.cpu().numpy(), host) and buf[0].item() == 0 and buf[-1].item() == 0
+
+
+# Tiles of many kinds and sizes: several launches per pass, and enough work that they take turns on several streams.
+LANES = [(300, 1000, 4, 1e-3), (40, 6000, 1, 1e-3), (2000, 64, 2, 1e-3), (60, 777, 8, 1e-3), (100, 200, 16, 1e-3),
+         (9, 3000, 33, 1e-3), (30, 6000, 2, 3e-3)]
+
+
+@pytest.mark.parametrize("dtype", [B.F64, B.F32], ids=["f64", "f32"])
+def test_batch_on_several_streams_stays_between_the_callers_work(cuda, dtype):
+    """A long run of a batch between a copy into its arrays and one out of them, on a stream of the caller's, twice."""
+    import torch
+    npdt, tdt = (np.float64, torch.float64) if dtype == B.F64 else (np.float32, torch.float32)
+    arrays = [torch.empty(c[:3], dtype=tdt, device="cuda") for c in LANES]
+    params = [B.make_params(*c[:3], dt=c[3], minRealVx=-1, maxRealVx=1) for c in LANES]
+    batch = B.AdvBatch(arrays, params, dtype)
+    hosts = [O.uniform(a.numel(), 50 + j, npdt).reshape(tuple(a.shape)) for j, a in enumerate(arrays)]
+    sources = [torch.from_numpy(h).cuda() for h in hosts]
+    torch.cuda.synchronize()
+    s, got = torch.cuda.Stream(), []
+    for _ in range(2):
+        with torch.cuda.stream(s):
+            for a, src in zip(arrays, sources):
+                a.copy_(src)
+            batch.run(130, stream=s)
+            got.append([a.clone() for a in arrays])
+    torch.cuda.synchronize()
+    batch.close()
+    for j, (c, ref) in enumerate(zip(LANES, hosts)):
+        po = O.make_params(*c[:3], dt=c[3], minRealVx=-1, maxRealVx=1)
+        if dtype == B.F64:
+            O.advect_f64(ref, po, 130)
+        else:
+            O.advect_f32_blocked(ref, po, 130, 1)
+        for g in got:
+            assert np.array_equal(g[j].cpu().numpy(), ref), j
