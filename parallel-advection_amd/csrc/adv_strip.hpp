@@ -16,8 +16,9 @@
 //
 // The window's first offset -d-2 is the same for all rows of a wavefront and a
 // compile-time constant of the body that it selects.  A wavefront whose rows
-// round to two shifts runs a body that picks each row's own six cells from a
-// window of seven.
+// round to two shifts (slabs of shifts around an integer, such as the one at
+// rest) runs a body that sums a row's own six cells out of a window of seven:
+// 17 instructions per row instead of 11 (FP64).
 #pragma once
 
 #include "adv_shfl.hpp"
@@ -38,7 +39,8 @@ template <int H> __device__ __forceinline__ double strip_shift(double x) {
 }
 
 // g = one step of this lane's E cells f; windows start at offset DMIN.  MIXED:
-// rows with their bit of `up` set start one cell later.
+// rows with their bit of `up` set (late rows) start one cell later; their
+// coefficients are turned by one, the last one first.
 template <bool FUSED, int E, int DMIN, bool MIXED>
 __device__ __forceinline__ void strip_step(const double (&f)[E], double (&g)[E], const double (&c)[E][6], unsigned up) {
     constexpr int NW = E + 5 + (MIXED ? 1 : 0);
@@ -49,16 +51,41 @@ __device__ __forceinline__ void strip_step(const double (&f)[E], double (&g)[E],
         constexpr int hop = o >= 0 ? o / E : -((-o + E - 1) / E);
         w[t] = strip_shift<hop>(f[o - hop * E]);
     });
+    if constexpr (MIXED) {
+        // c[e][0] is the first tap of an early row and the last of a late one;
+        // -0.0 + x is x for every x
 #pragma unroll
-    for (int e = 0; e < E; ++e) {
-        if constexpr (MIXED) {
-            double v[6];
+        for (int e = 0; e < E; ++e) {
             const bool late = (up >> e) & 1;
+            const double first = c[e][0] * w[e];
+            double acc = late ? -0.0 : first;
 #pragma unroll
-            for (int k = 0; k < 6; ++k) v[k] = late ? w[e + k + 1] : w[e + k];
-            g[e] = tile_taps<FUSED>(c[e], v);
-        } else {
-            g[e] = tile_taps<FUSED>(c[e], w + e);
+            for (int k = 1; k < 6; ++k) acc = FUSED ? fma(c[e][k], w[e + k], acc) : acc + c[e][k] * w[e + k];
+            const double last = FUSED ? fma(c[e][0], w[e + 6], acc) : acc + c[e][0] * w[e + 6];
+            g[e] = late ? last : acc;
+        }
+    } else {
+        // a few rows tap by tap: FP64 results are ready after two issue slots
+        constexpr int G = E % 3 == 0 ? 3 : 4;
+#pragma unroll
+        for (int e0 = 0; e0 < E; e0 += G) {
+#pragma unroll
+            for (int k = 0; k < 6; ++k) {
+                double t[G];
+#pragma unroll
+                for (int e = 0; e < G; ++e) {
+                    const double x = w[e0 + e + k];
+                    if (k == 0) g[e0 + e] = c[e0 + e][0] * x;
+                    else if constexpr (FUSED) g[e0 + e] = fma(c[e0 + e][k], x, g[e0 + e]);
+                    else t[e] = c[e0 + e][k] * x;
+                }
+                if constexpr (!FUSED) {
+#pragma unroll
+                    for (int e = 0; e < G; ++e)
+                        if (k > 0) g[e0 + e] = g[e0 + e] + t[e];
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
         }
     }
 }
@@ -186,6 +213,16 @@ __device__ __forceinline__ void strip_unit(T *data, const T *__restrict__ halo, 
     const bool mixed = __any(differ != 0);
     const int dmax = __any((differ >> 16) != 0) ? d0 + 1 : d0;
     const unsigned up = dmax > d0 ? ~(differ >> 16) : differ & 0xffffu;
+    if (mixed) {
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            const bool late = (up >> e) & 1;
+            const double c5 = c[e][5];
+#pragma unroll
+            for (int k = 5; k > 0; --k) c[e][k] = late ? c[e][k - 1] : c[e][k];
+            c[e][0] = late ? c5 : c[e][0];
+        }
+    }
     const int dmin = min(max(-dmax - 2, -kStripDHi - 2), -kStripDLo - 2);
     __syncthreads();
 

@@ -149,10 +149,10 @@ struct TunedPlan {
     // the tiles of consecutive slabs and their snapshot buffers (owned)
     std::vector<TileShape> tiles;
     std::vector<void *> tile_halos;
-    // Runs of at most few_steps steps (default plans; owned): the column pair,
-    // whose results are the same
-    std::unique_ptr<TunedPlan> few;
-    u64 few_steps = 0;
+    // Default plans: runs of alt_min to alt_max steps take another plan with
+    // the same results (owned)
+    std::unique_ptr<TunedPlan> alt;
+    u64 alt_min = 1, alt_max = 0;
     void *halo = nullptr;  // segmented mode: halo snapshot buffer (owned)
     ~TunedPlan() {
         if (halo) (void)hipFree(halo);
@@ -493,7 +493,7 @@ bkma_status plan_launch(const TunedPlan &pl, void *data, hipStream_t s, int ns) 
 
 // nsteps steps: full passes of the plan's steps per pass, then the rest.
 bkma_status plan_steps(const TunedPlan &pl, void *data, u64 nsteps, hipStream_t s) {
-    if (pl.few && nsteps <= pl.few_steps) return plan_steps(*pl.few, data, nsteps, s);
+    if (pl.alt && nsteps >= pl.alt_min && nsteps <= pl.alt_max) return plan_steps(*pl.alt, data, nsteps, s);
     u64 ns = (u64)pl.ns;
     // FP64 storage of the register tiles: equal passes (the split does not
     // change the results, and a short last pass pays a whole staging)
@@ -953,6 +953,38 @@ int heuristic_score(const bkma_tuned_config &c, bkma_dtype dt, const bkma_adv_pa
                                  (c.waves_per_wg == 16 ? 5 : 0);
 }
 
+// The other plan of a default plan, and the step counts that take it (max = 0:
+// none): the column pair for short runs of strips (pair_steps), and strips for
+// long runs of few contiguous lines.  A LINE_SHFL line exchanges the cells at
+// its wavefronts' ends at every step, and with one line or less per CU nothing
+// hides it; FP64, [n0][n1][1], LINE_SHFL / strips, us: [256][1024] 20 steps
+// 9.0 / 10.0, 100 steps 33.2 / 26.3, [256][512] 100 steps 28.2 / 19.6,
+// [256][2048] 41.5 / 38.2, but [512][1024] 38.5 / 38.2.
+struct Alternative {
+    bkma_tuned_config cfg{};
+    u64 min = 1, max = 0;
+};
+Alternative alternative(const bkma_adv_params &p, bkma_dtype dt, const TunedPlan &pl,
+                        const std::vector<bkma_tuned_config> &cands) {
+    Alternative a;
+    const bool shfl = pl.cfg.strategy == BKMA_STRATEGY_LINE_SHFL && pl.cfg.vec != 1 && p.n0 <= 256;
+    if (pl.tiles.empty() && !shfl) return a;
+    const bkma_tuned_config *best = nullptr;
+    for (const auto &c : cands) {
+        if (shfl ? !(is_tile(c) && c.prefetch == kStripForm) : c.strategy != BKMA_STRATEGY_COLUMN_PAIR) continue;
+        if (!best || heuristic_score(*best, dt, p) < heuristic_score(c, dt, p)) best = &c;
+    }
+    if (!best) return a;
+    a.cfg = *best;
+    if (!shfl) {
+        a.max = pair_steps(p, dt, *best);
+    } else if (steps_per_pass(*best) == pl.ns) {  // FP32: the same passes
+        a.min = 33;
+        a.max = ~(u64)0;
+    }
+    return a;
+}
+
 bkma_status time_plan(const TunedPlan &pl, void *buf, int reps, hipStream_t s, float *ms) {
     hipEvent_t e0, e1;
     BKMA_HIP_TRY(hipEventCreate(&e0));
@@ -1047,21 +1079,15 @@ extern "C" bkma_status bkma_adv_plan_create(const bkma_adv_params *params, bkma_
         delete pl;
         return st;
     }
-    if (!pl->tiles.empty()) {
-        cands.erase(std::remove_if(cands.begin(), cands.end(),
-                                   [](const auto &c) { return c.strategy != BKMA_STRATEGY_COLUMN_PAIR; }),
-                    cands.end());
-        if (!cands.empty()) {
-            const bkma_tuned_config pair = *std::max_element(cands.begin(), cands.end(), [&](const auto &a, const auto &b) {
-                return heuristic_score(a, dtype, *params) < heuristic_score(b, dtype, *params);
-            });
-            const u64 n = pair_steps(*params, dtype, pair);
-            if (n) {
-                pl->few.reset(new (std::nothrow) TunedPlan());
-                if (pl->few && build_plan(*params, dtype, pair, pl->few.get()) == BKMA_OK) pl->few_steps = n;
-                else pl->few.reset();
-                (void)hipGetLastError();
-            }
+    if (const auto alt = alternative(*params, dtype, *pl, cands); alt.max) {
+        pl->alt.reset(new (std::nothrow) TunedPlan());
+        if (pl->alt && build_plan(*params, dtype, alt.cfg, pl->alt.get()) == BKMA_OK) {
+            pl->alt_min = alt.min;
+            pl->alt_max = alt.max;
+            pl->name += "+" + pl->alt->name;
+        } else {
+            pl->alt.reset();
+            (void)hipGetLastError();
         }
     }
     *out = pl;

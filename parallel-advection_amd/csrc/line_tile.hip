@@ -216,7 +216,7 @@ bool tile_shape(const bkma_adv_params &p, u64 s0, u64 s1, u64 elem_size, int ns,
                     a.pl = pitch;
                     a.rows = (int)n1;
                     a.nct = (int)ceil_div(n2, (u64)cols);
-                    a.ns = ns > 0 ? ns : 64;  // staging and feet cost about 4 steps
+                    a.ns = ns > 0 ? ns : kTileMaxSteps;  // staging and feet cost about 4 steps
                     a.units = (i64)units;
                     sh.threads = waves * 64;
                     sh.lds_bytes = b;
@@ -355,7 +355,7 @@ bool strip_shape(const bkma_adv_params &p, u64 s0, u64 s1, u64 elem_size, int ns
                         a.nct = (int)nct;
                         a.pl = pitch;
                         a.rows = (int)n1;
-                        a.ns = ns > 0 ? ns : 64;
+                        a.ns = ns > 0 ? ns : kTileMaxSteps;
                         a.units = (i64)units;
                         set_columns(a, (u64)cols, elem_size);
                         sh.threads = 64 * sb * strips * ct;

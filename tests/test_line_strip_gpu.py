@@ -152,3 +152,12 @@ def test_batch_on_several_streams_stays_between_the_callers_work(cuda, dtype):
             O.advect_f32_blocked(ref, po, 130, 1)
         for g in got:
             assert np.array_equal(g[j].cpu().numpy(), ref), j
+
+
+@pytest.mark.parametrize("dtype", [B.F64, B.F32], ids=["f64", "f32"])
+@pytest.mark.parametrize("n0,n1", [(5, 512), (256, 1024)])
+def test_default_plan_of_few_lines(cuda, dtype, n0, n1):
+    """Few contiguous lines: runs on both sides of the line between LINE_SHFL and strips, and beyond one pass."""
+    for n in (32, 33, 257):
+        cfg, name = _check((n0, n1, 1), dtype, n, 1, explicit=False, dt=1e-3, minRealVx=-1, maxRealVx=1)
+        assert name.startswith("line_shfl<") and "strip" in name and cfg.steps_per_pass == 256
