@@ -427,6 +427,7 @@ const void *mfma_kernel_of(int mb, int nb) {
     if (mb == 2)
         return nb == 8 ? (const void *)conv_mfma32_kernel<2, 8>
                        : nb == 4 ? (const void *)conv_mfma32_kernel<2, 4> : (const void *)conv_mfma32_kernel<2, 2>;
+    if (mb == 3) return (const void *)conv_mfma32_kernel<3, 2>;  // one group: the waves split 128 columns
     return nb == 8 ? (const void *)conv_mfma32_kernel<1, 8>
                    : nb == 4 ? (const void *)conv_mfma32_kernel<1, 4> : (const void *)conv_mfma32_kernel<1, 2>;
 }
@@ -474,7 +475,7 @@ bkma_status direct_conv_create(bkma_dtype dt, int B, int C, int L, int K, const 
     d.mfma = dt == BKMA_F32 && C >= 12;
     u64 wcount = 0;
     if (d.mfma) {
-        d.ocb = C > 16 ? 2 : 1;
+        d.ocb = C <= 16 ? 1 : C > 32 && C <= 48 && K <= 64 ? 3 : 2;  // three blocks of 16 channels instead of two times two
         d.groups = (int)ceil_div((u64)C, (u64)(16 * d.ocb));
         d.parts = d.groups >= 4 ? 1 : d.groups >= 2 ? 2 : 4;
         const u64 rows = ceil_div((u64)C, 4) * 4;
@@ -520,11 +521,16 @@ bkma_status direct_conv_create(bkma_dtype dt, int B, int C, int L, int K, const 
         wcount = (u64)d.groups * C * K * d.ocb;
     }
     if (!d.mfma && !d.lane) {
-        // channels per thread: the fewest padded channels, then the fewest groups
+        // channels per thread: padded channels times what one of them costs, an
+        // LDS read shared by o of them included (FP64 [2659][11][771], K = 5:
+        // 239 us with one channel, 177 with six of twelve)
         int best = 0;
+        double least = 0;
         for (int o : {8, 6, 5, 4, 3, 2, 1}) {
-            const int padded = (C + o - 1) / o * o;
-            if (!best || padded < (C + best - 1) / best * best) best = o;
+            const double cost = (double)((C + o - 1) / o * o) * (2.0 + 1.5 / o);
+            if (best && cost >= least) continue;
+            best = o;
+            least = cost;
         }
         d.ocb = best;
         d.groups = (C + best - 1) / best;
@@ -667,7 +673,8 @@ template <class T> bkma_status run_direct(const DirectConv &d, T *x, const T *bi
     }
     if constexpr (sizeof(T) == 4) {
         if (d.mfma) {
-            if (d.ocb == 2) launch_mfma_nb<2>(d, x, bias, s);
+            if (d.ocb == 3) launch_mfma<3, 2>(d, x, bias, s);
+            else if (d.ocb == 2) launch_mfma_nb<2>(d, x, bias, s);
             else launch_mfma_nb<1>(d, x, bias, s);
             return check_launch("conv_mfma32_kernel");
         }

@@ -76,3 +76,24 @@ def test_values_that_are_not_finite_stay_in_their_windows(cuda, mode, shape):
     want = np.zeros_like(inf)
     want[0, :, 70 - K + 1:71] = True
     assert np.array_equal(inf, want) and not torch.isnan(x).any()
+
+
+# Three blocks of 16 channels (FP32, 33 to 48) up to the longest kernel of the form and beyond it; channel counts
+# that no number of channels per thread divides.
+THREE_BLOCKS = [(3, 33, 70, 1), (200, 40, 301, 3), (2, 48, 1030, 5), (1, 47, 400, 64), (1, 48, 400, 65)]
+ODD = [(300, 7, 300, 5), (40, 11, 513, 3), (9, 13, 129, 2)]
+
+
+@pytest.mark.parametrize("mode,shape", [(B.CONV_F32, s) for s in THREE_BLOCKS + ODD[:2]] + [(B.CONV_F64, s) for s in ODD],
+                         ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
+def test_channel_splits(cuda, mode, shape):
+    got, ref, x, w, b = _run(mode, shape)
+    if mode == B.CONV_F64:
+        assert np.array_equal(got, ref)
+        return
+    Bn, C, L, K = shape
+    S = np.abs(x).astype(np.float64)
+    O.conv_torch_f64(S, np.abs(w).astype(np.float64), np.abs(b).astype(np.float64))
+    n = L - K + 1
+    err = np.abs(got[:, :, :n].astype(np.float64) - ref[:, :, :n])
+    assert np.all(err <= (C * K + 2) * 2.0 ** -24 * S[:, :, :n])
