@@ -212,27 +212,49 @@ def check(status: int) -> None:
 # ---------------------------------------------------------------------------
 # Helpers over torch tensors
 # ---------------------------------------------------------------------------
+# A step of a small array takes the GPU 5 us, so the helpers of a call build no
+# objects that they can do without: addresses and streams go through ctypes as
+# integers, and the current stream is asked for by handle where torch offers it
+# (adv_run on [256][1024][1], host time per call: 8.3 -> 5.2 us).
+_DTYPES = {}
+_raw_stream = None
+
+
 def _torch():
     import torch
     return torch
 
 
 def dtype_code(t) -> int:
-    torch = _torch()
-    return {torch.float64: F64, torch.float32: F32, torch.bfloat16: BF16}[t.dtype]
+    if not _DTYPES:
+        torch = _torch()
+        _DTYPES.update({torch.float64: F64, torch.float32: F32, torch.bfloat16: BF16})
+    return _DTYPES[t.dtype]
 
 
 def _ptr(t):
     if t is None:
         return None
     assert t.is_cuda and t.is_contiguous(), "BKMA arrays are contiguous device tensors"
-    return ctypes.c_void_p(t.data_ptr())
+    return t.data_ptr()
+
+
+def _current_stream_of():
+    """A function that returns the handle of the current device's current stream."""
+    torch = _torch()
+    raw, device = getattr(torch._C, "_cuda_getCurrentRawStream", None), torch.cuda.current_device
+    if raw is None:
+        return lambda: torch.cuda.current_stream().cuda_stream
+    return lambda: raw(device())
 
 
 def _stream(stream=None):
-    torch = _torch()
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return ctypes.c_void_p(s.cuda_stream)
+    global _raw_stream
+    if stream is not None:
+        return stream.cuda_stream
+    if _raw_stream is None:
+        _raw_stream = _current_stream_of()
+    return _raw_stream()
 
 
 def make_params(n0, n1, n2, dt=1e-4, minRealX=0.0, maxRealX=1.0, minRealVx=0.0, maxRealVx=1.0,
@@ -264,9 +286,12 @@ def scratch_extents(impl, optim, n0, n1, n2, window):
     return tuple(x.value for x in e)
 
 
+_NO_SPAN = Span3d(None, 0, 0, 0)
+
+
 def _span(scratch, extents=None):
     if scratch is None:
-        return Span3d(None, 0, 0, 0)
+        return _NO_SPAN
     e = extents if extents is not None else tuple(scratch.shape)
     return Span3d(ctypes.c_void_p(scratch.data_ptr()), *e)
 
@@ -397,7 +422,7 @@ class AdvBatch:
         n = len(arrays)
         probs = (AdvProblem * n)()
         for j, (a, p) in enumerate(zip(arrays, params)):
-            probs[j].data = _ptr(a).value
+            probs[j].data = _ptr(a)
             probs[j].params = p
         self.arrays = list(arrays)
         self._h = ctypes.c_void_p()

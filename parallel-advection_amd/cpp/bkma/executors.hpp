@@ -184,10 +184,16 @@ template <class T, class Solver> struct WholeStep {
 inline Status lds_limit(u64 *bytes) {
     int dev = 0;
     BKMA_EXEC_TRY(hip_status(hipGetDevice(&dev), "hipGetDevice"));
-    int v = 0;
-    BKMA_EXEC_TRY(hip_status(hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, dev),
-                             "hipDeviceGetAttribute"));
-    *bytes = (u64)v;
+    static thread_local int known = -1;  // the device whose limit `limit` is
+    static thread_local u64 limit = 0;
+    if (dev != known) {
+        int v = 0;
+        BKMA_EXEC_TRY(hip_status(hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, dev),
+                                 "hipDeviceGetAttribute"));
+        limit = (u64)v;
+        known = dev;
+    }
+    *bytes = limit;
     return Status{};
 }
 

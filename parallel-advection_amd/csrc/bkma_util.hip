@@ -37,10 +37,13 @@ bkma_status check_launch(const char *what) {
 }
 
 bkma_status require_device() {
+    static thread_local bool seen = false;  // the devices of a process do not go away
+    if (seen) return BKMA_OK;
     int n = 0;
     hipError_t e = hipGetDeviceCount(&n);
     if (e != hipSuccess || n == 0)
         return fail(BKMA_ERR_DEVICE, "no HIP device available (this library has no CPU fallback)");
+    seen = true;
     return BKMA_OK;
 }
 
