@@ -985,18 +985,24 @@ Alternative alternative(const bkma_adv_params &p, bkma_dtype dt, const TunedPlan
     return a;
 }
 
+// Time per step of full passes, of at most kTimedSteps steps: the staging of a
+// pass of up to 256 steps weighs as in a run of a few tens (FP32
+// [2048][1024][512], 50 steps: column pair 18.3 ms, strips 18.6, which passes
+// of 256 steps would favour by a tenth).
+constexpr int kTimedSteps = 48;
 bkma_status time_plan(const TunedPlan &pl, void *buf, int reps, hipStream_t s, float *ms) {
+    const int ns = std::min(pl.ns, kTimedSteps);
     hipEvent_t e0, e1;
     BKMA_HIP_TRY(hipEventCreate(&e0));
     BKMA_HIP_TRY(hipEventCreate(&e1));
-    bkma_status st = plan_launch(pl, buf, s, pl.ns);  // warm-up
+    bkma_status st = plan_launch(pl, buf, s, ns);  // warm-up
     if (st == BKMA_OK) {
         (void)hipEventRecord(e0, s);
-        for (int r = 0; r < reps && st == BKMA_OK; ++r) st = plan_launch(pl, buf, s, pl.ns);
+        for (int r = 0; r < reps && st == BKMA_OK; ++r) st = plan_launch(pl, buf, s, ns);
         (void)hipEventRecord(e1, s);
         (void)hipEventSynchronize(e1);
         (void)hipEventElapsedTime(ms, e0, e1);
-        *ms /= (float)(reps * pl.ns);  // per step
+        *ms /= (float)(reps * ns);  // per step
     }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
