@@ -246,7 +246,10 @@ typedef struct bkma_tuned_config {
 typedef struct bkma_adv_plan bkma_adv_plan;
 
 /* autotune = 0: heuristic choice; 1: time the feasible variants on a scratch
- * array of the same line shape (allocated and freed inside the call). */
+ * array of the same line shape (allocated and freed inside the call).  Either
+ * may hold a second kernel with the same results for short or for long runs;
+ * the plan's name then gives both, joined by a plus, and its configuration the
+ * first. */
 bkma_status bkma_adv_plan_create(const bkma_adv_params *params, bkma_dtype dtype, int32_t autotune, void *stream,
                                  bkma_adv_plan **out);
 /* A plan with an explicit configuration (BKMA_ERR_UNSUPPORTED if it is not
@@ -267,9 +270,9 @@ int32_t bkma_adv_plan_variants(bkma_dtype dtype, bkma_tuned_config *out, int32_t
 /* ------------------------------------------------------------------ */
 /* Many independent problems (each its own [n0][n1][n2] array, dt and
  * velocity grid; the reference runs one bkma_run per problem and step)
- * advanced together: every pass of ns steps (the batch's steps per pass,
- * 1 .. 4) is one persistent launch over all problems' work items (plus a
- * halo-snapshot launch when a problem's lines exceed the LDS budget), and
+ * advanced together: as groups of LINE_LDS tiles (bkma_adv_batch_create), or
+ * with every pass of ns steps (the batch's steps per pass, 1 .. 4) as one persistent launch over all problems' work items (plus a
+ * halo-snapshot launch when a problem's lines exceed the LDS budget), which
  * bkma_adv_batch_run(use_graph = 1) captures the passes into hipGraphs,
  * replayed on later calls.  A run of nsteps steps makes nsteps / ns passes of
  * ns steps, then one pass of the rest.  Results are bit-identical to running

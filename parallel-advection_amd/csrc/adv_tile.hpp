@@ -15,7 +15,8 @@
 //    one, so a window never wraps inside.  A pass may fuse any number of
 //    steps.
 //  - SEG tiles hold a segment of a longer line and the halo rows that the
-//    pass's steps reach (per slab: |s| + 6 rows per step), every row of the
+//    pass's steps reach (per slab: 5 rows per step, |s| + 3 where the shift
+//    leaves the stencil on one side), every row of the
 //    buffer is computed at every step and the rows next to the ends, which
 //    read outside the buffer, are discarded as the halo shrinks.  Rows that
 //    other work-groups overwrite in the same pass come from a snapshot.
@@ -26,11 +27,12 @@
 // What bounds it: at 20 steps on [512][1024][512] the VALU is 58% and the LDS
 // 55% busy (FP32 storage 45% and 64%), with two work-groups per CU whose
 // barriers alternate the two.  Measured (steps kernel before -> this one):
-//   [300][1000][100]    FP64, 20 steps   2.93 -> 0.57 ms (column pair before)
-//   [4096][10000][1]    FP64, 20 steps  11.68 -> 0.70 ms
-//   [256][262144][4]    FP32, 20 steps  12.93 -> 7.4 ms (halo rows are 28% of
+//   [300][1000][100]    FP64, 20 steps   2.93 -> 0.45 ms (column pair before)
+//   [4096][10000][1]    FP64, 20 steps  11.68 -> 0.67 ms
+//   [256][262144][4]    FP32, 20 steps  12.93 -> 6.4 ms (halo rows are 28% of
 //                       a tile there, the shifts reach 262 cells)
-//   [512][1024][512]    20 steps        1240 Gcell/s FP64, 1480 FP32
+//   [512][1024][512]    20 steps        1440 Gcell/s FP64, 1620 FP32
+// Slabs with shifts of a few cells take the strips of adv_strip.hpp instead.
 // Rows of one thread that round to different shifts (a slab whose shift is an
 // integer up to rounding) take a form that reads every row's own six taps.
 //

@@ -1,8 +1,8 @@
 // Ragged batches of independent advection problems.
 //
-// Where every problem has a tile of adv_tile.hpp, the batch runs those: the
-// problems whose tiles are of one kind, work-group size and depth share a
-// launch, and a launch fuses as many steps as the depth, the values rounded
+// Where every problem has tiles (adv_tile.hpp, adv_strip.hpp), the batch runs
+// those: the slab ranges whose tiles are of one kind, work-group size and depth
+// share a launch, and a launch fuses as many steps as the depth, the values rounded
 // to FP32 after every step (FP32 storage), so that the results are those of
 // one step per pass.  Otherwise, and for an explicit configuration, one
 // persistent launch per pass:

@@ -7,8 +7,10 @@
 // Strategy COLUMN_PAIR: the column stream for slabs whose rows take at most
 // two adjacent shifts (adv_pair.hpp): seven-tap windows, no shift branches.
 // Strategy LINE_LDS (any n2, any shift): slabs or segments of them staged in
-// LDS: with the coefficients in registers (adv_tile.hpp, lines from 16 rows
-// on), or computed at every step (adv_lds.hpp, up to 4 steps per pass).
+// LDS: with the coefficients in registers (lines from 16 rows on; the steps in
+// LDS, adv_tile.hpp, or several of them in a wavefront's registers,
+// adv_strip.hpp), or computed at every step (adv_lds.hpp, up to 4 steps per
+// pass).
 // Strategy LINE_SHFL (contiguous lines, n2 = 1, of 256 k <= 4096 cells, or
 // of 16): each line held in registers by one work-group (or one 16-lane row)
 // for a pass of up to 256 steps, stencil neighbours through DPP wavefront
