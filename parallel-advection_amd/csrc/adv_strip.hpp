@@ -164,7 +164,7 @@ __device__ __forceinline__ void strip_unit(T *data, const T *__restrict__ halo, 
         m = max(1, slack / (s.hb + s.ha));
     }
     T *base = data + i0b * n1 * n2 + col0;
-    tile_stage<T, U, WRAP>(base, hsrc, lds, a, nrow, cbw, hbn, r0, nr);
+    tile_stage<T, U, WRAP>(a.apart ? halo + i0b * n1 * n2 + col0 : base, hsrc, lds, a, nrow, cbw, hbn, r0, nr);
 
     // ---- this wave's strip ----
     const int lane = (int)threadIdx.x & 63;

@@ -71,6 +71,7 @@ struct TileArgs {
     unsigned mcw;        // ceil(2^32 / (cb / W)), W elements of 16 bytes
     int wide;            // staged and stored 16 bytes at a time: columns and addresses allow it
     int strips, sr;      // strip form: wavefronts per plane, rows of a strip that are its own
+    int apart;           // rows come from another array (the kernels' `halo`), nothing is overwritten
     i64 s0, s1;          // the launch's slabs
     i64 units;
 };
@@ -178,6 +179,10 @@ __device__ __forceinline__ void tile_stage_w(const T *base, const T *__restrict_
                 const T *src;
                 if constexpr (WRAP) {
                     src = base + (i64)row * n2;
+                } else if (a.apart) {
+                    int lr = r0 - hbn + (int)row;
+                    lr += lr < 0 ? n1 : lr >= n1 ? -n1 : 0;
+                    src = base + (i64)lr * n2;
                 } else {
                     const int b = (int)row - hbn;
                     src = b >= 0 && b < nr ? base + (i64)(r0 + b) * n2 : hsrc + (i64)(b < 0 ? (int)row : (int)row - nr) * n2;
@@ -308,7 +313,7 @@ __device__ __forceinline__ void tile_unit(T *__restrict__ data, const T *__restr
     }
     T *base = data + i0b * n1 * n2 + col0;
 
-    tile_stage<T, E, WRAP>(base, hsrc, lds, a, nrow, cbw, hbn, r0, nr);
+    tile_stage<T, E, WRAP>(a.apart ? halo + i0b * n1 * n2 + col0 : base, hsrc, lds, a, nrow, cbw, hbn, r0, nr);
     __builtin_amdgcn_sched_barrier(0);
 
     // ---- this thread's rows: feet, coefficients, window position ----
@@ -460,9 +465,10 @@ bool strip_shape(const bkma_adv_params &p, u64 s0, u64 s1, u64 elem_size, int ns
 std::vector<TileShape> tile_parts(const bkma_adv_params &p, u64 elem_size, int ns, u64 lds_max, bool strips);
 
 // One pass of ns steps (at most the shape's).  `fused`: fused sums (FP32
-// storage), `rnd`: rounded to FP32 after every step.
+// storage), `rnd`: rounded to FP32 after every step.  `from`: the array to read
+// (of the same extents; no snapshot), else `data` in place.
 bkma_status launch_tile(const TileShape &sh, bkma_dtype dt, bool fused, bool rnd, void *data, void *halo, int ns,
-                        hipStream_t s);
+                        hipStream_t s, void *from = nullptr);
 
 // Several problems' parts in one launch (ragged batches): tiles of one kind.
 struct TileProblem {

@@ -423,15 +423,21 @@ std::vector<TileShape> tile_parts(const bkma_adv_params &p, u64 elem_size, int n
 }
 
 bkma_status launch_tile(const TileShape &sh, bkma_dtype dt, bool fused, bool rnd, void *data, void *halo, int ns,
-                        hipStream_t s) {
+                        hipStream_t s, void *from) {
     if (ns < 1 || ns > sh.a.ns) return fail(BKMA_ERR_RUNTIME, "LINE_LDS tiles: steps per pass out of range");
     TileArgs a = sh.a;
     a.ns = ns;
     if ((uintptr_t)data % 16 != 0) a.wide = 0;
+    if (from) {
+        a.apart = 1;
+        halo = from;
+    }
     if (!sh.wrap) {  // fewer steps: smaller halos, longer segments (the snapshot keeps its row stride)
         const int h = a.hrows / sh.a.ns;
         a.nseg = (int)ceil_div((u64)a.p.n1, (u64)(a.rows - ns * h));
         a.units = (a.s1 - a.s0) * a.nseg * a.nct;
+    }
+    if (!sh.wrap && !from) {
         const unsigned groups = (unsigned)((a.s1 - a.s0) * a.nseg);
         const unsigned nt = (i64)a.hrows * a.p.n2 >= 512 ? 256 : 64;
         if (dt == BKMA_F64)

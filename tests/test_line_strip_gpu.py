@@ -161,3 +161,12 @@ def test_default_plan_of_few_lines(cuda, dtype, n0, n1):
     for n in (32, 33, 257):
         cfg, name = _check((n0, n1, 1), dtype, n, 1, explicit=False, dt=1e-3, minRealVx=-1, maxRealVx=1)
         assert name.startswith("line_shfl<") and "strip" in name and cfg.steps_per_pass == 256
+
+
+@pytest.mark.parametrize("dtype", [B.F64, B.F32], ids=["f64", "f32"])
+@pytest.mark.parametrize("shape,lo,hi", [((3, 20000, 4), -100.0, 100.0), ((13, 6000, 3), -4.0, 30.0)], ids=["tiles", "both"])
+@pytest.mark.parametrize("nsteps", [4, 5, 8, 12, 13])
+def test_passes_through_a_second_array(cuda, dtype, shape, lo, hi, nsteps):
+    """Large shifts, four steps per pass: one pass, even and odd numbers of passes, a shorter last one."""
+    _, name = _check(shape, dtype, nsteps, 4, dt=1.0 / shape[1], minRealVx=lo, maxRealVx=hi)
+    assert "seg" in name and ("strip" in name) == (lo == -4.0)
