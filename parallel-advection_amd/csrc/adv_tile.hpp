@@ -29,8 +29,9 @@
 // barriers alternate the two.  Measured (steps kernel before -> this one):
 //   [300][1000][100]    FP64, 20 steps   2.93 -> 0.45 ms (column pair before)
 //   [4096][10000][1]    FP64, 20 steps  11.68 -> 0.67 ms
-//   [256][262144][4]    FP32, 20 steps  12.93 -> 6.4 ms (halo rows are 28% of
-//                       a tile there, the shifts reach 262 cells)
+//   [256][262144][4]    FP32, 20 steps  12.93 -> 5.7 ms (halo rows are 28% of
+//                       a tile there, the shifts reach 262 cells; 6.4 ms with
+//                       a snapshot in every pass)
 //   [512][1024][512]    20 steps        1440 Gcell/s FP64, 1620 FP32
 // Slabs with shifts of a few cells take the strips of adv_strip.hpp instead.
 // Rows of one thread that round to different shifts (a slab whose shift is an
