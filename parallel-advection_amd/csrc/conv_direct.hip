@@ -23,7 +23,7 @@
 // pass the 16 KB scalar cache, and a wait for LDS waits for them too
 // ([256][128][4096], K = 5: 18.4 ms with it, 6.9 ms = 24.8 TFLOP/s here).
 //
-// conv_mfma32_kernel (FP32, C >= 12).  v_mfma_f32_16x16x4_f32 keeps FP32
+// conv_mfma32_kernel (FP32, 12 channels and more but for some that pad much).  v_mfma_f32_16x16x4_f32 keeps FP32
 // products and sums (partial sums of 160 products are added up separately: the
 // error against FP64 is half that of one long FP32 sum); its rate is twice that of the VALU without packed math.
 // Waves split the output channels (blocks of 16) and, when there are few, the
@@ -472,32 +472,52 @@ bkma_status direct_conv_create(bkma_dtype dt, int B, int C, int L, int K, const 
     const int Lout = L - K + 1;
     u64 lds_max = 0;
     BKMA_TRY(lds_limit_bytes(&lds_max));
-    d.mfma = dt == BKMA_F32 && C >= 12;
+    // FP32: the matrix cores where 16 channels, or 32, do not pad too much
+    // ([B][C][1000], K = 5, matrix cores / VALU, us: C = 12 39 / 33, 16 33 / 42,
+    // 17 55 / 40, 20 53 / 50, 24 51 / 55, 32 53 / 72)
+    // (kernels so long that only the narrowest tile fits stay with it, and so do
+    // few columns, [81][18][1152], K = 1: 7.3 / 11.9, and K = 3, 57 / 52 to 60 / 64)
+    const bool pads = (C == 12 || (C >= 17 && C <= 20 && K >= 5)) && (u64)B * (u64)Lout >= (1u << 18);
+    d.mfma = dt == BKMA_F32 && C >= 12 && (!pads || K > 1024);
     u64 wcount = 0;
     if (d.mfma) {
         d.ocb = C <= 16 ? 1 : C > 32 && C <= 48 && K <= 64 ? 3 : 2;  // three blocks of 16 channels instead of two times two
         d.groups = (int)ceil_div((u64)C, (u64)(16 * d.ocb));
         d.parts = d.groups >= 4 ? 1 : d.groups >= 2 ? 2 : 4;
         const u64 rows = ceil_div((u64)C, 4) * 4;
-        // widest tile of 128, 64 or 32 columns (at most 8 blocks a wave) that
-        // leaves room for two work-groups per CU, else that fits
-        auto bytes = [&](int tn, int *pitch) {
-            *pitch = tn + K - 1 + ((16 - (tn + K - 1)) % 64 + 64) % 64;  // 16 banks modulo 64
-            return rows * (u64)*pitch * esz;
-        };
-        for (u64 room : {lds_max / 2, lds_max}) {
-            for (int tn : {128, 64, 32}) {
-                const int nb = tn / 16 / d.parts;
-                if (d.TN || nb > 8 || nb < 2) continue;
-                if (tn > 32 && tn / 2 >= Lout && nb > 2) continue;  // half of the tile would stay empty
-                int pitch;
-                const u64 b = bytes(tn, &pitch);
-                if (b > room) continue;
-                d.TN = tn;
-                d.jt = nb;
-                d.pitch = pitch;
-                d.lds_bytes = b;
-            }
+        // Tiles of 128, 64 or 32 columns (at most 8 blocks a wave): the rounds
+        // of the resident work-groups, their share of a CU, the tile's columns
+        // and what narrower tiles lose (weights are read once per tile).  FP32,
+        // 128 -> 64 columns, us: [256][128][4096], K = 5: 1546 -> 1773;
+        // [65][128][1000], 520 tiles of 128 on 512 work-groups: 208 -> 181;
+        // [344][128][190], K = 1: 71 -> 55.
+        int cus = 0, dev = 0;
+        if (hipGetDevice(&dev) != hipSuccess ||
+            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+            return fail(BKMA_ERR_DEVICE, "conv1d plan: device query");
+        double least = 0;
+        for (int tn : {128, 64, 32}) {
+            const int nb = tn / 16 / d.parts;
+            if (nb > 8 || nb < 2) continue;
+            if (tn > 32 && tn / 2 >= Lout && nb > 2) continue;  // half of the tile would stay empty
+            const int pitch = tn + K - 1 + ((16 - (tn + K - 1)) % 64 + 64) % 64;  // 16 banks modulo 64
+            const u64 b = rows * (u64)pitch * esz;
+            if (b > lds_max) continue;
+            const void *kern = mfma_kernel_of(d.ocb, nb);
+            int blocks = 0;
+            if (hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_max) != hipSuccess ||
+                hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, kern, 256, (size_t)b) != hipSuccess)
+                return fail(BKMA_ERR_DEVICE, "conv1d plan: occupancy query");
+            blocks = std::max(blocks, 1);
+            const u64 all = ceil_div((u64)Lout, (u64)tn) * (u64)B;
+            const double cost = (double)ceil_div(all, (u64)blocks * (u64)cus) * blocks * tn *
+                                (tn == 128 ? 1.0 : tn == 64 ? 1.1 : 1.6) * (blocks == 1 ? 1.3 : 1.0);
+            if (d.TN && cost >= least) continue;
+            least = cost;
+            d.TN = tn;
+            d.jt = nb;
+            d.pitch = pitch;
+            d.lds_bytes = b;
         }
         if (!d.TN) d.mfma = false;  // too many channels for the padded tile
         wcount = ((u64)d.groups * (rows / 4) * K + kMfmaPad) * d.ocb * 64;

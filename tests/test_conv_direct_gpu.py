@@ -97,3 +97,20 @@ def test_channel_splits(cuda, mode, shape):
     n = L - K + 1
     err = np.abs(got[:, :, :n].astype(np.float64) - ref[:, :, :n])
     assert np.all(err <= (C * K + 2) * 2.0 ** -24 * S[:, :, :n])
+
+
+# Around the channel counts that leave the matrix cores (12, 17 to 21), kernels beyond 1024 among them, and tiles of
+# 128, 64 and 32 columns on work-groups that they fill unevenly.
+FORMS = [(9, 12, 300, 3), (1, 12, 1100, 1030), (4, 17, 200, 5), (3, 21, 130, 1), (3, 22, 131, 3), (1, 20, 1060, 1025),
+         (70, 128, 1000, 2), (344, 64, 190, 1), (5, 99, 300, 3), (1, 300, 40, 3)]
+
+
+@pytest.mark.parametrize("shape", FORMS, ids=lambda s: "x".join(map(str, s)))
+def test_f32_forms_within_their_sum_bound(cuda, shape):
+    got, ref, x, w, b = _run(B.CONV_F32, shape)
+    Bn, C, L, K = shape
+    S = np.abs(x).astype(np.float64)
+    O.conv_torch_f64(S, np.abs(w).astype(np.float64), np.abs(b).astype(np.float64))
+    n = L - K + 1
+    err = np.abs(got[:, :, :n].astype(np.float64) - ref[:, :, :n])
+    assert np.all(err <= (C * K + 2) * 2.0 ** -24 * S[:, :, :n])
