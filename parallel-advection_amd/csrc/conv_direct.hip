@@ -4,8 +4,10 @@
 // A tile of TN columns of one batch element is staged in LDS with the K-1
 // columns after it, then every output channel of it is computed and stored;
 // an owner (a wavefront, two, or a work-group) takes a chunk of consecutive
-// tiles in increasing order, so a tile's neighbour is still unwritten, except
-// for the last tile of a chunk, whose K-1 neighbour columns are copied first.
+// tiles in increasing order, so the columns after a tile are still unwritten
+// as far as the chunk goes.  The K-1 columns after a chunk belong to another
+// owner: they are copied first, and every tile that reaches past its chunk (with
+// K-1 > TN not only the last) takes them from the copy.
 //
 // conv_valu_kernel (FP64; FP32 with few channels).  A lane holds JT columns
 // and OCB output channels of its wave's channel group.  The weights of a tap
@@ -75,20 +77,18 @@ __global__ void conv_pack_mfma32_kernel(const float *__restrict__ w, int C, int 
     }
 }
 
-// Neighbour columns of every chunk's last tile (none for a row's last tile).
+// The K-1 columns after every chunk (none where it ends with a row).
 template <class T>
 __global__ void conv_owner_halo_kernel(const T *__restrict__ x, T *__restrict__ halo, int C, int L, int K, int TN,
                                        int tiles, int total, int chunk) {
     const int c = blockIdx.x;
-    const int last = min((c + 1) * chunk, total) - 1;
-    if (last < c * chunk) return;
-    const int b = last / tiles, t = last - b * tiles;
-    if (t >= tiles - 1) return;
+    const ConvChunk ck = conv_chunk(c, chunk, total, tiles, TN);
+    if (ck.end <= ck.first || ck.b < 0) return;
     const int H = K - 1;
     for (int e = threadIdx.x; e < C * H; e += blockDim.x) {
         const int ic = e / H, kk = e - ic * H;
-        const int j = (t + 1) * TN + kk;
-        halo[(i64)c * C * H + e] = j < L ? x[((i64)b * C + ic) * L + j] : (T)0;
+        const int j = ck.j + kk;
+        halo[(i64)c * C * H + e] = j < L ? x[((i64)ck.b * C + ic) * L + j] : (T)0;
     }
 }
 
@@ -122,18 +122,19 @@ __device__ __forceinline__ void stage_columns(const T *__restrict__ xb, T *__res
     }
 }
 
+// hsnap: the owner's copy of the columns after its chunk ck.
 template <class T>
-__device__ __forceinline__ void stage_tile(const T *__restrict__ xb, const T *__restrict__ hsnap, T *__restrict__ xs,
-                                           int C, int rows, int L, int j0, int tsh, int H, int pitch, bool vec, int t,
-                                           int nt) {
+__device__ __forceinline__ void stage_tile(const T *__restrict__ xb, const T *__restrict__ hsnap, const ConvChunk &ck,
+                                           int b, T *__restrict__ xs, int C, int rows, int L, int j0, int tsh, int H,
+                                           int pitch, bool vec, int t, int nt) {
     const int TN = 1 << tsh;
     // the H columns after the tile, from the snapshot or the row
     for (int e = t; e < rows * H; e += nt) {
-        const int row = e / H, col = e - row * H;
+        const int row = e / H, col = e - row * H, j = j0 + TN + col;
         T v = (T)0;
         if (row < C) {
-            if (hsnap) v = hsnap[e];
-            else if (j0 + TN + col < L) v = xb[(i64)row * L + j0 + TN + col];
+            if (ck.copied(b, j)) v = hsnap[row * H + (j - ck.j)];
+            else if (j < L) v = xb[(i64)row * L + j];
         }
         xs[row * pitch + TN + col] = v;
     }
@@ -154,16 +155,15 @@ __global__ __launch_bounds__(256) void conv_valu_kernel(T *__restrict__ x, const
     const int owner = (int)blockIdx.x * (4 / wpt) + slot;
     T *xs = reinterpret_cast<T *>(conv_lds) + (i64)slot * C * pitch;
     const int Lout = L - K + 1;
-    const int first = owner * chunk, end = min(first + chunk, total);
+    const ConvChunk ck = conv_chunk(owner, chunk, total, tiles, TN);
     for (int it = 0; it < chunk; ++it) {  // the same count for all waves: the barriers are uniform
-        const int tile = first + it;
-        const bool on = tile < end;
+        const int tile = ck.first + it;
+        const bool on = tile < ck.end;
         const int b = tile / tiles, t = tile - b * tiles;
         const int j0 = t * TN;
         T *xb = x + (i64)b * C * L;
         if (on) {
-            const bool snap = tile == end - 1 && t < tiles - 1;
-            stage_tile(xb, snap ? halo + (i64)owner * C * (K - 1) : (const T *)nullptr, xs, C, C, L, j0,
+            stage_tile(xb, halo + (i64)owner * C * (K - 1), ck, b, xs, C, C, L, j0,
                        JT == 4 ? 8 : JT == 2 ? 7 : 6, K - 1, pitch, vec, ws * 64 + lane, wpt * 64);
         }
         __syncthreads();
@@ -238,14 +238,13 @@ __global__ __launch_bounds__(256) void conv_lane64_kernel(double *__restrict__ x
     const int ol = lane & (cw - 1), part = lane / cw;
     const int span = JT * (64 / cw);  // columns of a wavefront
     const int blocks = TN / span;
-    const int first = (int)blockIdx.x * chunk, end = min(first + chunk, total);
-    for (int tile = first; tile < end; ++tile) {
+    const ConvChunk ck = conv_chunk((int)blockIdx.x, chunk, total, tiles, TN);
+    for (int tile = ck.first; tile < ck.end; ++tile) {
         const int b = tile / tiles, t = tile - b * tiles;
         const int j0 = t * TN;
         double *xb = x + (i64)b * C * L;
-        const bool snap = tile == end - 1 && t < tiles - 1;
-        stage_tile(xb, snap ? halo + (i64)blockIdx.x * C * (KT - 1) : (const double *)nullptr, xs, C, C, L, j0, tsh,
-                   KT - 1, pitch, vec, (int)threadIdx.x, 256);
+        stage_tile(xb, halo + (i64)blockIdx.x * C * (KT - 1), ck, b, xs, C, C, L, j0, tsh, KT - 1, pitch, vec,
+                   (int)threadIdx.x, 256);
         __syncthreads();
         for (int item = wave; item < groups * blocks; item += 4) {
             const int g = item / blocks, blk = item - g * blocks;
@@ -304,14 +303,13 @@ __global__ __launch_bounds__(256) void conv_mfma32_kernel(float *__restrict__ x,
     const int TN = 1 << tsh, Lout = L - K + 1;
     const int c4 = (C + 3) / 4, steps = c4 * K;
     const int lc = lane & 15, lr = lane >> 4;
-    const int first = (int)blockIdx.x * chunk, end = min(first + chunk, total);
-    for (int tile = first; tile < end; ++tile) {
+    const ConvChunk ck = conv_chunk((int)blockIdx.x, chunk, total, tiles, TN);
+    for (int tile = ck.first; tile < ck.end; ++tile) {
         const int b = tile / tiles, t = tile - b * tiles;
         const int j0 = t * TN;
         float *xb = x + (i64)b * C * L;
-        const bool snap = tile == end - 1 && t < tiles - 1;
-        stage_tile(xb, snap ? halo + (i64)blockIdx.x * C * (K - 1) : (const float *)nullptr, xs, C, 4 * c4, L, j0, tsh,
-                   K - 1, pitch, vec, (int)threadIdx.x, 256);
+        stage_tile(xb, halo + (i64)blockIdx.x * C * (K - 1), ck, b, xs, C, 4 * c4, L, j0, tsh, K - 1, pitch, vec,
+                   (int)threadIdx.x, 256);
         __syncthreads();
         for (int item = wave; item < groups * parts; item += 4) {
             const int g = item / parts, part = item - g * parts;

@@ -20,8 +20,27 @@ struct DirectConv {
     unsigned grid = 0;
     u64 lds_bytes = 0;
     void *w = nullptr;       // packed weights (device, owned by the plan)
-    void *halo = nullptr;    // last tiles' neighbour columns, [owners][C][K-1] (device, owned by the plan)
+    void *halo = nullptr;    // the columns after the owners' chunks, [owners][C][K-1] (device, owned by the plan)
 };
+
+// The chunk of an owner: tiles [first, end) of the flattened (batch element,
+// tile) sequence.  Where it ends inside a row, b is that batch element and j
+// the first column after the chunk, which the next owner overwrites; else
+// b = -1.
+struct ConvChunk {
+    int first, end, b, j;
+    // whether column cj of batch element cb comes from the copy made before the launch
+    __host__ __device__ __forceinline__ bool copied(int cb, int cj) const { return cb == b && cj >= j; }
+};
+__host__ __device__ __forceinline__ ConvChunk conv_chunk(int owner, int chunk, int total, int tiles, int TN) {
+    ConvChunk c;
+    c.first = owner * chunk;
+    c.end = c.first + chunk < total ? c.first + chunk : total;
+    const int last = c.end - 1, t = last % tiles;
+    c.b = t < tiles - 1 ? last / tiles : -1;
+    c.j = (t + 1) * TN;
+    return c;
+}
 
 // Chooses the launch, allocates and packs the weights on `s`.
 bkma_status direct_conv_create(bkma_dtype dt, int B, int C, int L, int K, const void *weight, hipStream_t s,

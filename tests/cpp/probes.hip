@@ -1,9 +1,11 @@
 // Operand-layout and conversion probes of the MFMA Conv1d kernels: single
 // MFMAs on lane fragments and the kernels' FP32 -> FP8 e4m3 conversion
-// (parallel-advection_amd/csrc/mfma_ops.hpp).  TEST INFRASTRUCTURE: built into
-// tests/cpp/libbkma_probes.so, called by tests/test_conv_gpu.py.
+// (parallel-advection_amd/csrc/mfma_ops.hpp), and host probes of launch
+// geometry.  TEST INFRASTRUCTURE: built into tests/cpp/libbkma_probes.so, called
+// by tests/test_conv_gpu.py and others.
 #include <algorithm>
 
+#include "conv_direct.hpp"
 #include "mfma_ops.hpp"
 
 using namespace bkma;
@@ -125,5 +127,26 @@ int probe_fp8_convert(const void *in, void *out, unsigned long long n, void *str
     hipLaunchKernelGGL(fp8_convert_kernel, dim3(g ? g : 1), dim3(256), 0, (hipStream_t)stream, (const float *)in,
                        (unsigned char *)out, np);
     return done("fp8_convert_kernel");
+}
+// Host only.  The chunks of a direct convolution of B batch elements, `tiles`
+// tiles of TN columns each, kernels of K taps, `chunk` tiles per owner: how many
+// columns of all tiles' windows are read from the array although another owner
+// writes them, or from a copy past its end.
+long long probe_conv_chunk_faults(int B, int tiles, int TN, int K, int chunk) {
+    long long bad = 0;
+    const int total = B * tiles, owners = (total + chunk - 1) / chunk;
+    for (int o = 0; o < owners; ++o) {
+        const ConvChunk ck = conv_chunk(o, chunk, total, tiles, TN);
+        if (ck.first != o * chunk || ck.end != std::min(total, (o + 1) * chunk)) return -1;
+        for (int tile = ck.first; tile < ck.end; ++tile) {
+            const int b = tile / tiles, j0 = (tile - b * tiles) * TN;
+            for (int j = j0; j < j0 + TN + K - 1; ++j) {
+                if (j >= tiles * TN) break;  // columns that nobody writes
+                if (ck.copied(b, j)) bad += j - ck.j >= K - 1;
+                else bad += b * tiles + j / TN >= ck.end || b * tiles + j / TN < tile;
+            }
+        }
+    }
+    return bad;
 }
 }

@@ -1,0 +1,63 @@
+"""Direct convolutions (FP64 and FP32 Conv1d modes) whose kernels reach past the next tile, K - 1 > TN: the columns
+after an owner's chunk belong to another owner, so every tile that reaches them takes them from the copy made before
+the launch."""
+import ctypes
+import os
+
+import numpy as np
+import pytest
+
+import bkma_amd as B
+import oracle as O
+
+PROBES = os.path.join(os.path.dirname(os.path.abspath(__file__)), "cpp", "libbkma_probes.so")
+
+
+@pytest.mark.parametrize("tn", [32, 64, 128, 256])
+@pytest.mark.parametrize("chunk", [1, 2, 3, 7, 64])
+def test_windows_read_no_column_of_another_owner(tn, chunk):
+    """On the host: no window reads a live column that another owner writes, nor past the copied columns."""
+    B.lib()  # first: the probes share its HIP runtime
+    P = ctypes.CDLL(PROBES)
+    P.probe_conv_chunk_faults.restype = ctypes.c_longlong
+    for tiles in (1, 2, 3, 8, 9):
+        for k in (1, 2, tn, tn + 1, tn + 2, 2 * tn + 1, 2 * tn + 2, 5 * tn):
+            assert P.probe_conv_chunk_faults(5, tiles, tn, k, chunk) == 0, (tiles, k)
+
+
+# (B, C, L, K): several tiles per row and several tiles per owner, K - 1 > TN.
+VALU = [(600, 4, 1200, 300), (3000, 2, 1100, 290)]
+MATRIX = [(600, 13, 600, 140)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mode,shape", [(B.CONV_F64, s) for s in VALU] + [(B.CONV_F32, s) for s in VALU + MATRIX],
+                         ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else "f64" if v == B.CONV_F64 else "f32")
+def test_kernels_longer_than_a_tile(cuda, mode, shape):
+    """FP64 bit for bit, FP32 within the bound of a sum of n = C K products, (n + 2) 2^-24 (sum |w||x| + |bias|);
+    three runs, since a column read too late shows only now and then."""
+    import torch
+    Bn, C, L, K = shape
+    f32 = mode == B.CONV_F32
+    npdt, code = (np.float32, B.F32) if f32 else (np.float64, B.F64)
+    rng = np.random.default_rng(K)
+    w = (rng.standard_normal((C, C, K)) / np.sqrt(C * K)).astype(npdt)
+    b = (0.1 * rng.standard_normal(C)).astype(npdt)
+    x = rng.standard_normal((Bn, C, L)).astype(npdt)
+    ref = x.astype(np.float64)
+    O.conv_torch_f64(ref, w.astype(np.float64), b.astype(np.float64))
+    plan = B.Conv1dPlan(mode, code, Bn, C, L, K, torch.from_numpy(w).cuda(), torch.from_numpy(b).cuda())
+    n = L - K + 1
+    if f32:
+        bound = np.abs(x).astype(np.float64)
+        O.conv_torch_f64(bound, np.abs(w).astype(np.float64), np.abs(b).astype(np.float64))
+        bound *= (C * K + 2) * 2.0 ** -24
+    for _ in range(3):
+        tx = torch.from_numpy(x).cuda()
+        plan.run(tx)
+        got = tx.cpu().numpy()
+        assert np.array_equal(got[:, :, n:], x[:, :, n:])
+        if f32:
+            assert np.all(np.abs(got[:, :, :n].astype(np.float64) - ref[:, :, :n]) <= bound[:, :, :n])
+        else:
+            assert np.array_equal(got, ref)
