@@ -157,8 +157,8 @@ __global__ __launch_bounds__(256) void conv_valu_kernel(T *__restrict__ x, const
     const int Lout = L - K + 1;
     const ConvChunk ck = conv_chunk(owner, chunk, total, tiles, TN);
     for (int it = 0; it < chunk; ++it) {  // the same count for all waves: the barriers are uniform
-        const int tile = ck.first + it;
-        const bool on = tile < ck.end;
+        const bool on = it < ck.end - ck.first;
+        const int tile = on ? ck.first + it : 0;
         const int b = tile / tiles, t = tile - b * tiles;
         const int j0 = t * TN;
         T *xb = x + (i64)b * C * L;

@@ -33,9 +33,11 @@ struct ConvChunk {
     __host__ __device__ __forceinline__ bool copied(int cb, int cj) const { return cb == b && cj >= j; }
 };
 __host__ __device__ __forceinline__ ConvChunk conv_chunk(int owner, int chunk, int total, int tiles, int TN) {
+    // in 64 bits: total goes up to 2^31 - 1, and an owner past the last one has no tiles
+    const i64 first = (i64)owner * chunk, end = first + chunk;
     ConvChunk c;
-    c.first = owner * chunk;
-    c.end = c.first + chunk < total ? c.first + chunk : total;
+    c.first = first < total ? (int)first : total;
+    c.end = end < total ? (int)end : total;
     const int last = c.end - 1, t = last % tiles;
     c.b = t < tiles - 1 ? last / tiles : -1;
     c.j = (t + 1) * TN;

@@ -128,6 +128,12 @@ int probe_fp8_convert(const void *in, void *out, unsigned long long n, void *str
                        (unsigned char *)out, np);
     return done("fp8_convert_kernel");
 }
+// Host only: the tiles [first, end) of a direct convolution's owner.
+void probe_conv_chunk(int owner, int chunk, int total, int *first, int *end) {
+    const ConvChunk ck = conv_chunk(owner, chunk, total, total, 64);
+    *first = ck.first;
+    *end = ck.end;
+}
 // Host only.  The chunks of a direct convolution of B batch elements, `tiles`
 // tiles of TN columns each, kernels of K taps, `chunk` tiles per owner: how many
 // columns of all tiles' windows are read from the array although another owner

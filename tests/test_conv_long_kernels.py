@@ -1,6 +1,6 @@
-"""Direct convolutions (FP64 and FP32 Conv1d modes) whose kernels reach past the next tile, K - 1 > TN: the columns
-after an owner's chunk belong to another owner, so every tile that reaches them takes them from the copy made before
-the launch."""
+"""The owners of the direct convolutions (FP64 and FP32 Conv1d modes): kernels that reach past the next tile,
+K - 1 > TN, take the columns after an owner's chunk, which belong to another owner, from the copy made before the
+launch; chunk bounds for tile counts up to 2^31 - 1."""
 import ctypes
 import os
 
@@ -23,6 +23,34 @@ def test_windows_read_no_column_of_another_owner(tn, chunk):
     for tiles in (1, 2, 3, 8, 9):
         for k in (1, 2, tn, tn + 1, tn + 2, 2 * tn + 1, 2 * tn + 2, 5 * tn):
             assert P.probe_conv_chunk_faults(5, tiles, tn, k, chunk) == 0, (tiles, k)
+
+
+@pytest.mark.parametrize("chunk", [1, 262144, 262145, 2 ** 30, 2 ** 31 - 1])
+def test_chunks_of_the_largest_tile_count(chunk):
+    """On the host: chunk bounds stay within 2^31 - 1 tiles, also those of the owners past the last one."""
+    B.lib()
+    P = ctypes.CDLL(PROBES)
+    P.probe_conv_chunk.restype = None
+    total, f, e = 2 ** 31 - 1, ctypes.c_int(), ctypes.c_int()
+    last = -(-total // chunk) - 1
+    for owner in (0, last // 2, last, last + 1, last + 7):
+        P.probe_conv_chunk(min(owner, 2 ** 31 - 1), chunk, total, ctypes.byref(f), ctypes.byref(e))
+        assert f.value == min(owner * chunk, total) and e.value == min((owner + 1) * chunk, total)
+
+
+@pytest.mark.gpu
+def test_largest_batch(cuda):
+    """2^31 - 1 batch elements of one cell: every one is written."""
+    import torch
+    n = 2 ** 31 - 1
+    if torch.cuda.mem_get_info()[0] < 40 << 30:
+        pytest.skip("needs 40 GB of device memory")
+    x = torch.ones((n, 1, 1), dtype=torch.float32, device="cuda")
+    one = torch.ones(1, dtype=torch.float32, device="cuda")
+    B.Conv1dPlan(B.CONV_F32, B.F32, n, 1, 1, 1, 2 * one.view(1, 1, 1), 0.5 * one).run(x)
+    assert x.min().item() == 2.5 and x.max().item() == 2.5
+    del x
+    torch.cuda.empty_cache()
 
 
 # (B, C, L, K): several tiles per row and several tiles per owner, K - 1 > TN.
