@@ -67,15 +67,19 @@ __global__ __launch_bounds__(64 * kStepWaves) void adv_step_column_kernel(double
 namespace {
 
 // Shapes of the register form: whole 128-column (64 below 128) tiles, shifts
-// within [-3, 3], and wavefronts enough to fill the GPU.  Time of the tiles
+// within [-3, 3] up to the rounding of the feet (tile_shifts; the kernel has no
+// body for any other), and wavefronts enough to fill the GPU.  Time of the tiles
 // over it, one FP64 step of [n0][1000][n2]: n2 = 64: 512 slabs 0.78, 1024
 // 1.23; n2 = 128: 256 slabs 0.70, 512 1.23; [n0][3000][64]: 256 slabs 1.1.
-bool column_form(const AdvDev &p, const void *data, double smin, double smax) {
+bool column_form(const AdvDev &p, const void *data) {
     const i64 width = p.n2 >= 128 ? 128 : 64;
     if (p.n2 % width != 0 || p.n1 < 64 || p.n1 > (1 << 20)) return false;
     if (width == 128 && reinterpret_cast<uintptr_t>(data) % 16 != 0) return false;
     if (p.n0 * (p.n2 / 64) < (p.n1 > 2500 ? 256 : 1024) || p.n0 * (p.n2 / width) > 0x7fffffffLL) return false;
-    return std::ceil(smin - 1e-6) >= -3.0 && std::ceil(smax + 1e-6) <= 3.0;
+    double lo0, hi0, lo1, hi1;
+    tile_shifts(p, 0, lo0, hi0);
+    tile_shifts(p, p.n0 - 1, lo1, hi1);
+    return std::min(lo0, lo1) >= -3.0 && std::max(hi0, hi1) <= 3.0;
 }
 
 template <int VEC> bkma_status launch_column(const AdvDev &p, double *data, hipStream_t s) {
@@ -126,7 +130,7 @@ bkma_status adv_step_whole(const AdvDev &p, bkma_dtype dt, void *data, hipStream
     if (p.n1 < 16 || !(std::isfinite(s0) && std::isfinite(s1) && std::isfinite(p.minRealX) && p.realWidthX > 0 &&
                        std::isfinite(p.realWidthX) && std::max(-smin, smax) + 4 < (double)p.n1 / 2))
         return BKMA_OK;
-    if (dt == BKMA_F64 && column_form(p, data, smin, smax)) {
+    if (dt == BKMA_F64 && column_form(p, data)) {
         *done = true;
         return p.n2 >= 128 ? launch_column<2>(p, (double *)data, s) : launch_column<1>(p, (double *)data, s);
     }
