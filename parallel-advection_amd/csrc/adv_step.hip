@@ -13,7 +13,6 @@
 //    pass, one foot per row and four columns: 0.60 ms on that shape.
 #include <algorithm>
 #include <climits>
-#include <cmath>
 
 #include "adv_pair.hpp"
 #include "adv_step.hpp"
@@ -123,13 +122,7 @@ const StepShape &step_shape(const AdvDev &p, u64 esz, u64 lds_max) {
 
 bkma_status adv_step_whole(const AdvDev &p, bkma_dtype dt, void *data, hipStream_t s, bool *done) {
     *done = false;
-    // as the plans: finite parameters, shifts below half a line
-    const double s0 = p.minRealVx * p.dt * p.inv_dx;
-    const double s1 = (p.minRealVx + (double)(p.n0 - 1) * p.dvx) * p.dt * p.inv_dx;
-    const double smin = std::min(s0, s1), smax = std::max(s0, s1);
-    if (p.n1 < 16 || !(std::isfinite(s0) && std::isfinite(s1) && std::isfinite(p.minRealX) && p.realWidthX > 0 &&
-                       std::isfinite(p.realWidthX) && std::max(-smin, smax) + 4 < (double)p.n1 / 2))
-        return BKMA_OK;
+    if (p.n1 < 16 || !tile_covers(p)) return BKMA_OK;
     if (dt == BKMA_F64 && column_form(p, data)) {
         *done = true;
         return p.n2 >= 128 ? launch_column<2>(p, (double *)data, s) : launch_column<1>(p, (double *)data, s);

@@ -43,7 +43,10 @@
 // step each.
 #pragma once
 
+#include <algorithm>
 #include <atomic>
+#include <climits>
+#include <cmath>
 #include <vector>
 
 #include "common.hpp"
@@ -84,6 +87,20 @@ __host__ __device__ __forceinline__ void tile_shifts(const AdvDev &p, i64 i0, do
     const double e = 1e-6 + 1e-15 * (fabs(p.minRealX) + 2.0 * p.realWidthX) * p.inv_dx;
     dlo = ceil(s - e);
     dhi = ceil(s + e);
+}
+
+// Whether tile_shifts holds for every slab of the problem, as all tiles take
+// for granted: a regular periodic grid (the derived fields agree to a small part
+// of the 1e-6 above, added up over a line), coordinates that resolve the cells,
+// so that a slab's rows take at most two adjacent shifts, and shifts below half
+// a line.  The executors' own kernels, and the others, evaluate any foot.
+inline bool tile_covers(const AdvDev &p) {
+    const double n1 = (double)p.n1, v1 = p.minRealVx + (double)(p.n0 - 1) * p.dvx;
+    const double s = std::fabs(p.dt * p.inv_dx) * std::max(std::fabs(p.minRealVx), std::fabs(v1));
+    const double apart = n1 * (std::fabs(p.dx * p.inv_dx - 1.0) + std::fabs(p.dx * n1 / p.realWidthX - 1.0));
+    const double round = 1e-15 * (std::fabs(p.minRealX) + 2.0 * p.realWidthX) * p.inv_dx;
+    return p.realWidthX > 0 && std::isfinite(p.realWidthX) && p.n0 <= INT_MAX && p.n1 <= INT_MAX && apart <= 5e-7 &&
+           round <= 0.25 && s + 4.0 < n1 / 2.0;  // NaN is false
 }
 
 // Halo rows per step of slab i0 before and after a segment (the stencil of
@@ -462,7 +479,7 @@ bool strip_shape(const bkma_adv_params &p, u64 s0, u64 s1, u64 elem_size, int ns
 // A problem's tiles for passes of ns steps (0: chosen here; the same for all
 // parts, in parts[0].a.ns): with `strips`, strips for the slabs whose shifts
 // they cover (first in the list, if there are any) and LDS tiles for the
-// others.  Empty where there are none.
+// others.  Empty where there are none (tile_covers among the reasons).
 std::vector<TileShape> tile_parts(const bkma_adv_params &p, u64 elem_size, int ns, u64 lds_max, bool strips);
 
 // One pass of ns steps (at most the shape's).  `fused`: fused sums (FP32

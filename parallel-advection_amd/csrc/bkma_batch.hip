@@ -367,9 +367,6 @@ static bool build_groups(AdvBatch &b) {
     std::vector<Part> parts;
     for (size_t j = 0; j < n; ++j) {
         const bkma_adv_params &p = b.problems[j].params;
-        if (!std::isfinite(p.minRealVx) || !std::isfinite(p.dvx) || !std::isfinite(p.inv_dx) ||
-            !std::isfinite(p.minRealX) || !std::isfinite(p.realWidthX))
-            return false;
         const std::vector<TileShape> ts = tile_parts(p, esz, 0, lds_max, true);
         if (ts.empty()) return false;
         for (const TileShape &t : ts) parts.push_back(Part{j, t});

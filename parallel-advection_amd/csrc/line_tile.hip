@@ -372,7 +372,7 @@ bool strip_shape(const bkma_adv_params &p, u64 s0, u64 s1, u64 elem_size, int ns
 std::vector<TileShape> tile_parts(const bkma_adv_params &p, u64 elem_size, int ns, u64 lds_max, bool strips) {
     std::vector<TileShape> parts;
     TileShape all;
-    if (!tile_shape(p, 0, p.n0, elem_size, ns, lds_max, &all)) return parts;
+    if (!tile_covers(make_adv_dev(p)) || !tile_shape(p, 0, p.n0, elem_size, ns, lds_max, &all)) return parts;
     // Slabs [lo, hi) whose shifts the strips cover (monotone in the slab).
     const AdvDev d = make_adv_dev(p);
     auto covered = [&](u64 i0) {
