@@ -52,13 +52,12 @@ __device__ __forceinline__ void strip_step(const double (&f)[E], double (&g)[E],
         w[t] = strip_shift<hop>(f[o - hop * E]);
     });
     if constexpr (MIXED) {
-        // c[e][0] is the first tap of an early row and the last of a late one;
-        // -0.0 + x is x for every x
+        // c[e][0] is the first tap of an early row and the last of a late one
 #pragma unroll
         for (int e = 0; e < E; ++e) {
             const bool late = (up >> e) & 1;
-            const double first = c[e][0] * w[e];
-            double acc = late ? -0.0 : first;
+            const double first = fma(c[e][0], w[e], 0.0);  // as tile_taps
+            double acc = late ? 0.0 : first;
 #pragma unroll
             for (int k = 1; k < 6; ++k) acc = FUSED ? fma(c[e][k], w[e + k], acc) : acc + c[e][k] * w[e + k];
             const double last = FUSED ? fma(c[e][0], w[e + 6], acc) : acc + c[e][0] * w[e + 6];
@@ -75,7 +74,7 @@ __device__ __forceinline__ void strip_step(const double (&f)[E], double (&g)[E],
 #pragma unroll
                 for (int e = 0; e < G; ++e) {
                     const double x = w[e0 + e + k];
-                    if (k == 0) g[e0 + e] = c[e0 + e][0] * x;
+                    if (k == 0) g[e0 + e] = fma(c[e0 + e][0], x, 0.0);
                     else if constexpr (FUSED) g[e0 + e] = fma(c[e0 + e][k], x, g[e0 + e]);
                     else t[e] = c[e0 + e][k] * x;
                 }

@@ -283,9 +283,10 @@ __device__ __forceinline__ void tile_store(T *base, const double *__restrict__ s
     else tile_store_w<T, U, 1, WRAP>(base, src, a, nout, cbw, hbn, r0);
 }
 
-// Six-tap sum over w[0..5].
+// Six-tap sum over w[0..5], from 0. on as the reference's: 0. + -0. is 0., so
+// the first product is fused with 0. (at no cost).
 template <bool FUSED> __device__ __forceinline__ double tile_taps(const double (&c)[6], const double *w) {
-    double acc = c[0] * w[0];
+    double acc = fma(c[0], w[0], 0.0);
 #pragma unroll
     for (int k = 1; k < 6; ++k) {
         if constexpr (FUSED)
