@@ -483,6 +483,15 @@ bool strip_shape(const bkma_adv_params &p, u64 s0, u64 s1, u64 elem_size, int ns
 // others.  Empty where there are none (tile_covers among the reasons).
 std::vector<TileShape> tile_parts(const bkma_adv_params &p, u64 elem_size, int ns, u64 lds_max, bool strips);
 
+// Work-groups of `threads` threads that one launch may have (HIP counts threads
+// in 32 bits; the snapshots' work-groups have up to 256).
+inline i64 tile_launch_units(int threads) { return 0xffffffffLL / std::max(threads, 256); }
+// Slabs of a shape, cut into nseg segments each, that one launch may cover.
+inline i64 tile_slabs_per_launch(const TileShape &sh, int nseg) {
+    const i64 units = tile_launch_units(sh.threads) / sh.a.nct;
+    return std::max<i64>(1, sh.wrap ? units * sh.a.sb : units / nseg);
+}
+
 // One pass of ns steps (at most the shape's).  `fused`: fused sums (FP32
 // storage), `rnd`: rounded to FP32 after every step.  `from`: the array to read
 // (of the same extents; no snapshot), else `data` in place.

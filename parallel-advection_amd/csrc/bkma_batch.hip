@@ -369,7 +369,10 @@ static bool build_groups(AdvBatch &b) {
         const bkma_adv_params &p = b.problems[j].params;
         const std::vector<TileShape> ts = tile_parts(p, esz, 0, lds_max, true);
         if (ts.empty()) return false;
-        for (const TileShape &t : ts) parts.push_back(Part{j, t});
+        for (const TileShape &t : ts) {
+            if (t.a.units > tile_launch_units(t.threads)) return false;  // a group's part is in one launch
+            parts.push_back(Part{j, t});
+        }
     }
     for (void *h : b.halos) (void)hipFree(h);
     b.halos.clear();
@@ -399,7 +402,7 @@ static bool build_groups(AdvBatch &b) {
         for (size_t j = f; j < parts.size(); ++j) {
             if (taken[j] || !ok || !same(parts[f].t, parts[j].t)) continue;
             const TileShape &t = parts[j].t;
-            if ((u64)(g.units + t.a.units) > 0x7fffffffULL) continue;  // a group of its own
+            if (!tab.empty() && g.units + t.a.units > tile_launch_units(threads(t))) continue;  // a group of its own
             taken[j] = true;
             TileProblem pr{};
             pr.a = t.a;

@@ -155,7 +155,7 @@ bool set_segments(TileShape &sh, int ns, int hmax, u64 elem_size) {
     a.hrows = ns * hmax;
     a.nseg = (int)ceil_div((u64)a.p.n1, (u64)(a.rows - a.hrows));
     a.units = (a.s1 - a.s0) * a.nseg * a.nct;
-    if ((u64)(a.s1 - a.s0) * a.nseg * a.nct > 0x7fffffffULL) return false;
+    if ((u64)a.units > 0x7fffffffULL || (i64)a.nseg * a.nct > tile_launch_units(sh.threads)) return false;
     sh.halo_bytes = (u64)(a.s1 - a.s0) * (u64)a.nseg * (u64)a.hrows * (u64)a.p.n2 * elem_size;
     return true;
 }
@@ -422,21 +422,11 @@ std::vector<TileShape> tile_parts(const bkma_adv_params &p, u64 elem_size, int n
     return parts;
 }
 
-bkma_status launch_tile(const TileShape &sh, bkma_dtype dt, bool fused, bool rnd, void *data, void *halo, int ns,
-                        hipStream_t s, void *from) {
-    if (ns < 1 || ns > sh.a.ns) return fail(BKMA_ERR_RUNTIME, "LINE_LDS tiles: steps per pass out of range");
-    TileArgs a = sh.a;
-    a.ns = ns;
-    if ((uintptr_t)data % 16 != 0) a.wide = 0;
-    if (from) {
-        a.apart = 1;
-        halo = from;
-    }
-    if (!sh.wrap) {  // fewer steps: smaller halos, longer segments (the snapshot keeps its row stride)
-        const int h = a.hrows / sh.a.ns;
-        a.nseg = (int)ceil_div((u64)a.p.n1, (u64)(a.rows - ns * h));
-        a.units = (a.s1 - a.s0) * a.nseg * a.nct;
-    }
+namespace {
+
+// One pass over the slabs [a.s0, a.s1).
+bkma_status launch_slabs(const TileShape &sh, const TileArgs &a, bkma_dtype dt, bool fused, bool rnd, void *data,
+                         void *halo, hipStream_t s, void *from) {
     if (!sh.wrap && !from) {
         const unsigned groups = (unsigned)((a.s1 - a.s0) * a.nseg);
         const unsigned nt = (i64)a.hrows * a.p.n2 >= 512 ? 256 : 64;
@@ -456,6 +446,34 @@ bkma_status launch_tile(const TileShape &sh, bkma_dtype dt, bool fused, bool rnd
     if (rnd) return launch_v<float, true, true>(sh, a, data, halo, s);
     if (fused) return launch_v<float, true, false>(sh, a, data, halo, s);
     return launch_v<float, false, false>(sh, a, data, halo, s);
+}
+
+}  // namespace
+
+bkma_status launch_tile(const TileShape &sh, bkma_dtype dt, bool fused, bool rnd, void *data, void *halo, int ns,
+                        hipStream_t s, void *from) {
+    if (ns < 1 || ns > sh.a.ns) return fail(BKMA_ERR_RUNTIME, "LINE_LDS tiles: steps per pass out of range");
+    TileArgs a = sh.a;
+    a.ns = ns;
+    if ((uintptr_t)data % 16 != 0) a.wide = 0;
+    if (from) {
+        a.apart = 1;
+        halo = from;
+    }
+    if (!sh.wrap) {  // fewer steps: smaller halos, longer segments (the snapshot keeps its row stride)
+        const int h = a.hrows / sh.a.ns;
+        a.nseg = (int)ceil_div((u64)a.p.n1, (u64)(a.rows - ns * h));
+    }
+    // HIP launches have fewer than 2^32 threads: slabs in several launches where
+    // they need more ([2^24][1000][1]: one work-group of 256 per slab)
+    const i64 per = tile_slabs_per_launch(sh, a.nseg);
+    for (i64 s0 = sh.a.s0; s0 < sh.a.s1; s0 += per) {
+        a.s0 = s0;
+        a.s1 = std::min(s0 + per, sh.a.s1);
+        a.units = sh.wrap ? (i64)ceil_div((u64)(a.s1 - a.s0), (u64)a.sb) * a.nct : (a.s1 - a.s0) * a.nseg * a.nct;
+        BKMA_TRY(launch_slabs(sh, a, dt, fused, rnd, data, halo, s, from));
+    }
+    return BKMA_OK;
 }
 
 bkma_status launch_tile_group(const TileGroup &g, bkma_dtype dt, bool rnd, int ns, hipStream_t s) {
