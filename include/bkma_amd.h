@@ -351,6 +351,12 @@ typedef struct bkma_conv1d_plan bkma_conv1d_plan;
 bkma_status bkma_conv1d_plan_create(bkma_conv_mode mode, bkma_dtype io_dtype, uint64_t B, uint64_t C, uint64_t L,
                                     uint64_t K, bkma_dtype w_dtype, const void *weight, const void *bias,
                                     void *stream, bkma_conv1d_plan **out);
+/* F64 and F32 modes: runs of one plan on different arrays may overlap on
+ * several streams, in several graphs and from several threads.  The plan keeps
+ * a small buffer (some columns of x) for each of up to 8 streams and 8 graph
+ * captures, allocated at a stream's first run (the first stream's at creation);
+ * runs beyond them need none and split the work less finely.  The other modes
+ * share one buffer: runs of one plan must not overlap. */
 bkma_status bkma_conv1d_plan_run(bkma_conv1d_plan *plan, void *x, void *stream);
 bkma_status bkma_conv1d_plan_describe(const bkma_conv1d_plan *plan, char *name, uint64_t name_len);
 /* FP8 mode: the input is quantized as x / scale (scale > 0; default 1). */

@@ -36,6 +36,7 @@
 //   (112 TFLOP/s, the matrix cores 65-75% busy: a tile is staged while only
 //   the CU's other work-group computes).
 #include <algorithm>
+#include <new>
 
 #include "conv_direct.hpp"
 
@@ -454,8 +455,8 @@ const void *kernel_of(const DirectConv &d) {
 
 void direct_conv_free(DirectConv &d) {
     if (d.w) (void)hipFree(d.w);
-    if (d.halo) (void)hipFree(d.halo);
-    d.w = d.halo = nullptr;
+    d.w = nullptr;
+    d.halo.reset();
 }
 
 bkma_status direct_conv_create(bkma_dtype dt, int B, int C, int L, int K, const void *weight, hipStream_t s,
@@ -576,7 +577,7 @@ bkma_status direct_conv_create(bkma_dtype dt, int B, int C, int L, int K, const 
     if (tiles * (u64)B > 0x7fffffffULL) return fail(BKMA_ERR_UNSUPPORTED, "conv1d plan: sizes beyond 32-bit indexing");
     d.tiles = (int)tiles;
     d.total = (int)(tiles * B);
-    const int slots = d.mfma || d.lane ? 1 : 4 / d.wpt;
+    d.slots = d.mfma || d.lane ? 1 : 4 / d.wpt;
     int dev = 0, cus = 0, blocks = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
@@ -585,12 +586,16 @@ bkma_status direct_conv_create(bkma_dtype dt, int B, int C, int L, int K, const 
     if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_max) != hipSuccess ||
         hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, k, 256, (size_t)d.lds_bytes) != hipSuccess)
         return fail(BKMA_ERR_DEVICE, "conv1d plan: occupancy query");
-    const u64 resident = (u64)std::max(1, blocks) * (u64)cus * (u64)slots;
+    const u64 resident = (u64)std::max(1, blocks) * (u64)cus * (u64)d.slots;
     d.chunk = (int)ceil_div((u64)d.total, std::min<u64>((u64)d.total, resident));
     d.owners = (int)ceil_div((u64)d.total, (u64)d.chunk);
-    d.grid = (unsigned)ceil_div((u64)d.owners, (u64)slots);
-    if (hipMalloc(&d.w, wcount * esz) != hipSuccess ||
-        (d.tiles > 1 && K > 1 && hipMalloc(&d.halo, (u64)d.owners * C * (K - 1) * esz) != hipSuccess)) {
+    d.grid = (unsigned)ceil_div((u64)d.owners, (u64)d.slots);
+    bool room = hipMalloc(&d.w, wcount * esz) == hipSuccess;
+    if (room && d.tiles > 1 && K > 1) {
+        d.halo.reset(new (std::nothrow) StreamScratch());
+        room = d.halo && d.halo->create((u64)d.owners * C * (K - 1) * esz);
+    }
+    if (!room) {
         direct_conv_free(d);
         return fail(BKMA_ERR_OUT_OF_MEMORY, "conv1d plan: weight copy");
     }
@@ -609,7 +614,7 @@ bkma_status direct_conv_create(bkma_dtype dt, int B, int C, int L, int K, const 
         direct_conv_free(d);
         return fail(BKMA_ERR_DEVICE, "conv1d plan: weight packing");
     }
-    *out = d;
+    *out = std::move(d);
     return BKMA_OK;
 }
 
@@ -626,81 +631,104 @@ bool row_vec(const DirectConv &d, const void *x) {
     return reinterpret_cast<uintptr_t>(x) % 16 == 0 && ((u64)d.L * (d.dt == BKMA_F64 ? 8 : 4)) % 16 == 0;
 }
 
-template <class T, int OCB, int JT> void launch_valu(const DirectConv &d, T *x, const T *bias, hipStream_t s) {
-    hipLaunchKernelGGL((conv_valu_kernel<T, OCB, JT>), dim3(d.grid), dim3(256), (size_t)d.lds_bytes, s, x,
-                       (const T *)d.halo, (const T *)d.w, bias, d.C, d.L, d.K, d.tiles, d.total, d.chunk, d.wpt,
+// One run's share of the tiles.
+struct ConvRun {
+    int chunk = 0;
+    unsigned grid = 0;
+    void *halo = nullptr;
+};
+
+template <class T, int OCB, int JT>
+void launch_valu(const DirectConv &d, const ConvRun &r, T *x, const T *bias, hipStream_t s) {
+    hipLaunchKernelGGL((conv_valu_kernel<T, OCB, JT>), dim3(r.grid), dim3(256), (size_t)d.lds_bytes, s, x,
+                       (const T *)r.halo, (const T *)d.w, bias, d.C, d.L, d.K, d.tiles, d.total, r.chunk, d.wpt,
                        d.groups, d.pitch, row_vec(d, x));
 }
 
-template <class T, int OCB> void launch_valu_jt(const DirectConv &d, T *x, const T *bias, hipStream_t s) {
-    if (d.jt == 4) launch_valu<T, OCB, 4>(d, x, bias, s);
-    else if (d.jt == 2) launch_valu<T, OCB, 2>(d, x, bias, s);
-    else launch_valu<T, OCB, 1>(d, x, bias, s);
+template <class T, int OCB>
+void launch_valu_jt(const DirectConv &d, const ConvRun &r, T *x, const T *bias, hipStream_t s) {
+    if (d.jt == 4) launch_valu<T, OCB, 4>(d, r, x, bias, s);
+    else if (d.jt == 2) launch_valu<T, OCB, 2>(d, r, x, bias, s);
+    else launch_valu<T, OCB, 1>(d, r, x, bias, s);
 }
 
-template <class T> void launch_valu_of(const DirectConv &d, T *x, const T *bias, hipStream_t s) {
+template <class T>
+void launch_valu_of(const DirectConv &d, const ConvRun &r, T *x, const T *bias, hipStream_t s) {
     switch (d.ocb) {
-        case 8: launch_valu_jt<T, 8>(d, x, bias, s); break;
-        case 6: launch_valu_jt<T, 6>(d, x, bias, s); break;
-        case 5: launch_valu_jt<T, 5>(d, x, bias, s); break;
-        case 4: launch_valu_jt<T, 4>(d, x, bias, s); break;
-        case 3: launch_valu_jt<T, 3>(d, x, bias, s); break;
-        case 2: launch_valu_jt<T, 2>(d, x, bias, s); break;
-        default: launch_valu_jt<T, 1>(d, x, bias, s); break;
+        case 8: launch_valu_jt<T, 8>(d, r, x, bias, s); break;
+        case 6: launch_valu_jt<T, 6>(d, r, x, bias, s); break;
+        case 5: launch_valu_jt<T, 5>(d, r, x, bias, s); break;
+        case 4: launch_valu_jt<T, 4>(d, r, x, bias, s); break;
+        case 3: launch_valu_jt<T, 3>(d, r, x, bias, s); break;
+        case 2: launch_valu_jt<T, 2>(d, r, x, bias, s); break;
+        default: launch_valu_jt<T, 1>(d, r, x, bias, s); break;
     }
 }
 
-template <int MB, int NB> void launch_mfma(const DirectConv &d, float *x, const float *bias, hipStream_t s) {
-    hipLaunchKernelGGL((conv_mfma32_kernel<MB, NB>), dim3(d.grid), dim3(256), (size_t)d.lds_bytes, s, x,
-                       (const float *)d.halo, (const float *)d.w, bias, d.C, d.L, d.K, d.tiles, d.total, d.chunk,
+template <int MB, int NB>
+void launch_mfma(const DirectConv &d, const ConvRun &r, float *x, const float *bias, hipStream_t s) {
+    hipLaunchKernelGGL((conv_mfma32_kernel<MB, NB>), dim3(r.grid), dim3(256), (size_t)d.lds_bytes, s, x,
+                       (const float *)r.halo, (const float *)d.w, bias, d.C, d.L, d.K, d.tiles, d.total, r.chunk,
                        d.groups, d.parts, log2_of(d.TN), d.pitch, row_vec(d, x));
 }
 
-template <int MB> void launch_mfma_nb(const DirectConv &d, float *x, const float *bias, hipStream_t s) {
-    if (d.jt == 8) launch_mfma<MB, 8>(d, x, bias, s);
-    else if (d.jt == 4) launch_mfma<MB, 4>(d, x, bias, s);
-    else launch_mfma<MB, 2>(d, x, bias, s);
+template <int MB>
+void launch_mfma_nb(const DirectConv &d, const ConvRun &r, float *x, const float *bias, hipStream_t s) {
+    if (d.jt == 8) launch_mfma<MB, 8>(d, r, x, bias, s);
+    else if (d.jt == 4) launch_mfma<MB, 4>(d, r, x, bias, s);
+    else launch_mfma<MB, 2>(d, r, x, bias, s);
 }
 
-template <int KT> void launch_lane_k(const DirectConv &d, double *x, const double *bias, hipStream_t s) {
-    hipLaunchKernelGGL(conv_lane64_kernel<KT>, dim3(d.grid), dim3(256), (size_t)d.lds_bytes, s, x,
-                       (const double *)d.halo, (const double *)d.w, bias, d.C, d.L, d.tiles, d.total, d.chunk,
+template <int KT>
+void launch_lane_k(const DirectConv &d, const ConvRun &r, double *x, const double *bias, hipStream_t s) {
+    hipLaunchKernelGGL(conv_lane64_kernel<KT>, dim3(r.grid), dim3(256), (size_t)d.lds_bytes, s, x,
+                       (const double *)r.halo, (const double *)d.w, bias, d.C, d.L, d.tiles, d.total, r.chunk,
                        d.groups, d.ocb, log2_of(d.TN), d.pitch, row_vec(d, x));
 }
 
-bkma_status launch_lane(const DirectConv &d, double *x, const double *bias, hipStream_t s) {
+bkma_status launch_lane(const DirectConv &d, const ConvRun &r, double *x, const double *bias, hipStream_t s) {
     switch (d.K) {
-        case 1: launch_lane_k<1>(d, x, bias, s); break;
-        case 2: launch_lane_k<2>(d, x, bias, s); break;
-        case 3: launch_lane_k<3>(d, x, bias, s); break;
-        case 4: launch_lane_k<4>(d, x, bias, s); break;
-        case 5: launch_lane_k<5>(d, x, bias, s); break;
-        case 7: launch_lane_k<7>(d, x, bias, s); break;
-        case 9: launch_lane_k<9>(d, x, bias, s); break;
-        case 11: launch_lane_k<11>(d, x, bias, s); break;
+        case 1: launch_lane_k<1>(d, r, x, bias, s); break;
+        case 2: launch_lane_k<2>(d, r, x, bias, s); break;
+        case 3: launch_lane_k<3>(d, r, x, bias, s); break;
+        case 4: launch_lane_k<4>(d, r, x, bias, s); break;
+        case 5: launch_lane_k<5>(d, r, x, bias, s); break;
+        case 7: launch_lane_k<7>(d, r, x, bias, s); break;
+        case 9: launch_lane_k<9>(d, r, x, bias, s); break;
+        case 11: launch_lane_k<11>(d, r, x, bias, s); break;
         default: return fail(BKMA_ERR_RUNTIME, "conv1d run: no lane kernel for this K");
     }
     return check_launch("conv_lane64_kernel");
 }
 
 template <class T> bkma_status run_direct(const DirectConv &d, T *x, const T *bias, hipStream_t s) {
+    ConvRun r{d.chunk, d.grid, nullptr};
+    std::unique_lock<std::mutex> held;
     if (d.halo) {
-        hipLaunchKernelGGL(conv_owner_halo_kernel<T>, dim3((unsigned)d.owners), dim3(256), 0, s, (const T *)x,
-                           (T *)d.halo, d.C, d.L, d.K, d.TN, d.tiles, d.total, d.chunk);
-        BKMA_TRY(check_launch("conv_owner_halo_kernel"));
+        held = d.halo->lock();
+        r.halo = d.halo->get(s, false);
+        if (r.halo) {
+            hipLaunchKernelGGL(conv_owner_halo_kernel<T>, dim3((unsigned)d.owners), dim3(256), 0, s, (const T *)x,
+                               (T *)r.halo, d.C, d.L, d.K, d.TN, d.tiles, d.total, d.chunk);
+            BKMA_TRY(check_launch("conv_owner_halo_kernel"));
+        } else {
+            // no copy for this stream: chunks of whole rows, which need none
+            r.chunk = (int)std::min<u64>((u64)d.total, ceil_div((u64)d.chunk, (u64)d.tiles) * (u64)d.tiles);
+            r.grid = (unsigned)ceil_div(ceil_div((u64)d.total, (u64)r.chunk), (u64)d.slots);
+        }
     }
     if constexpr (sizeof(T) == 4) {
         if (d.mfma) {
-            if (d.ocb == 3) launch_mfma<3, 2>(d, x, bias, s);
-            else if (d.ocb == 2) launch_mfma_nb<2>(d, x, bias, s);
-            else launch_mfma_nb<1>(d, x, bias, s);
+            if (d.ocb == 3) launch_mfma<3, 2>(d, r, x, bias, s);
+            else if (d.ocb == 2) launch_mfma_nb<2>(d, r, x, bias, s);
+            else launch_mfma_nb<1>(d, r, x, bias, s);
             return check_launch("conv_mfma32_kernel");
         }
     }
     if constexpr (sizeof(T) == 8) {
-        if (d.lane) return launch_lane(d, x, bias, s);
+        if (d.lane) return launch_lane(d, r, x, bias, s);
     }
-    launch_valu_of<T>(d, x, bias, s);
+    launch_valu_of<T>(d, r, x, bias, s);
     return check_launch("conv_valu_kernel");
 }
 

@@ -1,7 +1,9 @@
 // The FP64 and FP32 modes of the Conv1d plans (conv_direct.hip).
 #pragma once
 
-#include "common.hpp"
+#include <memory>
+
+#include "stream_scratch.hpp"
 
 namespace bkma {
 
@@ -17,10 +19,11 @@ struct DirectConv {
     int groups = 0;          // channel groups
     int TN = 0, pitch = 0;   // columns per tile, LDS row pitch in elements
     int tiles = 0, total = 0, chunk = 0, owners = 0;
+    int slots = 1;           // owners per work-group
     unsigned grid = 0;
     u64 lds_bytes = 0;
     void *w = nullptr;       // packed weights (device, owned by the plan)
-    void *halo = nullptr;    // the columns after the owners' chunks, [owners][C][K-1] (device, owned by the plan)
+    std::unique_ptr<StreamScratch> halo;  // the columns after the owners' chunks, [owners][C][K-1]
 };
 
 // The chunk of an owner: tiles [first, end) of the flattened (batch element,
@@ -48,6 +51,7 @@ __host__ __device__ __forceinline__ ConvChunk conv_chunk(int owner, int chunk, i
 bkma_status direct_conv_create(bkma_dtype dt, int B, int C, int L, int K, const void *weight, hipStream_t s,
                                DirectConv *out);
 void direct_conv_free(DirectConv &d);
+// Runs of one plan may overlap on several streams.
 bkma_status direct_conv_run(const DirectConv &d, void *x, const void *bias, hipStream_t s);
 
 }  // namespace bkma
