@@ -258,7 +258,15 @@ bkma_status bkma_adv_plan_create_with(const bkma_adv_params *params, bkma_dtype 
                                       const bkma_tuned_config *cfg, bkma_adv_plan **out);
 bkma_status bkma_adv_plan_describe(const bkma_adv_plan *plan, bkma_tuned_config *cfg, char *name,
                                    uint64_t name_len);
-/* nsteps in-place steps on `data` (16-byte aligned, the plan's dtype). */
+/* nsteps in-place steps on `data` (16-byte aligned, the plan's dtype).  Runs of
+ * one plan on different arrays may overlap on several streams, in several
+ * graphs and from several threads (not with HYBRID, whose scratch is shared).
+ * Plans that cut lines into segments (large shifts, long lines) keep a buffer
+ * for the segments' halos, some part of the array's size, for each of up to 8
+ * streams and 8 graph captures: the first stream's is allocated with the plan,
+ * another's at its first run.  A run on a ninth stream waits for the device and
+ * takes over the buffer used longest ago; a ninth capture takes over the first
+ * one's, whose graph must then not run beside it. */
 bkma_status bkma_adv_plan_run(bkma_adv_plan *plan, void *data, uint64_t nsteps, void *stream);
 void bkma_adv_plan_destroy(bkma_adv_plan *plan);
 /* The compiled configurations of `dtype` (the autotuner's search space):

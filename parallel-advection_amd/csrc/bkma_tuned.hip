@@ -36,6 +36,7 @@
 #include "adv_stream.hpp"
 #include "adv_tile.hpp"
 #include "common.hpp"
+#include "stream_scratch.hpp"
 
 namespace bkma {
 
@@ -148,19 +149,17 @@ struct TunedPlan {
     u64 lds_bytes = 0;
     int lds_threads = 256;  // threads per work-group: 256, 512 or 1024
     // LINE_LDS with the coefficients in registers (adv_tile.hpp, adv_strip.hpp):
-    // the tiles of consecutive slabs and their snapshot buffers (owned)
+    // the tiles of consecutive slabs and where their halo snapshots lie in a
+    // stream's buffer
     std::vector<TileShape> tiles;
-    std::vector<void *> tile_halos;
-    void *spare = nullptr;  // a second array that pairs of passes go through (owned)
+    std::vector<u64> tile_halo_at;
+    void *spare = nullptr;  // a second array that pairs of passes go through (owned; for the first stream)
     // Default plans: runs of alt_min to alt_max steps take another plan with
     // the same results (owned)
     std::unique_ptr<TunedPlan> alt;
     u64 alt_min = 1, alt_max = 0;
-    void *halo = nullptr;  // segmented mode: halo snapshot buffer (owned)
+    std::unique_ptr<StreamScratch> scratch;  // segments: a stream's halo snapshots
     ~TunedPlan() {
-        if (halo) (void)hipFree(halo);
-        for (void *h : tile_halos)
-            if (h) (void)hipFree(h);
         if (spare) (void)hipFree(spare);
         if (slab_shift) (void)hipFree(slab_shift);
         if (gscratch.data) (void)hipFree(gscratch.data);
@@ -406,7 +405,7 @@ bkma_status lds_shape(const bkma_adv_params &p, bkma_dtype dt, i64 seg_rows, i64
 }
 
 template <class T, int NT>
-bkma_status launch_lds_nt(const TunedPlan &pl, void *data, hipStream_t s, int ns) {
+bkma_status launch_lds_nt(const TunedPlan &pl, void *data, hipStream_t s, int ns, void *halo) {
     LdsArgs a = pl.lds;
     a.ns = ns;
     const i64 nunits = a.slabs > 1 ? ((i64)pl.params.n0 + a.slabs - 1) / a.slabs : (i64)pl.params.n0 * a.nseg;
@@ -417,11 +416,11 @@ bkma_status launch_lds_nt(const TunedPlan &pl, void *data, hipStream_t s, int ns
         sa.seg_rows = a.seg_rows * a.chunk_segs;
         sa.nseg = a.nchunk;
         const unsigned cunits = (unsigned)std::min<i64>((i64)pl.params.n0 * a.nchunk, kLdsMaxGrid);
-        hipLaunchKernelGGL(halo_snapshot_kernel<T>, dim3(cunits), dim3(256), 0, s, (const T *)data, (T *)pl.halo, sa);
+        hipLaunchKernelGGL(halo_snapshot_kernel<T>, dim3(cunits), dim3(256), 0, s, (const T *)data, (T *)halo, sa);
         BKMA_TRY(check_launch("halo_snapshot_kernel"));
         auto k = ns > 1 ? adv_line_chunk_kernel<T, NT, true> : adv_line_chunk_kernel<T, NT, false>;
         BKMA_HIP_TRY(hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)pl.lds_bytes));
-        hipLaunchKernelGGL(k, dim3(cunits), dim3(NT), (size_t)pl.lds_bytes, s, (T *)data, (const T *)pl.halo, a);
+        hipLaunchKernelGGL(k, dim3(cunits), dim3(NT), (size_t)pl.lds_bytes, s, (T *)data, (const T *)halo, a);
     } else {
         auto k = adv_line_lds_kernel<T, false, NT>;
         BKMA_HIP_TRY(hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)pl.lds_bytes));
@@ -433,16 +432,17 @@ bkma_status launch_lds_nt(const TunedPlan &pl, void *data, hipStream_t s, int ns
 // LINE_LDS work-groups of 4, 8 or 16 wavefronts (one work-group per CU when
 // the staged rows take most of the LDS: more waves hide the HBM latency)
 template <class T>
-bkma_status launch_lds(const TunedPlan &pl, void *data, hipStream_t s, int ns) {
+bkma_status launch_lds(const TunedPlan &pl, void *data, hipStream_t s, int ns, void *halo) {
     switch (pl.lds_threads) {
-        case 512: return launch_lds_nt<T, 512>(pl, data, s, ns);
-        case 1024: return launch_lds_nt<T, 1024>(pl, data, s, ns);
-        default: return launch_lds_nt<T, 256>(pl, data, s, ns);
+        case 512: return launch_lds_nt<T, 512>(pl, data, s, ns, halo);
+        case 1024: return launch_lds_nt<T, 1024>(pl, data, s, ns, halo);
+        default: return launch_lds_nt<T, 256>(pl, data, s, ns, halo);
     }
 }
 
-// One pass of ns steps (ns <= the plan's steps per pass).
-bkma_status plan_launch(const TunedPlan &pl, void *data, hipStream_t s, int ns, void *from = nullptr) {
+// One pass of ns steps (ns <= the plan's steps per pass).  `halo`: the stream's
+// buffer for snapshots, `from`: the array to read instead of `data`.
+bkma_status plan_launch(const TunedPlan &pl, void *data, hipStream_t s, int ns, void *halo, void *from = nullptr) {
     if (pl.cfg.strategy == BKMA_STRATEGY_PLAIN) {
         const bkma_span3d none{nullptr, 0, 0, 0};
         return bkma_adv_run(BKMA_IMPL_ADAPTIVE_WG, pl.dtype, data, &pl.params, &pl.optim, none, s);
@@ -464,12 +464,15 @@ bkma_status plan_launch(const TunedPlan &pl, void *data, hipStream_t s, int ns, 
         return st;
     }
     if (!pl.tiles.empty()) {
-        for (size_t k = 0; k < pl.tiles.size(); ++k)
-            BKMA_TRY(launch_tile(pl.tiles[k], pl.dtype, true, false, data, pl.tile_halos[k], ns, s, from));
+        for (size_t k = 0; k < pl.tiles.size(); ++k) {
+            void *h = halo ? (char *)halo + pl.tile_halo_at[k] : nullptr;
+            BKMA_TRY(launch_tile(pl.tiles[k], pl.dtype, true, false, data, h, ns, s, from));
+        }
         return BKMA_OK;
     }
     if (pl.cfg.strategy == BKMA_STRATEGY_LINE_LDS)
-        return pl.dtype == BKMA_F64 ? launch_lds<double>(pl, data, s, ns) : launch_lds<float>(pl, data, s, ns);
+        return pl.dtype == BKMA_F64 ? launch_lds<double>(pl, data, s, ns, halo)
+                                    : launch_lds<float>(pl, data, s, ns, halo);
     if (pl.cfg.strategy == BKMA_STRATEGY_LINE_SHFL) {
         ShflArgs a;
         a.p = make_adv_dev(pl.params);
@@ -502,20 +505,27 @@ bkma_status plan_steps(const TunedPlan &pl, void *data, u64 nsteps, hipStream_t 
     // FP64 storage of the register tiles: equal passes (the split does not
     // change the results, and a short last pass pays a whole staging)
     if (!pl.tiles.empty() && pl.dtype == BKMA_F64 && nsteps > ns) ns = ceil_div(nsteps, ceil_div(nsteps, ns));
-    if (pl.spare && nsteps > ns) {
+    std::unique_lock<std::mutex> held;  // until everything is enqueued
+    void *halo = nullptr;
+    if (pl.scratch) {
+        held = pl.scratch->lock();
+        halo = pl.scratch->get(s, true);
+        if (!halo) return fail(BKMA_ERR_OUT_OF_MEMORY, "tuned advection: no halo buffer for another stream");
+    }
+    if (pl.spare && pl.scratch->first(halo) && nsteps > ns) {
         // an odd number of passes: the first in place
         u64 t = 0;
         for (u64 left = ceil_div(nsteps, ns); left > 0; --left) {
             const int k = (int)std::min<u64>(ns, nsteps - t);
             t += (u64)k;
-            if (t == (u64)k && left % 2 == 1) BKMA_TRY(plan_launch(pl, data, s, k));
-            else if (left % 2 == 0) BKMA_TRY(plan_launch(pl, pl.spare, s, k, data));
-            else BKMA_TRY(plan_launch(pl, data, s, k, pl.spare));
+            if (t == (u64)k && left % 2 == 1) BKMA_TRY(plan_launch(pl, data, s, k, halo));
+            else if (left % 2 == 0) BKMA_TRY(plan_launch(pl, pl.spare, s, k, halo, data));
+            else BKMA_TRY(plan_launch(pl, data, s, k, halo, pl.spare));
         }
         return BKMA_OK;
     }
-    for (u64 t = 0; t + ns <= nsteps; t += ns) BKMA_TRY(plan_launch(pl, data, s, (int)ns));
-    if (nsteps % ns) BKMA_TRY(plan_launch(pl, data, s, (int)(nsteps % ns)));
+    for (u64 t = 0; t + ns <= nsteps; t += ns) BKMA_TRY(plan_launch(pl, data, s, (int)ns, halo));
+    if (nsteps % ns) BKMA_TRY(plan_launch(pl, data, s, (int)(nsteps % ns), halo));
     return BKMA_OK;
 }
 
@@ -558,6 +568,15 @@ i64 resident_blocks(const StreamVariant &v, int ns, int pair_ahead) {
 struct Candidate {
     bkma_tuned_config cfg;
 };
+
+bkma_status make_scratch(TunedPlan *pl, u64 bytes) {
+    pl->scratch.reset(new (std::nothrow) StreamScratch());
+    if (!pl->scratch || !pl->scratch->create(bytes)) {
+        pl->scratch.reset();
+        return fail(BKMA_ERR_OUT_OF_MEMORY, "tuned advection: halo buffer allocation failed");
+    }
+    return BKMA_OK;
+}
 
 bkma_status build_plan(const bkma_adv_params &p, bkma_dtype dt, const bkma_tuned_config &cfg, TunedPlan *pl) {
     std::string why;
@@ -656,19 +675,16 @@ bkma_status build_plan(const bkma_adv_params &p, bkma_dtype dt, const bkma_tuned
         const int ns = steps_per_pass(cfg);
         if (ns <= kTileMaxSteps && shift_supported(p, &why)) pl->tiles = tile_parts(p, dt == BKMA_F64 ? 8 : 4, ns, lds_max, cfg.prefetch == kStripForm);
         if (!pl->tiles.empty()) {
+            u64 halo_bytes = 0;
             for (const TileShape &t : pl->tiles) {
-                pl->tile_halos.push_back(nullptr);
-                if (t.halo_bytes && hipMalloc(&pl->tile_halos.back(), t.halo_bytes) != hipSuccess) {
-                    pl->tile_halos.back() = nullptr;
-                    return fail(BKMA_ERR_OUT_OF_MEMORY, "tuned advection: halo buffer allocation failed");
-                }
+                pl->tile_halo_at.push_back(halo_bytes);
+                halo_bytes += (t.halo_bytes + 255) / 256 * 256;
             }
+            if (halo_bytes) BKMA_TRY(make_scratch(pl, halo_bytes));
             // Long halos (large shifts, so few steps per pass): their snapshot
             // is read and written in every pass, so pairs of passes go through a
             // second array instead, where there is room for one of up to 4 GiB
             // ([256][262144][4] FP32, 20 steps of 4 per pass: 6.42 -> 5.66 ms).
-            u64 halo_bytes = 0;
-            for (const TileShape &t : pl->tiles) halo_bytes += t.halo_bytes;
             const u64 bytes = p.n0 * p.n1 * p.n2 * (dt == BKMA_F64 ? 8 : 4);
             if (ns <= 16 && halo_bytes * 8 >= bytes && bytes <= (4ull << 30) && hipMalloc(&pl->spare, bytes) != hipSuccess) {
                 (void)hipGetLastError();
@@ -701,10 +717,7 @@ bkma_status build_plan(const bkma_adv_params &p, bkma_dtype dt, const bkma_tuned
             const u64 esz = dt == BKMA_F64 ? 8 : 4;
             const u64 bytes =
                 p.n0 * (u64)pl->lds.nchunk * (u64)pl->lds.ns * (u64)(pl->lds.hb_max + pl->lds.ha_max) * p.n2 * esz;
-            if (hipMalloc(&pl->halo, std::max<u64>(bytes, 16)) != hipSuccess) {
-                pl->halo = nullptr;
-                return fail(BKMA_ERR_OUT_OF_MEMORY, "tuned advection: halo buffer allocation failed");
-            }
+            BKMA_TRY(make_scratch(pl, bytes));
         }
         pl->cfg.seg_rows = pl->lds.nseg > 1 ? (int32_t)pl->lds.seg_rows : 0;
         pl->cfg.chunk_segs = (int32_t)(pl->lds.nseg > 1 ? pl->lds.chunk_segs : pl->lds.slabs);
@@ -1022,10 +1035,10 @@ bkma_status time_plan(const TunedPlan &pl, void *buf, int reps, hipStream_t s, f
     hipEvent_t e0, e1;
     BKMA_HIP_TRY(hipEventCreate(&e0));
     BKMA_HIP_TRY(hipEventCreate(&e1));
-    bkma_status st = plan_launch(pl, buf, s, ns);  // warm-up
+    bkma_status st = plan_steps(pl, buf, (u64)ns, s);  // warm-up
     if (st == BKMA_OK) {
         (void)hipEventRecord(e0, s);
-        for (int r = 0; r < reps && st == BKMA_OK; ++r) st = plan_launch(pl, buf, s, ns);
+        for (int r = 0; r < reps && st == BKMA_OK; ++r) st = plan_steps(pl, buf, (u64)ns, s);
         (void)hipEventRecord(e1, s);
         (void)hipEventSynchronize(e1);
         (void)hipEventElapsedTime(ms, e0, e1);

@@ -33,7 +33,7 @@ public:
         buffers_.push_back(b);
         return true;
     }
-    u64 bytes() const { return bytes_; }
+    bool first(const void *data) const { return !buffers_.empty() && buffers_[0].data == data; }
 
     // Held from get() until the run is enqueued: a buffer may change hands.
     std::unique_lock<std::mutex> lock() { return std::unique_lock<std::mutex>(mutex_); }

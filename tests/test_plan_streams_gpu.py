@@ -99,3 +99,33 @@ def test_conv(cuda, case):
     _check_streams(plan.run, arrays, [torch.cuda.Stream() for _ in arrays])
     _check_graphs(plan.run, arrays[:3])
     _check_threads(plan.run, arrays[:4])
+
+
+# (n0, n1, n2), dt * n1, what: strips and LDS segments through halo snapshots, large shifts through a second array (the
+# first stream) and through snapshots (the others), whole lines, column pairs beside strips, old LINE_LDS segments
+PLANS = [((64, 9000, 6), 3.0, "strip"), ((16, 20000, 4), 100.0, "regs"), ((200, 500, 3), 2.0, "whole"),
+         ((1024, 160, 64), 1.0, "pair"), ((8, 9000, 6), 3.0, "old")]
+
+
+@pytest.mark.parametrize("case", PLANS, ids=lambda c: f"{c[2]}-{'x'.join(map(str, c[0]))}")
+@pytest.mark.parametrize("dtype", [B.F64, B.F32], ids=["f64", "f32"])
+def test_advection(cuda, dtype, case):
+    import torch
+    (n0, n1, n2), s, what = case
+    p = B.make_params(n0, n1, n2, dt=s / n1, minRealVx=-1.0, maxRealVx=1.0)
+    c = None
+    if what in ("strip", "regs", "old"):
+        c = B.TunedConfig()
+        c.strategy, c.prefetch, c.steps_per_pass = B.STRATEGY_LINE_LDS, {"strip": 6, "regs": 5, "old": 0}[what], 3
+        c.seg_rows = 500 if what == "old" else 0
+    plan = B.AdvPlan(p, dtype, config=c)
+    name = plan.describe()[1]
+    print(name, flush=True)
+    assert ("seg" in name) == (what in ("strip", "regs", "old"))
+    t = torch.float64 if dtype == B.F64 else torch.float32
+    arrays = [torch.rand((n0, n1, n2), dtype=t, device="cuda") for _ in range(10)]  # two streams more than buffers
+    for steps in (6, 7):
+        run = lambda a: plan.run(a, steps)  # noqa: B023, E731
+        _check_streams(run, arrays, [torch.cuda.Stream() for _ in arrays], rounds=2)
+    _check_graphs(run, arrays[:3])
+    _check_threads(run, arrays[:4])
