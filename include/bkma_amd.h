@@ -264,7 +264,9 @@ bkma_status bkma_adv_plan_describe(const bkma_adv_plan *plan, bkma_tuned_config 
  * Plans that cut lines into segments (large shifts, long lines) keep a buffer
  * for the segments' halos, some part of the array's size, for each of up to 8
  * streams and 8 graph captures: the first stream's is allocated with the plan,
- * another's at its first run.  A run on a ninth stream waits for the device and
+ * another's at its first run.  Where the halos are more than an eighth of an
+ * array of up to 4 GiB, the first stream's buffer has the whole array's size
+ * if there is room, and pairs of passes go through it.  A run on a ninth stream waits for the device and
  * takes over the buffer used longest ago; a ninth capture takes over the first
  * one's, whose graph must then not run beside it. */
 bkma_status bkma_adv_plan_run(bkma_adv_plan *plan, void *data, uint64_t nsteps, void *stream);

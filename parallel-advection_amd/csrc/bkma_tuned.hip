@@ -153,14 +153,13 @@ struct TunedPlan {
     // stream's buffer
     std::vector<TileShape> tiles;
     std::vector<u64> tile_halo_at;
-    void *spare = nullptr;  // a second array that pairs of passes go through (owned; for the first stream)
+    bool spare = false;  // the first stream's buffer is also a second array, which pairs of passes go through
     // Default plans: runs of alt_min to alt_max steps take another plan with
     // the same results (owned)
     std::unique_ptr<TunedPlan> alt;
     u64 alt_min = 1, alt_max = 0;
     std::unique_ptr<StreamScratch> scratch;  // segments: a stream's halo snapshots
     ~TunedPlan() {
-        if (spare) (void)hipFree(spare);
         if (slab_shift) (void)hipFree(slab_shift);
         if (gscratch.data) (void)hipFree(gscratch.data);
         if (fork) (void)hipEventDestroy(fork);
@@ -513,14 +512,15 @@ bkma_status plan_steps(const TunedPlan &pl, void *data, u64 nsteps, hipStream_t 
         if (!halo) return fail(BKMA_ERR_OUT_OF_MEMORY, "tuned advection: no halo buffer for another stream");
     }
     if (pl.spare && pl.scratch->first(halo) && nsteps > ns) {
-        // an odd number of passes: the first in place
+        // an odd number of passes: the first in place, with its snapshot where
+        // the second array is from then on
         u64 t = 0;
         for (u64 left = ceil_div(nsteps, ns); left > 0; --left) {
             const int k = (int)std::min<u64>(ns, nsteps - t);
             t += (u64)k;
             if (t == (u64)k && left % 2 == 1) BKMA_TRY(plan_launch(pl, data, s, k, halo));
-            else if (left % 2 == 0) BKMA_TRY(plan_launch(pl, pl.spare, s, k, halo, data));
-            else BKMA_TRY(plan_launch(pl, data, s, k, halo, pl.spare));
+            else if (left % 2 == 0) BKMA_TRY(plan_launch(pl, halo, s, k, nullptr, data));
+            else BKMA_TRY(plan_launch(pl, data, s, k, nullptr, halo));
         }
         return BKMA_OK;
     }
@@ -569,9 +569,9 @@ struct Candidate {
     bkma_tuned_config cfg;
 };
 
-bkma_status make_scratch(TunedPlan *pl, u64 bytes) {
+bkma_status make_scratch(TunedPlan *pl, u64 bytes, u64 first) {
     pl->scratch.reset(new (std::nothrow) StreamScratch());
-    if (!pl->scratch || !pl->scratch->create(bytes)) {
+    if (!pl->scratch || !pl->scratch->create(bytes, first)) {
         pl->scratch.reset();
         return fail(BKMA_ERR_OUT_OF_MEMORY, "tuned advection: halo buffer allocation failed");
     }
@@ -680,16 +680,14 @@ bkma_status build_plan(const bkma_adv_params &p, bkma_dtype dt, const bkma_tuned
                 pl->tile_halo_at.push_back(halo_bytes);
                 halo_bytes += (t.halo_bytes + 255) / 256 * 256;
             }
-            if (halo_bytes) BKMA_TRY(make_scratch(pl, halo_bytes));
             // Long halos (large shifts, so few steps per pass): their snapshot
             // is read and written in every pass, so pairs of passes go through a
             // second array instead, where there is room for one of up to 4 GiB
             // ([256][262144][4] FP32, 20 steps of 4 per pass: 6.42 -> 5.66 ms).
             const u64 bytes = p.n0 * p.n1 * p.n2 * (dt == BKMA_F64 ? 8 : 4);
-            if (ns <= 16 && halo_bytes * 8 >= bytes && bytes <= (4ull << 30) && hipMalloc(&pl->spare, bytes) != hipSuccess) {
-                (void)hipGetLastError();
-                pl->spare = nullptr;
-            }
+            pl->spare = ns <= 16 && halo_bytes * 8 >= bytes && bytes <= (4ull << 30) &&
+                        make_scratch(pl, halo_bytes, std::max(bytes, halo_bytes)) == BKMA_OK;
+            if (halo_bytes && !pl->spare) BKMA_TRY(make_scratch(pl, halo_bytes, halo_bytes));
             const TileShape &t = pl->tiles[0];
             pl->ns = ns;
             pl->cfg.steps_per_pass = ns;
@@ -717,7 +715,7 @@ bkma_status build_plan(const bkma_adv_params &p, bkma_dtype dt, const bkma_tuned
             const u64 esz = dt == BKMA_F64 ? 8 : 4;
             const u64 bytes =
                 p.n0 * (u64)pl->lds.nchunk * (u64)pl->lds.ns * (u64)(pl->lds.hb_max + pl->lds.ha_max) * p.n2 * esz;
-            BKMA_TRY(make_scratch(pl, bytes));
+            BKMA_TRY(make_scratch(pl, bytes, bytes));
         }
         pl->cfg.seg_rows = pl->lds.nseg > 1 ? (int32_t)pl->lds.seg_rows : 0;
         pl->cfg.chunk_segs = (int32_t)(pl->lds.nseg > 1 ? pl->lds.chunk_segs : pl->lds.slabs);

@@ -593,7 +593,7 @@ bkma_status direct_conv_create(bkma_dtype dt, int B, int C, int L, int K, const 
     bool room = hipMalloc(&d.w, wcount * esz) == hipSuccess;
     if (room && d.tiles > 1 && K > 1) {
         d.halo.reset(new (std::nothrow) StreamScratch());
-        room = d.halo && d.halo->create((u64)d.owners * C * (K - 1) * esz);
+        room = d.halo && d.halo->create((u64)d.owners * C * (K - 1) * esz, (u64)d.owners * C * (K - 1) * esz);
     }
     if (!room) {
         direct_conv_free(d);

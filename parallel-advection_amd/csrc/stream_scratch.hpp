@@ -25,11 +25,12 @@ public:
         for (const Buffer &b : buffers_) (void)hipFree(b.data);
     }
 
-    // The first buffer, for the first stream that asks; false: no memory.
-    bool create(u64 bytes) {
+    // Buffers of `bytes` each, the first one, for the first stream that asks, of
+    // `first` bytes and allocated here; false: no memory.
+    bool create(u64 bytes, u64 first) {
         bytes_ = bytes;
         Buffer b;
-        if (!allocate(&b.data)) return false;
+        if (!allocate(&b.data, first)) return false;
         buffers_.push_back(b);
         return true;
     }
@@ -69,7 +70,7 @@ public:
         }
         if (alike < (k.captured ? kCaptures : kStreams)) {
             Buffer b;
-            if (allocate(&b.data)) {
+            if (allocate(&b.data, bytes_)) {
                 b.taken = true;
                 b.key = k;
                 buffers_.push_back(b);
@@ -107,10 +108,10 @@ private:
         return b.data;
     }
     // Also while this or another thread captures: an allocation is no part of it.
-    bool allocate(void **p) {
+    static bool allocate(void **p, u64 bytes) {
         hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
         const bool swapped = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
-        const bool ok = hipMalloc(p, bytes_ ? bytes_ : 16) == hipSuccess;
+        const bool ok = hipMalloc(p, bytes ? bytes : 16) == hipSuccess;
         if (!ok) {
             (void)hipGetLastError();
             *p = nullptr;

@@ -129,3 +129,16 @@ def test_advection(cuda, dtype, case):
         _check_streams(run, arrays, [torch.cuda.Stream() for _ in arrays], rounds=2)
     _check_graphs(run, arrays[:3])
     _check_threads(run, arrays[:4])
+
+
+def test_second_array_also_holds_the_snapshots(cuda):
+    """Large shifts: the plan keeps one array's size, not the halos' (0.7 of it here) beside it."""
+    import torch
+    p = B.make_params(64, 262144, 4, dt=1e-3, minRealVx=-1.0, maxRealVx=1.0)
+    size = 64 * 262144 * 4 * 4
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    plan = B.AdvPlan(p, B.F32)
+    taken = free - torch.cuda.mem_get_info()[0]
+    assert "seg" in plan.describe()[1] and 0.5 * size < taken < 1.2 * size
+    plan.close()
