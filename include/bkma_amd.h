@@ -246,10 +246,10 @@ typedef struct bkma_tuned_config {
 typedef struct bkma_adv_plan bkma_adv_plan;
 
 /* autotune = 0: heuristic choice; 1: time the feasible variants on a scratch
- * array of the same line shape (allocated and freed inside the call).  Either
- * may hold a second kernel with the same results for short or for long runs;
- * the plan's name then gives both, joined by a plus, and its configuration the
- * first. */
+ * array of the same line shape (allocated and freed inside the call), the best
+ * ones at runs of 1 to 96 steps.  Either may hold a second kernel with the same
+ * results for short or for long runs; the plan's name then gives both, joined
+ * by a plus, and its configuration the first. */
 bkma_status bkma_adv_plan_create(const bkma_adv_params *params, bkma_dtype dtype, int32_t autotune, void *stream,
                                  bkma_adv_plan **out);
 /* A plan with an explicit configuration (BKMA_ERR_UNSUPPORTED if it is not

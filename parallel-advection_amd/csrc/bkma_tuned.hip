@@ -36,6 +36,7 @@
 #include "adv_stream.hpp"
 #include "adv_tile.hpp"
 #include "common.hpp"
+#include "run_choice.hpp"
 #include "stream_scratch.hpp"
 
 namespace bkma {
@@ -1023,28 +1024,57 @@ Alternative alternative(const bkma_adv_params &p, bkma_dtype dt, const TunedPlan
     return a;
 }
 
-// Time per step of full passes, of at most kTimedSteps steps: the staging of a
-// pass of up to 256 steps weighs as in a run of a few tens (FP32
-// [2048][1024][512], 50 steps: column pair 18.3 ms, strips 18.6, which passes
-// of 256 steps would favour by a tenth).
-constexpr int kTimedSteps = 48;
-bkma_status time_plan(const TunedPlan &pl, void *buf, int reps, hipStream_t s, float *ms) {
-    const int ns = std::min(pl.ns, kTimedSteps);
+// Time of one run of `steps` steps (mean of `reps`), if `warm` after one that
+// is not timed.
+bkma_status time_run(const TunedPlan &pl, void *buf, u64 steps, int reps, bool warm, hipStream_t s, float *ms) {
     hipEvent_t e0, e1;
     BKMA_HIP_TRY(hipEventCreate(&e0));
     BKMA_HIP_TRY(hipEventCreate(&e1));
-    bkma_status st = plan_steps(pl, buf, (u64)ns, s);  // warm-up
+    bkma_status st = warm ? plan_steps(pl, buf, steps, s) : BKMA_OK;
     if (st == BKMA_OK) {
         (void)hipEventRecord(e0, s);
-        for (int r = 0; r < reps && st == BKMA_OK; ++r) st = plan_steps(pl, buf, (u64)ns, s);
+        for (int r = 0; r < reps && st == BKMA_OK; ++r) st = plan_steps(pl, buf, steps, s);
         (void)hipEventRecord(e1, s);
         (void)hipEventSynchronize(e1);
         (void)hipEventElapsedTime(ms, e0, e1);
-        *ms /= (float)(reps * ns);  // per step
+        *ms /= (float)reps;
     }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     return st;
+}
+
+// Time per step of full passes of at most kTimedSteps steps (two passes where
+// pairs of them go through a second array).
+constexpr int kTimedSteps = 48;
+bkma_status time_plan(const TunedPlan &pl, void *buf, int reps, hipStream_t s, float *ms) {
+    const int steps = pl.spare ? 2 * pl.ns : std::min(pl.ns, kTimedSteps);
+    BKMA_TRY(time_run(pl, buf, (u64)steps, reps, true, s, ms));
+    *ms /= (float)steps;
+    return BKMA_OK;
+}
+
+// Times the fastest tile candidate and the fastest other one over run lengths;
+// *alt has max = 0 where one of them takes all runs.
+bkma_status tune_runs(const bkma_adv_params &sub, bkma_dtype dt, const bkma_tuned_config &tile,
+                      const bkma_tuned_config &other, void *buf, hipStream_t s, bkma_tuned_config *main,
+                      Alternative *alt) {
+    TunedPlan pt, po;
+    BKMA_TRY(build_plan(sub, dt, tile, &pt));
+    BKMA_TRY(build_plan(sub, dt, other, &po));
+    float t[kRuns], o[kRuns];
+    for (int i = 0; i < kRuns; ++i) {
+        const bool brief = kRunSteps[i] < 20;
+        BKMA_TRY(time_run(pt, buf, kRunSteps[i], brief ? 3 : 1, brief, s, &t[i]));
+        BKMA_TRY(time_run(po, buf, kRunSteps[i], brief ? 3 : 1, brief, s, &o[i]));
+    }
+    const u64 shared = dt == BKMA_F64 || pt.ns == po.ns ? ~(u64)0 : (u64)std::min(pt.ns, po.ns);
+    const RunChoice c = choose_runs(t, o, shared);
+    *main = c.tile_long ? tile : other;
+    alt->cfg = c.tile_short ? tile : other;
+    alt->min = 1;
+    alt->max = c.up_to;
+    return BKMA_OK;
 }
 
 }  // namespace
@@ -1072,9 +1102,12 @@ extern "C" bkma_status bkma_adv_plan_create(const bkma_adv_params *params, bkma_
         return heuristic_score(a, dtype, *params) < heuristic_score(b, dtype, *params);
     });
 
+    bool tuned = false;  // candidates were timed: nothing that was not goes beside the choice
+    Alternative alt;
     if (autotune && cands.size() > 1) {
         // Time the candidates on a scratch array of whole slabs, large enough
-        // to fill the GPU several times over (contents do not affect timing).
+        // to fill the GPU several times over, and of random values (the clock
+        // under a load of arithmetic depends on the bits that switch).
         // The whole problem (up to 2 Gi cells) is used: occupancy and tail
         // effects depend on the number of work units.
         bkma_adv_params sub = *params;
@@ -1087,17 +1120,25 @@ extern "C" bkma_status bkma_adv_plan_create(const bkma_adv_params *params, bkma_
             (void)hipGetLastError();
             buf = nullptr;
         }
-        if (buf) (void)hipMemsetAsync(buf, 0, bytes, as_stream(stream));
-        float best_ms = 1e30f;
+        if (buf) (void)bkma_fill_uniform(dtype, buf, sub.n0 * elems_per_slab, 1, stream);
+        float best_ms[2] = {1e30f, 1e30f};  // of the other candidates, of the tiles
+        bkma_tuned_config fastest[2];
         for (const auto &c : cands) {
             if (!buf) break;
             TunedPlan pl;
             if (build_plan(sub, dtype, c, &pl) != BKMA_OK) continue;
             float ms = 0;
-            if (time_plan(pl, buf, 3, as_stream(stream), &ms) == BKMA_OK && ms < best_ms) {
-                best_ms = ms;
-                best = c;
+            if (time_plan(pl, buf, 3, as_stream(stream), &ms) == BKMA_OK && ms < best_ms[is_tile(c)]) {
+                best_ms[is_tile(c)] = ms;
+                fastest[is_tile(c)] = c;
             }
+        }
+        if (best_ms[0] < 1e30f || best_ms[1] < 1e30f) {
+            tuned = true;
+            best = fastest[best_ms[1] < best_ms[0]];
+            if (best_ms[0] < 1e30f && best_ms[1] < 1e30f &&
+                tune_runs(sub, dtype, fastest[1], fastest[0], buf, as_stream(stream), &best, &alt) != BKMA_OK)
+                alt.max = 0;
         }
         (void)hipFree(buf);
         (void)hipGetLastError();
@@ -1118,12 +1159,14 @@ extern "C" bkma_status bkma_adv_plan_create(const bkma_adv_params *params, bkma_
             });
             st = build_plan(*params, dtype, best, pl);
         }
+        alt.max = 0;
     }
     if (st != BKMA_OK) {
         delete pl;
         return st;
     }
-    if (const auto alt = alternative(*params, dtype, *pl, cands); alt.max) {
+    if (!tuned) alt = alternative(*params, dtype, *pl, cands);
+    if (alt.max) {
         pl->alt.reset(new (std::nothrow) TunedPlan());
         if (pl->alt && build_plan(*params, dtype, alt.cfg, pl->alt.get()) == BKMA_OK) {
             pl->alt_min = alt.min;

@@ -7,6 +7,7 @@
 
 #include "conv_direct.hpp"
 #include "mfma_ops.hpp"
+#include "run_choice.hpp"
 
 using namespace bkma;
 
@@ -154,5 +155,17 @@ long long probe_conv_chunk_faults(int B, int tiles, int TN, int K, int chunk) {
         }
     }
     return bad;
+}
+// Host only: the autotuner's choice for times t (tiles) and o (the other plan) of runs of steps[] steps; out =
+// {tiles take short runs, tiles take long runs}.  Returns the largest short run, or -1 - n where n lengths are timed.
+long long probe_choose_runs(const float *t, const float *o, int runs, unsigned long long shared, int out[2]) {
+    if (runs != kRuns) return -1 - kRuns;
+    const RunChoice c = choose_runs(t, o, shared);
+    out[0] = c.tile_short;
+    out[1] = c.tile_long;
+    return (long long)c.up_to;
+}
+void probe_run_steps(unsigned long long *steps) {
+    for (int i = 0; i < kRuns; ++i) steps[i] = kRunSteps[i];
 }
 }
