@@ -281,7 +281,7 @@ int32_t bkma_adv_plan_variants(bkma_dtype dtype, bkma_tuned_config *out, int32_t
 /* Many independent problems (each its own [n0][n1][n2] array, dt and
  * velocity grid; the reference runs one bkma_run per problem and step)
  * advanced together: as groups of LINE_LDS tiles (bkma_adv_batch_create), or
- * with every pass of ns steps (the batch's steps per pass, 1 .. 4) as one persistent launch over all problems' work items (plus a
+ * with every pass of ns steps (the batch's steps per pass) as one persistent launch over all problems' work items (plus a
  * halo-snapshot launch when a problem's lines exceed the LDS budget), which
  * bkma_adv_batch_run(use_graph = 1) captures the passes into hipGraphs,
  * replayed on later calls.  A run of nsteps steps makes nsteps / ns passes of
@@ -300,11 +300,13 @@ typedef struct bkma_adv_batch bkma_adv_batch;
  * many fused steps as its tiles hold, with the results of one step per pass;
  * long runs launch the groups on up to four streams between the caller's
  * earlier and later work, and use_graph makes no difference (there are few
- * launches).  autotune then has nothing to choose.  Otherwise autotune = 1 times the LDS
- * budgets (32 KB .. the device limit), work-group sizes and steps per pass
- * (1 .. 4) on the problems' own arrays, which the timing steps modify: create
- * the batch before initialising the data.  autotune = 0: 64 KB, 256 threads,
- * one step per pass. */
+ * launches).  autotune = 1 then chooses, for F32 storage, between these and
+ * passes of 2, 3, 4, 8, 16 or 32 steps with one rounding each (F64 results do
+ * not depend on it).
+ * Otherwise it times the LDS budgets (32 KB .. the device limit), work-group
+ * sizes and steps per pass (1 .. 4).  The timing steps run on the problems' own
+ * arrays and modify them: create the batch before initialising the data.
+ * autotune = 0: 64 KB, 256 threads, one step per pass. */
 bkma_status bkma_adv_batch_create(const bkma_adv_problem *problems, int32_t nproblems, bkma_dtype dtype,
                                   int32_t autotune, void *stream, bkma_adv_batch **out);
 /* A batch with an explicit configuration: LDS budget per work-group (bytes),

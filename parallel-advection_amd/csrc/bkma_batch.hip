@@ -4,8 +4,9 @@
 // those: the slab ranges whose tiles are of one kind, work-group size and depth
 // share a launch, and a launch fuses as many steps as the depth, the values rounded
 // to FP32 after every step (FP32 storage), so that the results are those of
-// one step per pass.  Otherwise, and for an explicit configuration, one
-// persistent launch per pass:
+// one step per pass.  An autotuned FP32 batch may take passes of several steps
+// instead, each one launch per group and one rounding.  Otherwise, and for an
+// explicit configuration, one persistent launch per pass:
 //
 // Each problem ([n0][n1][n2], its own dt and velocity grid) is cut into work
 // items of the LINE_LDS kind.  A problem whose slab fits the LDS budget is
@@ -166,6 +167,7 @@ struct AdvBatch {
     hipStream_t side[kBatchSides] = {};  // owned, created when groups use them
     hipEvent_t ev_fork = nullptr, ev_join[kBatchSides] = {};
     u64 tile_units = 0, tile_seg_units = 0;
+    bool each_step = true;  // results of one step per pass; else passes of ns steps
 
     void drop_groups() {
         for (auto &g : groups) (void)hipFree(g.table);
@@ -214,8 +216,8 @@ template <class T> static bkma_status batch_pass(const AdvBatch &b, hipStream_t 
 static bkma_status batch_steps(const AdvBatch &b, u64 nsteps, hipStream_t s) {
     if (!b.groups.empty()) {
         // one step per pass in the results (FP32 storage rounds after every
-        // step), as many fused steps as a group's tiles hold in the launches:
-        // equal passes
+        // step): as many fused steps as a group's tiles hold in the launches,
+        // equal passes; else passes of the batch's steps
         // The groups are independent: in long runs they take turns on a few
         // streams, so that the tails and the small groups do not leave the GPU
         // idle (one stream -> four: 6550 -> 6240 us for 48 problems and 32
@@ -234,8 +236,9 @@ static bkma_status batch_steps(const AdvBatch &b, u64 nsteps, hipStream_t s) {
             const TileGroup &g = b.groups[i];
             const u64 passes = ceil_div(nsteps, (u64)g.ns);
             for (u64 k = 0, t = 0; k < passes && st == BKMA_OK; ++k) {
-                const u64 end = nsteps * (k + 1) / passes;
-                st = launch_tile_group(g, b.dtype, true, (int)(end - t), lanes > 1 && b.lane[i] ? b.side[b.lane[i] - 1] : s);
+                const u64 end = b.each_step ? nsteps * (k + 1) / passes : std::min(t + (u64)g.ns, nsteps);
+                st = launch_tile_group(g, b.dtype, b.each_step, (int)(end - t),
+                                       lanes > 1 && b.lane[i] ? b.side[b.lane[i] - 1] : s);
                 t = end;
             }
         }
@@ -353,9 +356,10 @@ static bkma_status build_items(AdvBatch &b, u64 budget, int threads, int ns) {
     return BKMA_OK;
 }
 
-// The tile groups of a batch, one step per pass in its results; false (and
-// no groups) where some problem has no tile or there is no room.
-static bool build_groups(AdvBatch &b) {
+// The tile groups of a batch for passes of ns steps (0: the results of one
+// step per pass); false (and no groups) where some problem has no tile or there
+// is no room.
+static bool build_groups(AdvBatch &b, int ns) {
     u64 lds_max = 0;
     if (lds_limit_bytes(&lds_max) != BKMA_OK) return false;
     const u64 esz = b.dtype == BKMA_F64 ? 8 : 4;
@@ -367,7 +371,7 @@ static bool build_groups(AdvBatch &b) {
     std::vector<Part> parts;
     for (size_t j = 0; j < n; ++j) {
         const bkma_adv_params &p = b.problems[j].params;
-        const std::vector<TileShape> ts = tile_parts(p, esz, 0, lds_max, true);
+        const std::vector<TileShape> ts = tile_parts(p, esz, ns, lds_max, true);
         if (ts.empty()) return false;
         for (const TileShape &t : ts) {
             if (t.a.units > tile_launch_units(t.threads)) return false;  // a group's part is in one launch
@@ -446,7 +450,8 @@ static bool build_groups(AdvBatch &b) {
         b.halos.clear();
         return false;
     }
-    b.ns = 1;
+    b.ns = std::max(1, ns);
+    b.each_step = ns == 0;
     b.lds_budget = 0;
     b.grid = 0;
     for (const TileGroup &g : b.groups) {
@@ -542,11 +547,52 @@ extern "C" bkma_status bkma_adv_batch_create(const bkma_adv_problem *problems, i
             return bail(fail(BKMA_ERR_DEVICE, "batch: ordering after the caller's stream"));
     }
 
+    // Time of `steps` steps after `warm` that are not timed.  The timing runs
+    // update the problems in place: the autotuner is meant to run before the data
+    // is initialised (or on scratch data).
+    auto time_steps = [&](u64 warm, u64 steps, float *ms) {
+        hipEvent_t e0, e1;
+        (void)hipEventCreate(&e0);
+        (void)hipEventCreate(&e1);
+        bkma_status r = batch_steps(*b, warm, b->stream);
+        (void)hipEventRecord(e0, b->stream);
+        if (r == BKMA_OK) r = batch_steps(*b, steps, b->stream);
+        (void)hipEventRecord(e1, b->stream);
+        (void)hipEventSynchronize(e1);
+        (void)hipEventElapsedTime(ms, e0, e1);
+        (void)hipEventDestroy(e0);
+        (void)hipEventDestroy(e1);
+        return r;
+    };
+    // Later work on the caller's stream sees the timing runs' updates.
+    auto order_after = [&]() {
+        if (hipEventRecord(b->ev_out, b->stream) != hipSuccess ||
+            hipStreamWaitEvent(as_stream(stream), b->ev_out, 0) != hipSuccess)
+            return fail(BKMA_ERR_DEVICE, "batch: ordering the caller's stream after the timing runs");
+        return BKMA_OK;
+    };
+
     // The register tiles cover lines from 16 rows on; measured on 48 problems
     // of 16 .. 256 slabs, 64 .. 8192 rows and 1, 8 or 64 columns (345 M cells,
     // FP32, 32 steps): 0.28 ms per step against 0.94 of the persistent launch
     // below, whose every step reads and writes HBM and evaluates every foot.
-    if (build_groups(*b)) {
+    if (build_groups(*b, 0)) {
+        if (autotune && dtype == BKMA_F32) {
+            // rounded at every step, or passes of fewer roundings: what is fastest
+            int best = 0;
+            float best_ms = 1e30f;
+            for (int ns : {0, 2, 3, 4, 8, 16, 32}) {
+                float ms = 0;
+                if ((ns == 0 || build_groups(*b, ns)) && time_steps(32, 64, &ms) == BKMA_OK && ms < best_ms) {
+                    best_ms = ms;
+                    best = ns;
+                }
+            }
+            if (!build_groups(*b, best) && !build_groups(*b, 0))
+                return bail(fail(BKMA_ERR_OUT_OF_MEMORY, "batch: tile groups"));
+            st = order_after();
+            if (st != BKMA_OK) return bail(st);
+        }
         *out = b;
         return BKMA_OK;
     }
@@ -575,38 +621,24 @@ extern "C" bkma_status bkma_adv_batch_create(const bkma_adv_problem *problems, i
                     done = true;
                     break;
                 }
-                // The timing runs update the problems in place: the autotuner is
-                // meant to run before the data is initialised (or on scratch data).
-                hipEvent_t e0, e1;
-                (void)hipEventCreate(&e0);
-                (void)hipEventCreate(&e1);
-                st = batch_steps(*b, (u64)ns, b->stream);
-                (void)hipEventRecord(e0, b->stream);
-                if (st == BKMA_OK) st = batch_steps(*b, 3 * (u64)ns, b->stream);
-                (void)hipEventRecord(e1, b->stream);
-                (void)hipEventSynchronize(e1);
                 float ms = 0;
-                (void)hipEventElapsedTime(&ms, e0, e1);
-                (void)hipEventDestroy(e0);
-                (void)hipEventDestroy(e1);
+                if (time_steps((u64)ns, 3 * (u64)ns, &ms) != BKMA_OK) continue;
                 ms /= (float)ns;  // per 3 steps
-                if (st == BKMA_OK && ms < best_ms) {
+                if (ms < best_ms) {
                     best_ms = ms;
                     best_budget = bud;
                     best_threads = thr;
                     best_ns = ns;
                 }
-                st = BKMA_OK;
             }
         }
     }
     if (best_budget == 0) return bail(fail(BKMA_ERR_UNSUPPORTED, "advection batch: no LDS budget covers the problems"));
     st = build_items(*b, best_budget, best_threads, best_ns);
     if (st != BKMA_OK) return bail(st);
-    if (autotune) {  // later work on the caller's stream sees the timing runs' updates
-        if (hipEventRecord(b->ev_out, b->stream) != hipSuccess ||
-            hipStreamWaitEvent(as_stream(stream), b->ev_out, 0) != hipSuccess)
-            return bail(fail(BKMA_ERR_DEVICE, "batch: ordering the caller's stream after the timing runs"));
+    if (autotune) {
+        st = order_after();
+        if (st != BKMA_OK) return bail(st);
     }
     *out = b;
     return BKMA_OK;
