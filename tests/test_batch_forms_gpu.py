@@ -1,5 +1,6 @@
 """The forms of a ragged batch and what autotuning chooses in them: the groups of tiles (every problem has one), whose
-FP32 passes may round at every step or once per pass, against the oracle's restatement."""
+FP32 passes may round at every step or once per pass, and the persistent launch (an explicit configuration, or a
+problem whose shifts no tile holds), against the oracle's restatement."""
 import numpy as np
 import pytest
 
@@ -48,5 +49,35 @@ def test_autotuned_tiles(cuda, dtype, specs):
     batch, info, arrays, refs = _batch(dtype, specs, autotune=True)
     assert info["grid"] > 0 and info["steps_per_pass"] in ((1,) if dtype == B.F64 else (1, 2, 3, 4, 8, 16, 32))
     for nsteps in (37, 1, 37):
+        _check(batch, arrays, refs, specs, dtype, nsteps, info["steps_per_pass"])
+    batch.close()
+
+
+# Whole lines, chained segments, and one problem whose shifts (-410 to 358 cells) exceed its segments of 1024 rows less
+# the halos, which then are not chained: an item each.
+PERSISTENT = [(3, 8192, 8, 2e-3), (2, 16384, 1, 1e-3), (4, 640, 64, 1e-3), (5, 100, 1, 2e-3), (16, 16384, 8, 2.5e-2)]
+
+
+@pytest.mark.parametrize("threads", [256, 1024])
+@pytest.mark.parametrize("dtype", [B.F64, B.F32], ids=["f64", "f32"])
+def test_persistent_graphs_and_unchained_segments(cuda, dtype, threads):
+    """Runs of more and fewer steps than a graph holds (32), replayed, and without graphs."""
+    budget = 65536 if dtype == B.F64 else 32768
+    batch, info, arrays, refs = _batch(dtype, PERSISTENT, config=(budget, threads, 1))
+    assert info["lds_budget"] == budget and info["steps_per_pass"] == 1
+    assert info["items"] - info["segmented_items"] == 5 and info["segmented_items"] > 16 * 16384 // 256
+    for nsteps, graph in ((33, True), (2, True), (33, True), (3, False)):
+        _check(batch, arrays, refs, PERSISTENT, dtype, nsteps, 1, graph)
+    batch.close()
+
+
+@pytest.mark.parametrize("dtype", [B.F64, B.F32], ids=["f64", "f32"])
+def test_persistent_autotuned(cuda, dtype):
+    """A shift of 2000 cells leaves a tile's segment too few rows, so the batch stays with the persistent launch and its
+    own candidates."""
+    specs = [(3, 20000, 1, 0.1), (30, 6000, 2, 1e-3), (12, 300, 8, 1e-3)]
+    batch, info, arrays, refs = _batch(dtype, specs, autotune=True)
+    assert info["lds_budget"] in (32768, 65536, 98304, B.query_lds_bytes() - 1024) and 1 <= info["steps_per_pass"] <= 4
+    for nsteps in (5, 33, 5):
         _check(batch, arrays, refs, specs, dtype, nsteps, info["steps_per_pass"])
     batch.close()
