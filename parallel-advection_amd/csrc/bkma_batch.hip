@@ -644,8 +644,8 @@ extern "C" bkma_status bkma_adv_batch_create(const bkma_adv_problem *problems, i
     return BKMA_OK;
 }
 
-// Time steps per captured graph: a run of n steps replays the graph of
-// kGraphSteps steps n / kGraphSteps times, then the graph of the remainder.
+// Time steps per captured graph, at most: a run replays the graph of the most
+// whole passes that fit, then the graph of the remainder.
 constexpr u64 kGraphSteps = 32;
 
 // The instantiated graph of `nsteps` (<= kGraphSteps) batch steps, captured
@@ -680,11 +680,13 @@ extern "C" bkma_status bkma_adv_batch_run(bkma_adv_batch *b, uint64_t nsteps, in
     BKMA_HIP_TRY(hipEventRecord(b->ev_in, cs));
     BKMA_HIP_TRY(hipStreamWaitEvent(b->stream, b->ev_in, 0));
     if (use_graph && b->groups.empty()) {  // a group's pass fuses many steps: few launches, no graph
-        // Graphs of kGraphSteps steps and of the remainder: at most
-        // kGraphSteps graphs per batch, each captured on first use.
-        const u64 full = nsteps / kGraphSteps, rem = nsteps % kGraphSteps;
+        // Graphs of whole passes (FP32 results depend on where they end) and of
+        // the remainder: at most kGraphSteps graphs per batch, each captured on
+        // first use.
+        const u64 most = kGraphSteps / (u64)b->ns * (u64)b->ns;
+        const u64 full = nsteps / most, rem = nsteps % most;
         hipGraphExec_t gfull = nullptr, grem = nullptr;
-        if (full) BKMA_TRY(batch_graph(*b, kGraphSteps, &gfull));
+        if (full) BKMA_TRY(batch_graph(*b, most, &gfull));
         if (rem) BKMA_TRY(batch_graph(*b, rem, &grem));
         for (u64 i = 0; i < full; ++i) BKMA_HIP_TRY(hipGraphLaunch(gfull, b->stream));
         if (rem) BKMA_HIP_TRY(hipGraphLaunch(grem, b->stream));

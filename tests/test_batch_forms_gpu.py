@@ -71,6 +71,15 @@ def test_persistent_graphs_and_unchained_segments(cuda, dtype, threads):
     batch.close()
 
 
+def test_graphs_end_with_a_pass(cuda):
+    """Three steps per pass: a run of more steps than a graph holds makes the same passes with graphs as without."""
+    specs = [(4, 640, 8, 1e-3), (2, 16384, 1, 1e-3)]
+    for graph in (True, False):
+        batch, info, arrays, refs = _batch(B.F32, specs, config=(98304, 256, 3))
+        _check(batch, arrays, refs, specs, B.F32, 70, 3, graph)
+        batch.close()
+
+
 @pytest.mark.parametrize("dtype", [B.F64, B.F32], ids=["f64", "f32"])
 def test_persistent_autotuned(cuda, dtype):
     """A shift of 2000 cells leaves a tile's segment too few rows, so the batch stays with the persistent launch and its
