@@ -90,3 +90,14 @@ def test_persistent_autotuned(cuda, dtype):
     for nsteps in (5, 33, 5):
         _check(batch, arrays, refs, specs, dtype, nsteps, info["steps_per_pass"])
     batch.close()
+
+
+@pytest.mark.parametrize("autotune", [False, True], ids=["default", "autotuned"])
+@pytest.mark.parametrize("dtype", [B.F64, B.F32], ids=["f64", "f32"])
+def test_short_and_long_runs_in_turn(cuda, dtype, autotune):
+    """Many small problems: runs of a step or two take the persistent launch, longer ones the groups."""
+    specs = [(20 + 3 * j, 64 * (1 + j % 11), (1, 8, 64)[j % 3], 5e-4 + 4e-5 * j) for j in range(30)]
+    batch, info, arrays, refs = _batch(dtype, specs, autotune=autotune)
+    for nsteps in (1, 2, 3, 5, 1, 34, 2, 1):
+        _check(batch, arrays, refs, specs, dtype, nsteps, info["steps_per_pass"])
+    batch.close()
