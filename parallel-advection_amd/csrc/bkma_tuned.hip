@@ -159,6 +159,7 @@ struct TunedPlan {
     // the same results (owned)
     std::unique_ptr<TunedPlan> alt;
     u64 alt_min = 1, alt_max = 0;
+    std::unique_ptr<TunedPlan> one;  // runs of one step (owned; null: as the others)
     std::unique_ptr<StreamScratch> scratch;  // segments: a stream's halo snapshots
     ~TunedPlan() {
         if (slab_shift) (void)hipFree(slab_shift);
@@ -501,6 +502,7 @@ bkma_status plan_launch(const TunedPlan &pl, void *data, hipStream_t s, int ns, 
 // nsteps steps: full passes of the plan's steps per pass, then the rest.
 bkma_status plan_steps(const TunedPlan &pl, void *data, u64 nsteps, hipStream_t s) {
     if (pl.alt && nsteps >= pl.alt_min && nsteps <= pl.alt_max) return plan_steps(*pl.alt, data, nsteps, s);
+    if (pl.one && nsteps == 1) return plan_steps(*pl.one, data, nsteps, s);
     u64 ns = (u64)pl.ns;
     // FP64 storage of the register tiles: equal passes (the split does not
     // change the results, and a short last pass pays a whole staging)
@@ -1024,6 +1026,39 @@ Alternative alternative(const bkma_adv_params &p, bkma_dtype dt, const TunedPlan
     return a;
 }
 
+// The plan of a default tile plan's runs of one step, which a pass of many steps
+// is not laid out for; false: none.  One step, us, the plan's pass / the other
+// (by which alone these shapes had been quicker before there were tiles):
+//  - strips on whole lines / LDS tiles of one step: FP64 [2000][64][33] 44 / 23,
+//    [20000][64][8] 75 / 38, [300][1000][100] 126 / 92, [20000][777][1] 112 / 88,
+//    [4000][2000][8] 254 / 257; FP32 [2000][2500][8] 109 / 85, [3000][128][33]
+//    69 / 55;
+//  - FP32 segments with shifts so large that a pass has at most four steps /
+//    the longest segment of the form that computes the coefficients at every
+//    step: [256][262144][4] 738 / 646, [64][262144][4] 189 / 153 (FP64
+//    [256][262144][4] 977 / 1229; eight steps: FP32 [64][65536][8] 84 / 106).
+bool one_step(const bkma_adv_params &p, bkma_dtype dt, const TunedPlan &pl,
+              const std::vector<bkma_tuned_config> &cands, bkma_tuned_config *cfg) {
+    if (pl.tiles.empty() || (pl.alt && pl.alt_min <= 1)) return false;
+    bool segments = true;
+    for (const TileShape &t : pl.tiles) segments = segments && !t.wrap;
+    if (!segments) {
+        if (!pl.tiles[0].e || !pl.tiles[0].wrap || pl.tiles.size() > 1) return false;
+        *cfg = pl.cfg;
+        cfg->prefetch = kTileRows;
+        cfg->steps_per_pass = 1;
+        return true;
+    }
+    const bkma_tuned_config *best = nullptr;
+    for (const auto &c : cands)
+        if (c.strategy == BKMA_STRATEGY_LINE_LDS && !is_tile(c) && c.seg_rows > 0 && steps_per_pass(c) == 1 &&
+            (!best || heuristic_score(*best, dt, p) < heuristic_score(c, dt, p)))
+            best = &c;
+    if (!best || dt != BKMA_F32 || pl.ns > 4) return false;
+    *cfg = *best;
+    return true;
+}
+
 // Time of one run of `steps` steps (mean of `reps`), if `warm` after one that
 // is not timed.
 bkma_status time_run(const TunedPlan &pl, void *buf, u64 steps, int reps, bool warm, hipStream_t s, float *ms) {
@@ -1174,6 +1209,14 @@ extern "C" bkma_status bkma_adv_plan_create(const bkma_adv_params *params, bkma_
             pl->name += "+" + pl->alt->name;
         } else {
             pl->alt.reset();
+            (void)hipGetLastError();
+        }
+    }
+    bkma_tuned_config single;
+    if (!tuned && one_step(*params, dtype, *pl, cands, &single)) {
+        pl->one.reset(new (std::nothrow) TunedPlan());
+        if (!pl->one || build_plan(*params, dtype, single, pl->one.get()) != BKMA_OK) {
+            pl->one.reset();
             (void)hipGetLastError();
         }
     }
