@@ -37,6 +37,7 @@
 //   the CU's other work-group computes).
 #include <algorithm>
 #include <new>
+#include <utility>
 
 #include "conv_direct.hpp"
 
@@ -495,11 +496,15 @@ bkma_status direct_conv_create(bkma_dtype dt, int B, int C, int L, int K, const 
             hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
             return fail(BKMA_ERR_DEVICE, "conv1d plan: device query");
         double least = 0;
-        for (int tn : {128, 64, 32}) {
+        // rows 16 banks apart modulo 64; where no tile fits so but the VALU form's
+        // would, 48 apart, which also spreads an operand's four rows (32 columns
+        // and K - 1 of 600 channels: 80 or 48 a row)
+        for (const auto &[apart, tn] : {std::pair{16, 128}, {16, 64}, {16, 32}, {48, 32}}) {
             const int nb = tn / 16 / d.parts;
             if (nb > 8 || nb < 2) continue;
             if (tn > 32 && tn / 2 >= Lout && nb > 2) continue;  // half of the tile would stay empty
-            const int pitch = tn + K - 1 + ((16 - (tn + K - 1)) % 64 + 64) % 64;  // 16 banks modulo 64
+            if (apart == 48 && (d.TN || (u64)C * (u64)(64 + K - 1) * esz > lds_max)) continue;
+            const int pitch = tn + K - 1 + ((apart - (tn + K - 1)) % 64 + 64) % 64;
             const u64 b = rows * (u64)pitch * esz;
             if (b > lds_max) continue;
             const void *kern = mfma_kernel_of(d.ocb, nb);
