@@ -41,6 +41,7 @@ struct ShflArgs {
     AdvDev p;
     const int *slab_shift;  // [n0][2]: smallest and largest d = i1 - leftNode of each line
     int ns;                 // steps in this pass
+    i64 first;              // line of the launch's first work-group
 };
 
 // DPP on the two halves of an FP64 register.  Lanes without a source lane
@@ -192,7 +193,7 @@ __global__ __launch_bounds__(64 * NW) void adv_line_shfl_kernel(T *__restrict__ 
     static_assert(E == 4 || E == 8, "4 or 8 cells per lane");
     __shared__ double xch[NW > 1 ? 2 * NW * 2 * E : 1];
     const AdvDev &p = a.p;
-    const i64 i0 = blockIdx.x;
+    const i64 i0 = a.first + blockIdx.x;
     const int g = threadIdx.x, lane = g & 63, w = g >> 6;
     T *line = data + i0 * p.n1 + (i64)g * E;  // n1 = 64 * E * NW
 
@@ -238,7 +239,7 @@ __global__ __launch_bounds__(256) void adv_line_row16_kernel(T *__restrict__ dat
     static_assert(TW >= 6 && TW <= 8, "window of 6 to 8 cells");
     const AdvDev &p = a.p;
     const int r = threadIdx.x & 15;
-    const i64 i0 = (i64)blockIdx.x * 16 + (threadIdx.x >> 4);
+    const i64 i0 = a.first + (i64)blockIdx.x * 16 + (threadIdx.x >> 4);
     const bool valid = i0 < p.n0;  // whole rows are valid or not
     T *cell = data + (valid ? i0 : 0) * 16 + r;
     double f = valid ? (double)*cell : 0.0;

@@ -1,5 +1,7 @@
 // Instances and launcher of the register/DPP kernel for contiguous lines
 // (adv_shfl.hpp).
+#include <algorithm>
+
 #include "adv_shfl.hpp"
 
 namespace bkma {
@@ -8,8 +10,15 @@ namespace {
 
 template <class T, int E, int NW>
 bkma_status launch_nw(void *data, const ShflArgs &a, i64 n0, hipStream_t s) {
-    hipLaunchKernelGGL((adv_line_shfl_kernel<T, E, NW>), dim3((unsigned)n0), dim3(64 * NW), 0, s, (T *)data, a);
-    return check_launch("adv_line_shfl_kernel");
+    // a launch has fewer than 2^32 threads
+    constexpr i64 most = 0xffffffffLL / (64 * NW);
+    ShflArgs r = a;
+    for (r.first = 0; r.first < n0; r.first += most) {
+        const unsigned lines = (unsigned)std::min(most, n0 - r.first);
+        hipLaunchKernelGGL((adv_line_shfl_kernel<T, E, NW>), dim3(lines), dim3(64 * NW), 0, s, (T *)data, r);
+        BKMA_TRY(check_launch("adv_line_shfl_kernel"));
+    }
+    return BKMA_OK;
 }
 
 // Wavefronts per line: 1 .. 16 with 4 cells per lane, 1 .. 8 with 8.
@@ -37,9 +46,14 @@ bkma_status launch_t(int cells, int nw, void *data, const ShflArgs &a, i64 n0, h
 
 template <class T, int WMIN, int TW>
 bkma_status launch_row(void *data, const ShflArgs &a, i64 n0, hipStream_t s) {
-    const i64 groups = (n0 + 15) / 16;
-    hipLaunchKernelGGL((adv_line_row16_kernel<T, WMIN, TW>), dim3((unsigned)groups), dim3(256), 0, s, (T *)data, a);
-    return check_launch("adv_line_row16_kernel");
+    constexpr i64 most = 0xffffffffLL / 256 * 16;  // lines of a launch of fewer than 2^32 threads
+    ShflArgs r = a;
+    for (r.first = 0; r.first < n0; r.first += most) {
+        const i64 groups = (std::min(most, n0 - r.first) + 15) / 16;
+        hipLaunchKernelGGL((adv_line_row16_kernel<T, WMIN, TW>), dim3((unsigned)groups), dim3(256), 0, s, (T *)data, r);
+        BKMA_TRY(check_launch("adv_line_row16_kernel"));
+    }
+    return BKMA_OK;
 }
 
 template <class T, int WMIN>
