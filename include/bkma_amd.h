@@ -263,10 +263,10 @@ bkma_status bkma_adv_plan_describe(const bkma_adv_plan *plan, bkma_tuned_config 
  * graphs and from several threads (not with HYBRID, whose scratch is shared).
  * Plans that cut lines into segments (large shifts, long lines) keep a buffer
  * for the segments' halos, some part of the array's size, for each of up to 8
- * streams and 8 graph captures: the first stream's is allocated with the plan,
- * another's at its first run.  Where the halos are more than an eighth of an
- * array of up to 4 GiB, the first stream's buffer has the whole array's size
- * if there is room, and pairs of passes go through it.  A run on a ninth stream waits for the device and
+ * streams and 8 graph captures: the first one's is allocated with the plan,
+ * another's at its first run (no other run allocates anything).  Where the halos are more than an eighth of an
+ * array of up to 4 GiB, the first buffer has the whole array's size if there is
+ * room, and pairs of passes go through it.  A run on a ninth stream waits for the device and
  * takes over the buffer used longest ago; a ninth capture takes over the first
  * one's, whose graph must then not run beside it. */
 bkma_status bkma_adv_plan_run(bkma_adv_plan *plan, void *data, uint64_t nsteps, void *stream);
@@ -365,10 +365,10 @@ bkma_status bkma_conv1d_plan_create(bkma_conv_mode mode, bkma_dtype io_dtype, ui
                                     void *stream, bkma_conv1d_plan **out);
 /* F64 and F32 modes: runs of one plan on different arrays may overlap on
  * several streams, in several graphs and from several threads.  The plan keeps
- * a small buffer (some columns of x) for each of up to 8 streams and 8 graph
- * captures, allocated at a stream's first run (the first stream's at creation);
- * runs beyond them need none and split the work less finely.  The other modes
- * share one buffer: runs of one plan must not overlap. */
+ * small buffers (some columns of x), allocated at creation, for the first one to
+ * four streams and graph captures that run it; runs on others need none and
+ * split the work less finely.  The other modes share one buffer: runs of one
+ * plan must not overlap. */
 bkma_status bkma_conv1d_plan_run(bkma_conv1d_plan *plan, void *x, void *stream);
 bkma_status bkma_conv1d_plan_describe(const bkma_conv1d_plan *plan, char *name, uint64_t name_len);
 /* FP8 mode: the input is quantized as x / scale (scale > 0; default 1). */

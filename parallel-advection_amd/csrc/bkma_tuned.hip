@@ -574,7 +574,7 @@ struct Candidate {
 
 bkma_status make_scratch(TunedPlan *pl, u64 bytes, u64 first) {
     pl->scratch.reset(new (std::nothrow) StreamScratch());
-    if (!pl->scratch || !pl->scratch->create(bytes, first)) {
+    if (!pl->scratch || !pl->scratch->create(bytes, first, 0)) {
         pl->scratch.reset();
         return fail(BKMA_ERR_OUT_OF_MEMORY, "tuned advection: halo buffer allocation failed");
     }

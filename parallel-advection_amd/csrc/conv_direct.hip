@@ -597,8 +597,10 @@ bkma_status direct_conv_create(bkma_dtype dt, int B, int C, int L, int K, const 
     d.grid = (unsigned)ceil_div((u64)d.owners, (u64)d.slots);
     bool room = hipMalloc(&d.w, wcount * esz) == hipSuccess;
     if (room && d.tiles > 1 && K > 1) {
+        // for up to four streams and captures, within a quarter of x
+        const u64 bytes = (u64)d.owners * C * (K - 1) * esz, quarter = (u64)B * C * L * esz / 4;
         d.halo.reset(new (std::nothrow) StreamScratch());
-        room = d.halo && d.halo->create((u64)d.owners * C * (K - 1) * esz, (u64)d.owners * C * (K - 1) * esz);
+        room = d.halo && d.halo->create(bytes, bytes, (int)std::min<u64>(3, quarter / bytes));
     }
     if (!room) {
         direct_conv_free(d);

@@ -13,8 +13,8 @@ namespace bkma {
 
 class StreamScratch {
 public:
-    // Streams, and captures, that have a buffer of their own.  A buffer stays
-    // with its stream until the plan goes; further streams get none, or take
+    // Streams, and captures, that may have a buffer of their own.  A buffer
+    // stays with its stream until the plan goes; further streams get none, or take
     // over the one that was used longest ago.
     static constexpr size_t kStreams = 8, kCaptures = 8;
 
@@ -25,13 +25,15 @@ public:
         for (const Buffer &b : buffers_) (void)hipFree(b.data);
     }
 
-    // Buffers of `bytes` each, the first one, for the first stream that asks, of
-    // `first` bytes and allocated here; false: no memory.
-    bool create(u64 bytes, u64 first) {
+    // Buffers of `bytes` each.  The first one, for the first stream or capture
+    // that asks, has `first` bytes and is allocated here, and so are `more` others
+    // as far as there is memory; false: none for the first.
+    bool create(u64 bytes, u64 first, int more) {
         bytes_ = bytes;
         Buffer b;
         if (!allocate(&b.data, first)) return false;
         buffers_.push_back(b);
+        for (; more > 0 && allocate(&b.data, bytes); --more) buffers_.push_back(b);
         return true;
     }
     bool first(const void *data) const { return !buffers_.empty() && buffers_[0].data == data; }
@@ -41,10 +43,11 @@ public:
 
     // The buffer of a run on stream s, or null.  A stream under capture takes a
     // buffer per capture, since its graph may run beside others later.  Where
-    // there is no memory or there are too many streams: with `wait`, a run
+    // none is left: without `grow` the answer is null; with it another is
+    // allocated, and where there is no memory or there are too many streams, a run
     // outside a capture waits for the device and takes over a buffer (a capture
-    // takes over that of an older one); without it the answer is null.
-    void *get(hipStream_t s, bool wait) {
+    // takes over that of an older one).
+    void *get(hipStream_t s, bool grow) {
         Key k;
         k.stream = s;
         if (s == hipStreamPerThread) k.thread = std::this_thread::get_id();
@@ -59,15 +62,16 @@ public:
         Buffer *oldest = nullptr;
         for (Buffer &b : buffers_) {
             if (b.taken && b.key == k) return use(b);
-            if (!b.taken && !k.captured) {
+            if (!b.taken) {
                 b.taken = true;
                 b.key = k;
                 return use(b);
             }
-            if (!b.taken || b.key.captured != k.captured) continue;
+            if (b.key.captured != k.captured) continue;
             ++alike;
             if (!oldest || b.used < oldest->used) oldest = &b;
         }
+        if (!grow) return nullptr;
         if (alike < (k.captured ? kCaptures : kStreams)) {
             Buffer b;
             if (allocate(&b.data, bytes_)) {
@@ -77,7 +81,7 @@ public:
                 return use(buffers_.back());
             }
         }
-        if (!wait || !oldest) return nullptr;
+        if (!oldest) return nullptr;
         if (!k.captured && hipDeviceSynchronize() != hipSuccess) {
             (void)hipGetLastError();
             return nullptr;

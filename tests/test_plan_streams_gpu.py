@@ -142,3 +142,27 @@ def test_second_array_also_holds_the_snapshots(cuda):
     taken = free - torch.cuda.mem_get_info()[0]
     assert "seg" in plan.describe()[1] and 0.5 * size < taken < 1.2 * size
     plan.close()
+
+
+def test_conv_runs_allocate_nothing(cuda):
+    """On whatever stream, and in a capture."""
+    import torch
+    plan, inputs = _conv(B.CONV_F32, (256, 64, 4096, 33))
+    arrays = inputs(6)
+    streams = [torch.cuda.Stream() for _ in arrays]
+    torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    for a, s in zip(arrays[:3], streams):
+        with torch.cuda.stream(s):
+            plan.run(a)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        plan.run(arrays[3])
+        plan.run(arrays[3])
+    for a, s in zip(arrays[4:], streams[4:]):
+        with torch.cuda.stream(s):
+            plan.run(a)
+    torch.cuda.synchronize()
+    size = 256 * 64 * 32 * 4  # of the columns that one buffer holds, at least
+    assert free - torch.cuda.mem_get_info()[0] < size
