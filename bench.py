@@ -17,7 +17,7 @@ The other workloads run by default too, each with its own `roofline`:
   c0  plain FP64 [256][1024][1], 100 steps (cache-resident: timing only);
   c2  Conv1d x[1024][128][4096], w[128][128][5]: FP64, FP32, bf16 MFMA (FP32 and BF16 storage), bf16x3,
       bf16x6, with errors against the FP64 plan;
-  c3  64 ragged problems, FP32, 200 steps in one hipGraph, against loops of per-problem launches;
+  c3  64 ragged problems, FP32, 200 steps as one autotuned batch, against loops of per-problem launches;
   c4  long lines f[256][262144][4] FP64/FP32, 20 steps; FP8-e4m3 Conv1d x[512][256][8192], w[256][256][7].
 The CPU column is the oracle's FP64 restatement of the reference algorithm on a bounded sample of whole slabs
 of the headline workload.
@@ -392,8 +392,8 @@ def measure_conv(torch, B):
 
 def measure_batch(torch, B):
     """64 ragged problems (seed 3): n1 log-uniform in [64, 16384] (multiple of 64), n0 uniform in [16, 1024],
-    n2 in {1, 8, 64}, dt in [5e-4, 2e-3], FP32, 200 steps; persistent graph-captured batch vs loops of
-    per-problem launches."""
+    n2 in {1, 8, 64}, dt in [5e-4, 2e-3], FP32, 200 steps; one autotuned batch vs loops of per-problem
+    launches."""
     specs = ragged_specs(3, 64)
     arrays = [torch.empty((n0, n1, n2), dtype=torch.float32, device="cuda") for n0, n1, n2, _ in specs]
     params = [B.make_params(n0, n1, n2, dt=dt, minRealVx=-1, maxRealVx=1) for n0, n1, n2, dt in specs]
@@ -413,9 +413,10 @@ def measure_batch(torch, B):
         "s": round(ms * 1e-3, 4), "Gcell_s": round(cells * steps / ms / 1e6, 2),
         "roofline": roofline("hbm", cells * 8 / ns, step_ms, HBM_PEAK_GBS, "GB/s", ms_per_step=round(step_ms, 5),
                              steps_per_pass=ns, effective_GBps=round(cells * 8 / step_ms / 1e6, 1),
-                             note="one pass of steps_per_pass steps = halo snapshot + persistent launch; each "
-                                  "FP32 cell is read and written once per pass (achieved: those bytes per step "
-                                  "time; effective_GBps: one read and write per step)")}
+                             note="one pass of steps_per_pass steps, one FP32 rounding each, = the batch's launches "
+                                  "and their halo snapshots; each FP32 cell is read and written once per pass "
+                                  "(achieved: those bytes per step time, more than moved where launches fuse steps "
+                                  "and round at each; effective_GBps: one read and write per step)")}
     te = event_ms(torch, lambda: batch.run(steps, graph=False))
     out["persistent_no_graph"] = {"s": round(te * 1e-3, 4), "Gcell_s": round(cells * steps / te / 1e6, 2)}
     batch.run_loop(1, 1)
