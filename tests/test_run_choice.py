@@ -57,6 +57,16 @@ def test_choices():
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [B.F64, B.F32], ids=["f64", "f32"])
+def test_lines_in_registers_take_long_passes(cuda, dtype):
+    """LINE_SHFL candidates differ in their steps per pass only, which pay their staging a tenth or so apart."""
+    plan = B.AdvPlan(B.make_params(1 << 17, 1024, 1, dt=1e-3, minRealVx=-1, maxRealVx=1), dtype, autotune=True)
+    cfg, name = plan.describe()
+    plan.close()
+    assert name.startswith("line_shfl<") and cfg.steps_per_pass == 256
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [B.F64, B.F32], ids=["f64", "f32"])
 @pytest.mark.parametrize("shape", [(1024, 160, 64), (130, 256, 1), (6, 20000, 4)], ids=lambda s: "x".join(map(str, s)))
 def test_autotuned_plans_at_every_length(cuda, dtype, shape):
     import torch
