@@ -1158,22 +1158,26 @@ extern "C" bkma_status bkma_adv_plan_create(const bkma_adv_params *params, bkma_
             buf = nullptr;
         }
         if (buf) (void)bkma_fill_uniform(dtype, buf, sub.n0 * elems_per_slab, 1, stream);
-        float best_ms[2] = {1e30f, 1e30f};  // of the other candidates, of the tiles
-        bkma_tuned_config fastest[2];
+        // the fastest of the others, of the tiles, and of HYBRID, which is not
+        // put beside another plan: its runs must not overlap
+        float best_ms[3] = {1e30f, 1e30f, 1e30f};
+        bkma_tuned_config fastest[3];
         for (const auto &c : cands) {
             if (!buf) break;
             TunedPlan pl;
             if (build_plan(sub, dtype, c, &pl) != BKMA_OK) continue;
             float ms = 0;
-            if (time_plan(pl, buf, 3, as_stream(stream), &ms) == BKMA_OK && ms < best_ms[is_tile(c)]) {
-                best_ms[is_tile(c)] = ms;
-                fastest[is_tile(c)] = c;
+            const int kind = is_tile(c) ? 1 : c.strategy == BKMA_STRATEGY_HYBRID ? 2 : 0;
+            if (time_plan(pl, buf, 3, as_stream(stream), &ms) == BKMA_OK && ms < best_ms[kind]) {
+                best_ms[kind] = ms;
+                fastest[kind] = c;
             }
         }
-        if (best_ms[0] < 1e30f || best_ms[1] < 1e30f) {
+        const int win = (int)(std::min_element(best_ms, best_ms + 3) - best_ms);
+        if (best_ms[win] < 1e30f) {
             tuned = true;
-            best = fastest[best_ms[1] < best_ms[0]];
-            if (best_ms[0] < 1e30f && best_ms[1] < 1e30f &&
+            best = fastest[win];
+            if (win != 2 && best_ms[0] < 1e30f && best_ms[1] < 1e30f &&
                 tune_runs(sub, dtype, fastest[1], fastest[0], buf, as_stream(stream), &best, &alt) != BKMA_OK)
                 alt.max = 0;
         }
