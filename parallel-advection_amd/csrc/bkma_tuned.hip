@@ -1081,11 +1081,13 @@ bkma_status time_run(const TunedPlan &pl, void *buf, u64 steps, int reps, bool w
 
 // Time per step of full passes, of at most kTimedSteps steps with tiles (two
 // passes where pairs of them go through a second array).  LINE_SHFL passes of 64
-// and of 256 steps are the same kernel up to there: [2^21][1024][1] FP64 0.94 and
-// 0.84 ms per step of their own passes.
+// and of 256 steps are the same kernel up to there ([2^21][1024][1] FP64 0.94 and
+// 0.84 ms per step of their own passes); they are timed on runs of one length, as
+// the clock falls in the first hundreds of milliseconds of a load.
 constexpr int kTimedSteps = 48;
 bkma_status time_plan(const TunedPlan &pl, void *buf, int reps, hipStream_t s, float *ms) {
-    const int steps = pl.spare ? 2 * pl.ns : pl.tiles.empty() ? pl.ns : std::min(pl.ns, kTimedSteps);
+    const bool shfl = pl.cfg.strategy == BKMA_STRATEGY_LINE_SHFL && pl.ns >= 16;
+    const int steps = shfl ? 256 : pl.spare ? 2 * pl.ns : pl.tiles.empty() ? pl.ns : std::min(pl.ns, kTimedSteps);
     BKMA_TRY(time_run(pl, buf, (u64)steps, reps, true, s, ms));
     *ms /= (float)steps;
     return BKMA_OK;
