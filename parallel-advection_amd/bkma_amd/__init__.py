@@ -396,8 +396,8 @@ class AdvPlan:
 
     def describe(self):
         cfg = TunedConfig()
-        buf = ctypes.create_string_buffer(128)
-        check(lib().bkma_adv_plan_describe(self._h, ctypes.byref(cfg), buf, 128))
+        buf = ctypes.create_string_buffer(512)  # two plans of three parts each
+        check(lib().bkma_adv_plan_describe(self._h, ctypes.byref(cfg), buf, len(buf)))
         return cfg, buf.value.decode()
 
     def close(self) -> None:

@@ -27,6 +27,10 @@ def _fmt(v):
     return str(v)
 
 
+def _cell(text):
+    return text.replace("|", "\\|")  # the parts of a plan's name
+
+
 def report(path, command=None):
     recs = list(_rows(path))
     out = []
@@ -45,7 +49,7 @@ def report(path, command=None):
                 continue
             out.append(f"| {shape} | {r['impl']} | {_fmt(r.get('pref_wg_size'))} | {r['dtype']} | "
                        f"{r['ms_per_step']} | {r['gcell_s']} | {r['GBps']} | {r['arch_eff']} | {r.get('app_eff', '')} | "
-                       f"{_fmt(r.get('l1_err'))} | {r.get('kernel', '')} |")
+                       f"{_fmt(r.get('l1_err'))} | {_cell(r.get('kernel', ''))} |")
         out.append("")
     conv = [r for r in recs if r.get("kind") == "conv1d"]
     if conv:

@@ -292,7 +292,7 @@ class TunedAdvection {
         return Event(q.stream());
     }
     std::string name() const {
-        char buf[128];
+        char buf[512];
         throw_on(bkma_adv_plan_describe(plan_, nullptr, buf, sizeof(buf)));
         return buf;
     }

@@ -32,3 +32,11 @@ def test_single_steps_between_longer_runs(cuda, dtype, case):
             O.advect_f32_blocked(ref, po, n, cfg.steps_per_pass)
         assert np.array_equal(d.cpu().numpy(), ref), n
     plan.close()
+
+
+def test_names_are_whole(cuda):
+    """An autotuned plan of strips and tiles, and another kernel for short runs: more than 128 characters."""
+    plan = B.AdvPlan(B.make_params(4096, 10000, 1, dt=1e-3, minRealVx=-1, maxRealVx=1), B.F64, autotune=True)
+    name = plan.describe()[1]
+    plan.close()
+    assert name.endswith(">") and name.count("<") == name.count(">") == name.count("+") + 1

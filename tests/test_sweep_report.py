@@ -30,3 +30,12 @@ def test_report_tables(tmp_path):
     assert "| (16, 512, 3, 1) | 0.06 | 140.1 | 2241.7 | 33.85 | True |" in out
     assert "| advection tuned/f32 | 0.04 | 0.98 |" in out
     assert "| conv1d adaptivewg/w512/f64 | 0.1 | 1.0 |" in out
+
+
+def test_names_of_several_parts_stay_in_their_cell(tmp_path):
+    rec = {"kind": "advection", "size": "e0", "n0": 4, "n1": 16384, "n2": 1, "impl": "tuned", "dtype": "f64",
+           "kernel": "line_lds<f64,strip6x4|regs5>", "ms_per_step": 0.5, "gcell_s": 3.0, "GBps": 24.0, "arch_eff": 0.003,
+           "l1_err": 1.5e-8, "status": "ok", "app_eff": 1.0}
+    f = tmp_path / "sweep.jsonl"
+    f.write_text(json.dumps(rec) + "\n")
+    assert "| line_lds<f64,strip6x4\\|regs5> |" in R.report(str(f))
