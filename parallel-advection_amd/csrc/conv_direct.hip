@@ -84,13 +84,15 @@ template <class T>
 __global__ void conv_owner_halo_kernel(const T *__restrict__ x, T *__restrict__ halo, int C, int L, int K, int TN,
                                        int tiles, int total, int chunk) {
     const int c = blockIdx.x;
-    const ConvChunk ck = conv_chunk(c, chunk, total, tiles, TN);
-    if (ck.end <= ck.first || ck.b < 0) return;
+    const ConvChunk ck = conv_chunk(c, chunk, total);
+    if (ck.end <= ck.first) return;
+    const int b = (ck.end - 1) / tiles, j0 = ck.column_after(b, tiles, TN);
+    if (j0 == 0x7fffffff) return;
     const int H = K - 1;
     for (int e = threadIdx.x; e < C * H; e += blockDim.x) {
         const int ic = e / H, kk = e - ic * H;
-        const int j = ck.j + kk;
-        halo[(i64)c * C * H + e] = j < L ? x[((i64)ck.b * C + ic) * L + j] : (T)0;
+        const int j = j0 + kk;
+        halo[(i64)c * C * H + e] = j < L ? x[((i64)b * C + ic) * L + j] : (T)0;
     }
 }
 
@@ -124,10 +126,10 @@ __device__ __forceinline__ void stage_columns(const T *__restrict__ xb, T *__res
     }
 }
 
-// hsnap: the owner's copy of the columns after its chunk ck.
+// hsnap: the owner's copy of the row's columns from jend on, which come after its chunk.
 template <class T>
-__device__ __forceinline__ void stage_tile(const T *__restrict__ xb, const T *__restrict__ hsnap, const ConvChunk &ck,
-                                           int b, T *__restrict__ xs, int C, int rows, int L, int j0, int tsh, int H,
+__device__ __forceinline__ void stage_tile(const T *__restrict__ xb, const T *__restrict__ hsnap, int jend,
+                                           T *__restrict__ xs, int C, int rows, int L, int j0, int tsh, int H,
                                            int pitch, bool vec, int t, int nt) {
     const int TN = 1 << tsh;
     // the H columns after the tile, from the snapshot or the row
@@ -135,7 +137,7 @@ __device__ __forceinline__ void stage_tile(const T *__restrict__ xb, const T *__
         const int row = e / H, col = e - row * H, j = j0 + TN + col;
         T v = (T)0;
         if (row < C) {
-            if (ck.copied(b, j)) v = hsnap[row * H + (j - ck.j)];
+            if (j >= jend) v = hsnap[row * H + (j - jend)];
             else if (j < L) v = xb[(i64)row * L + j];
         }
         xs[row * pitch + TN + col] = v;
@@ -157,7 +159,7 @@ __global__ __launch_bounds__(256) void conv_valu_kernel(T *__restrict__ x, const
     const int owner = (int)blockIdx.x * (4 / wpt) + slot;
     T *xs = reinterpret_cast<T *>(conv_lds) + (i64)slot * C * pitch;
     const int Lout = L - K + 1;
-    const ConvChunk ck = conv_chunk(owner, chunk, total, tiles, TN);
+    const ConvChunk ck = conv_chunk(owner, chunk, total);
     for (int it = 0; it < chunk; ++it) {  // the same count for all waves: the barriers are uniform
         const bool on = it < ck.end - ck.first;
         const int tile = on ? ck.first + it : 0;
@@ -165,7 +167,7 @@ __global__ __launch_bounds__(256) void conv_valu_kernel(T *__restrict__ x, const
         const int j0 = t * TN;
         T *xb = x + (i64)b * C * L;
         if (on) {
-            stage_tile(xb, halo + (i64)owner * C * (K - 1), ck, b, xs, C, C, L, j0,
+            stage_tile(xb, halo + (i64)owner * C * (K - 1), ck.column_after(b, tiles, TN), xs, C, C, L, j0,
                        JT == 4 ? 8 : JT == 2 ? 7 : 6, K - 1, pitch, vec, ws * 64 + lane, wpt * 64);
         }
         __syncthreads();
@@ -240,13 +242,13 @@ __global__ __launch_bounds__(256) void conv_lane64_kernel(double *__restrict__ x
     const int ol = lane & (cw - 1), part = lane / cw;
     const int span = JT * (64 / cw);  // columns of a wavefront
     const int blocks = TN / span;
-    const ConvChunk ck = conv_chunk((int)blockIdx.x, chunk, total, tiles, TN);
+    const ConvChunk ck = conv_chunk((int)blockIdx.x, chunk, total);
     for (int tile = ck.first; tile < ck.end; ++tile) {
         const int b = tile / tiles, t = tile - b * tiles;
         const int j0 = t * TN;
         double *xb = x + (i64)b * C * L;
-        stage_tile(xb, halo + (i64)blockIdx.x * C * (KT - 1), ck, b, xs, C, C, L, j0, tsh, KT - 1, pitch, vec,
-                   (int)threadIdx.x, 256);
+        stage_tile(xb, halo + (i64)blockIdx.x * C * (KT - 1), ck.column_after(b, tiles, TN), xs, C, C, L, j0, tsh,
+                   KT - 1, pitch, vec, (int)threadIdx.x, 256);
         __syncthreads();
         for (int item = wave; item < groups * blocks; item += 4) {
             const int g = item / blocks, blk = item - g * blocks;
@@ -305,13 +307,13 @@ __global__ __launch_bounds__(256) void conv_mfma32_kernel(float *__restrict__ x,
     const int TN = 1 << tsh, Lout = L - K + 1;
     const int c4 = (C + 3) / 4, steps = c4 * K;
     const int lc = lane & 15, lr = lane >> 4;
-    const ConvChunk ck = conv_chunk((int)blockIdx.x, chunk, total, tiles, TN);
+    const ConvChunk ck = conv_chunk((int)blockIdx.x, chunk, total);
     for (int tile = ck.first; tile < ck.end; ++tile) {
         const int b = tile / tiles, t = tile - b * tiles;
         const int j0 = t * TN;
         float *xb = x + (i64)b * C * L;
-        stage_tile(xb, halo + (i64)blockIdx.x * C * (K - 1), ck, b, xs, C, 4 * c4, L, j0, tsh, K - 1, pitch, vec,
-                   (int)threadIdx.x, 256);
+        stage_tile(xb, halo + (i64)blockIdx.x * C * (K - 1), ck.column_after(b, tiles, TN), xs, C, 4 * c4, L, j0, tsh,
+                   K - 1, pitch, vec, (int)threadIdx.x, 256);
         __syncthreads();
         for (int item = wave; item < groups * parts; item += 4) {
             const int g = item / parts, part = item - g * parts;

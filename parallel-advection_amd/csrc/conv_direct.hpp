@@ -27,23 +27,23 @@ struct DirectConv {
 };
 
 // The chunk of an owner: tiles [first, end) of the flattened (batch element,
-// tile) sequence.  Where it ends inside a row, b is that batch element and j
-// the first column after the chunk, which the next owner overwrites; else
-// b = -1.
+// tile) sequence.
 struct ConvChunk {
-    int first, end, b, j;
-    // whether column cj of batch element cb comes from the copy made before the launch
-    __host__ __device__ __forceinline__ bool copied(int cb, int cj) const { return cb == b && cj >= j; }
+    int first, end;
+    // The first column of batch element b after the chunk, from where on another
+    // owner writes the row and a tile takes the copy made before the launch; beyond
+    // every column where the chunk goes on past the row.
+    __host__ __device__ __forceinline__ int column_after(int b, int tiles, int TN) const {
+        const int t = end - b * tiles;
+        return t < tiles ? t * TN : 0x7fffffff;
+    }
 };
-__host__ __device__ __forceinline__ ConvChunk conv_chunk(int owner, int chunk, int total, int tiles, int TN) {
+__host__ __device__ __forceinline__ ConvChunk conv_chunk(int owner, int chunk, int total) {
     // in 64 bits: total goes up to 2^31 - 1, and an owner past the last one has no tiles
     const i64 first = (i64)owner * chunk, end = first + chunk;
     ConvChunk c;
     c.first = first < total ? (int)first : total;
     c.end = end < total ? (int)end : total;
-    const int last = c.end - 1, t = last % tiles;
-    c.b = t < tiles - 1 ? last / tiles : -1;
-    c.j = (t + 1) * TN;
     return c;
 }
 

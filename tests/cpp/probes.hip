@@ -131,7 +131,7 @@ int probe_fp8_convert(const void *in, void *out, unsigned long long n, void *str
 }
 // Host only: the tiles [first, end) of a direct convolution's owner.
 void probe_conv_chunk(int owner, int chunk, int total, int *first, int *end) {
-    const ConvChunk ck = conv_chunk(owner, chunk, total, total, 64);
+    const ConvChunk ck = conv_chunk(owner, chunk, total);
     *first = ck.first;
     *end = ck.end;
 }
@@ -143,13 +143,13 @@ long long probe_conv_chunk_faults(int B, int tiles, int TN, int K, int chunk) {
     long long bad = 0;
     const int total = B * tiles, owners = (total + chunk - 1) / chunk;
     for (int o = 0; o < owners; ++o) {
-        const ConvChunk ck = conv_chunk(o, chunk, total, tiles, TN);
+        const ConvChunk ck = conv_chunk(o, chunk, total);
         if (ck.first != o * chunk || ck.end != std::min(total, (o + 1) * chunk)) return -1;
         for (int tile = ck.first; tile < ck.end; ++tile) {
-            const int b = tile / tiles, j0 = (tile - b * tiles) * TN;
+            const int b = tile / tiles, j0 = (tile - b * tiles) * TN, after = ck.column_after(b, tiles, TN);
             for (int j = j0; j < j0 + TN + K - 1; ++j) {
                 if (j >= tiles * TN) break;  // columns that nobody writes
-                if (ck.copied(b, j)) bad += j - ck.j >= K - 1;
+                if (j >= after) bad += j - after >= K - 1;
                 else bad += b * tiles + j / TN >= ck.end || b * tiles + j / TN < tile;
             }
         }
